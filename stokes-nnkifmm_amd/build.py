@@ -15,7 +15,7 @@ LIB = os.path.join(LIBDIR, "libnnkifmm.so")
 SELFTEST = os.path.join(LIBDIR, "libnnk_selftest.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["nnk_tree.cpp", "nnk_tree_gpu.hip", "nnk_svd.hip", "nnk_fmm.hip", "nnk_direct.hip", "nnk_reduced.hip",
+SOURCES = ["nnk_tree.cpp", "nnk_tree_gpu.hip", "nnk_svd.hip", "nnk_fmm.hip", "nnk_spectral.hip", "nnk_direct.hip", "nnk_reduced.hip",
            "nnk_nearest.hip", "nnk_mobility.hip", "nnk_mixed.hip", "nnk_batch.hip", "nnk_capi.cpp"]
 
 # -packed-fp32-ops: no packed FP32 instructions in device code.
@@ -63,11 +63,13 @@ def build(verbose=False):
     os.replace(tmp, LIB)
     # test-only companion library (GEMM / internal-array probes, host-only
     # planner checks; its source lives with the tests)
-    st = os.path.join(os.path.dirname(HERE), "tests", "native", "nnk_selftest.hip")
-    sto = os.path.join(objdir, "nnk_selftest.o")
-    _run([HIPCC, "-x", "hip"] + COMMON + DEVICE_FLAGS + ["-I" + CSRC, "-c", st, "-o", sto])
+    stos = []
+    for name in ("nnk_selftest", "nnk_spectral_selftest"):
+        st = os.path.join(os.path.dirname(HERE), "tests", "native", name + ".hip")
+        stos.append(os.path.join(objdir, name + ".o"))
+        _run([HIPCC, "-x", "hip"] + COMMON + DEVICE_FLAGS + ["-I" + CSRC, "-c", st, "-o", stos[-1]])
     tmp2 = SELFTEST + ".tmp"
-    _run([HIPCC, "-shared", "--offload-arch=gfx950", "-o", tmp2, sto, "-L" + LIBDIR, "-lnnkifmm",
+    _run([HIPCC, "-shared", "--offload-arch=gfx950", "-o", tmp2] + stos + ["-L" + LIBDIR, "-lnnkifmm",
           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath,/opt/rocm/lib"])
     os.replace(tmp2, SELFTEST)
     build_gateway()

@@ -969,9 +969,7 @@ Fmm::Fmm(std::shared_ptr<const Tree> t, double eps, double mu, int res, int shel
     OpCache &C = OpCache::get();
     std::vector<int> miss;
     for (int l = 2; l <= maxlev_; l++) {
-      // FP64 form: operators with T.  Mixed forms: any entry (T unused).
       auto hit = C.find(key(0, l));
-      if (!hit && prec_ >= 1) hit = C.find(key(1, l));
       if (hit) ops_[l] = std::static_pointer_cast<const LevelOps>(hit);
       else miss.push_back(l);
     }
@@ -991,8 +989,8 @@ Fmm::Fmm(std::shared_ptr<const Tree> t, double eps, double mu, int res, int shel
     if (nb) svd_batch(pa.data(), n, nb, pu.data(), ps.data(), pv.data());
     for (int b = 0; b < nb; b++) {
       const int l = miss[b];
-      ops_[l] = build_ops(l, prec_ == 0, std::move(U[b]), std::move(S[b]), std::move(V[b]));
-      C.put(key(prec_ == 0 ? 0 : 1, l), ops_[l], ops_[l]->bytes());
+      ops_[l] = build_ops(l, std::move(U[b]), std::move(S[b]), std::move(V[b]));
+      C.put(key(0, l), ops_[l], ops_[l]->bytes());
     }
   }
   plan();
@@ -1004,7 +1002,7 @@ Fmm::Fmm(std::shared_ptr<const Tree> t, double eps, double mu, int res, int shel
 }
 
 size_t LevelOps::bytes() const {
-  return Wup.bytes + Vup.bytes + Wdn.bytes + Udn.bytes + M2M.bytes + L2L.bytes + T.bytes +
+  return Wup.bytes + Vup.bytes + Wdn.bytes + Udn.bytes + M2M.bytes + L2L.bytes +
          sizeof(double) * (svdU.size() + svdS.size() + svdV.size());
 }
 
@@ -1153,7 +1151,7 @@ std::vector<double> Fmm::up_to_down(int l) const {
   return A;
 }
 
-std::shared_ptr<const LevelOps> Fmm::build_ops(int l, bool with_T, std::vector<double> U, std::vector<double> S,
+std::shared_ptr<const LevelOps> Fmm::build_ops(int l, std::vector<double> U, std::vector<double> S,
                                                std::vector<double> V) {
   auto op = std::make_shared<LevelOps>();
   LevelOps &O = *op;
@@ -1197,9 +1195,31 @@ std::shared_ptr<const LevelOps> Fmm::build_ops(int l, bool with_T, std::vector<d
       form_op(pdn, cup, nq_, e2, c, O.L2L.as<double>() + k * mat, Mpad_);  // parent down -> child up
     }
   }
-  if (with_T) form_T(l, O.T, O.tslot);
-  else O.tslot.assign(343, nullptr);
   return op;
+}
+
+std::shared_ptr<const TransOps> Fmm::trans_ops(int l) {
+  OpCache &C = OpCache::get();
+  auto t = std::static_pointer_cast<const TransOps>(C.find(key(kOpTrans, l)));
+  if (!t) {
+    auto n = std::make_shared<TransOps>();
+    form_T(l, n->T, n->tslot);
+    C.put(key(kOpTrans, l), n, n->bytes());
+    t = n;
+  }
+  return t;
+}
+
+std::shared_ptr<const SpecOps> Fmm::spec_ops(int l) {
+  OpCache &C = OpCache::get();
+  auto t = std::static_pointer_cast<const SpecOps>(C.find(key(kOpSpec, l)));
+  if (!t) {
+    auto n = std::make_shared<SpecOps>();
+    spectral_ops(res_, std::ldexp(w0_, -l), eps_, mu_, *n);
+    C.put(key(kOpSpec, l), n, n->bytes());
+    t = n;
+  }
+  return t;
 }
 
 void Fmm::form_T(int l, DBuf &T, std::vector<double *> &tslot) {
@@ -1263,6 +1283,9 @@ void Fmm::plan() {
       if (T.tgt_leaf[n]) hl_[l].tleaves.push_back(n - 1);
     }
   }
+  trans_.assign(maxlev_ + 1, nullptr);
+  std::vector<int32_t> child0(nc);
+  for (int n = 1; n <= nc; n++) child0[n - 1] = T.children[8 * (n - 1)] - 1;
   size_t maxn = 1;
   std::vector<std::vector<int>> bylev(maxlev_ + 1);
   for (int n = 1; n <= nc; n++) bylev[T.level[n - 1]].push_back(n);
@@ -1347,19 +1370,14 @@ void Fmm::plan() {
     P.n_down = (int)dn.size();
     maxn = std::max(maxn, dn.size());
     if (P.n_down) {
-      std::vector<GemmJob> jobs, ljobs;
-      std::vector<const double *> cops[8];  // per class: its operators in block order
+      std::vector<GemmJob> ljobs;
       const size_t mat = (size_t)Kpad_ * Mpad_;
       for (int a = 0; a < 8; a++) {
         if (cls[a].empty()) continue;
         auto offs = class_offsets(a);
         std::map<int, int> pos;
-        std::vector<const double *> &A = cops[a];
-        for (size_t b = 0; b < offs.size(); b++) {
-          pos[offset_slot(offs[b][0], offs[b][1], offs[b][2])] = (int)b;
-          A.push_back(O.tslot[offset_slot(offs[b][0], offs[b][1], offs[b][2])]);
-        }
-        const int nb = (int)A.size(), N = (int)cls[a].size();
+        for (size_t b = 0; b < offs.size(); b++) pos[offset_slot(offs[b][0], offs[b][1], offs[b][2])] = (int)b;
+        const int nb = (int)offs.size(), N = (int)cls[a].size();
         std::vector<int32_t> g((size_t)nb * N, -1);
         for (int j = 0; j < N; j++) {
           int n = clsnode[a][j];
@@ -1377,16 +1395,6 @@ void Fmm::plan() {
             stats_[0]++;
           }
         }
-        add_job(P.m2l, jobs, A, &g, &cls[a], N);
-        {  // active blocks per 64-column tile of the M2L launch
-          std::vector<int32_t> tp, tl;
-          tile_lists(g, nb, N, GBN1, tp, tl);
-          check_gather_job(g, nb, N, GBN1, tp, tl, T.count, "M2L job");
-          P.m2l.owned.emplace_back(make_dbuf(tp));
-          jobs.back().tptr = P.m2l.owned.back().as<int32_t>();
-          P.m2l.owned.emplace_back(make_dbuf(tl));
-          jobs.back().tlist = P.m2l.owned.back().as<int32_t>();
-        }
         std::vector<int32_t> gp(N);
         for (int j = 0; j < N; j++) gp[j] = T.parent[clsnode[a][j] - 1] - 1;
         if (l >= 3)  // parent's down density onto the child's up surface
@@ -1395,23 +1403,18 @@ void Fmm::plan() {
         hl_[l].gv[a] = std::move(g);
         hl_[l].gp[a] = std::move(gp);
       }
-      finish(P.m2l, jobs);
       finish(P.l2l, ljobs);
-      {  // split-K for levels with few output tiles
-        const int nj = P.m2l.njobs, mN = P.m2l.maxN;
-        std::vector<int32_t> slot((size_t)nj * mN, -1);
-        int j = 0, minnb = 512;
-        for (int a = 0; a < 8; a++) {
-          if (cls[a].empty()) continue;
-          for (size_t c = 0; c < cls[a].size(); c++) slot[(size_t)j * mN + c] = cls[a][c];
-          minnb = std::min(minnb, (int)class_offsets(a).size());
-          j++;
+      if (prec_ == 0 && spectral_res(res_) && shells_ == 1) {
+        SpecLevel S;
+        S.level = l;
+        plan_spectral_level(hl_[l].cls, hl_[l].gv, T.parent, child0, pot_below, S);
+        if (S.ok) {
+          if (!spec_) spec_ = std::make_unique<SpectralM2L>(res_, surface_codes(res_, shells_), K_);
+          spec_->add(S, spec_ops(l));
+          P.m2l_spec = P.m2l_spec_on = true;
         }
-        P.m2l_split = split_for((int64_t)nj * (Mpad_ / GBM) * ((mN + GBN1 - 1) / GBN1), minnb);
-        P.m2l_slot.upload(slot);  // also for the autotuner's split candidates
-        reserve_part((size_t)std::min(64, 2 * P.m2l_split) * nj * mN * K_);
       }
-      if (prec_ == 0) plan_m2l_pairs(P, hl_[l].cls, hl_[l].gv, cops, K_);
+      if (!P.m2l_spec) plan_m2l_dense(l);
       std::vector<GemmJob> j1, j2;
       add_job(P.dn_solve1, j1, {O.Wdn.as<double>()}, &dn, nullptr, P.n_down);
       finish(P.dn_solve1, j1);
@@ -1442,6 +1445,7 @@ void Fmm::plan() {
     if (n_x_all_ && prec_ == 0) xchk_.alloc(sizeof(double) * (size_t)nc * K_);
     else xchk_ = DBuf();
   }
+  if (spec_) spec_->finish();
   tmp_.alloc(sizeof(double) * maxn * K_);
   // remaining work counts
   std::vector<int64_t> srcn(nc + 2, 0), tgtn(nc + 2, 0);
@@ -1471,6 +1475,60 @@ void Fmm::plan() {
       if (l >= 3 && tgt_below[n]) stats_[9]++;
     }
   }
+}
+
+void Fmm::plan_m2l_dense(int l) {
+  LevelPlan &P = plans_[l];
+  const HostLevel &H = hl_[l];
+  if (P.m2l_dense) return;
+  if (prec_ == 0 && !trans_[l]) trans_[l] = trans_ops(l);
+  std::vector<GemmJob> jobs;
+  std::vector<const double *> cops[8];  // per class: its operators in block order
+  P.m2l = GemmBatch();
+  GemmBatch &B = P.m2l;
+  for (int a = 0; a < 8; a++) {
+    if (H.cls[a].empty()) continue;
+    for (int sl : class_offset_slots(a)) cops[a].push_back(trans_[l] ? trans_[l]->tslot[sl] : nullptr);
+    const int nb = (int)cops[a].size(), N = (int)H.cls[a].size();
+    if (nb > 512) throw Error(NNK_ESTATE, "too many operator blocks in one GEMM job");
+    // active blocks per 64-column tile of the M2L launch
+    std::vector<int32_t> tp, tl;
+    tile_lists(H.gv[a], nb, N, GBN1, tp, tl);
+    check_gather_job(H.gv[a], nb, N, GBN1, tp, tl, tree_.count, "M2L job");
+    GemmJob j{};
+    B.owned.emplace_back(make_dbuf(cops[a]));
+    j.A = B.owned.back().as<const double *>();
+    B.owned.emplace_back(make_dbuf(H.gv[a]));
+    j.gidx = B.owned.back().as<int32_t>();
+    B.owned.emplace_back(make_dbuf(H.cls[a]));
+    j.cidx = B.owned.back().as<int32_t>();
+    B.owned.emplace_back(make_dbuf(tp));
+    j.tptr = B.owned.back().as<int32_t>();
+    B.owned.emplace_back(make_dbuf(tl));
+    j.tlist = B.owned.back().as<int32_t>();
+    j.nb = nb;
+    j.N = N;
+    jobs.push_back(j);
+    B.maxN = std::max(B.maxN, N);
+  }
+  B.njobs = (int)jobs.size();
+  B.jobs.upload(jobs);
+  {  // split-K for levels with few output tiles
+    const int nj = B.njobs, mN = B.maxN;
+    std::vector<int32_t> slot((size_t)nj * mN, -1);
+    int j = 0, minnb = 512;
+    for (int a = 0; a < 8; a++) {
+      if (H.cls[a].empty()) continue;
+      for (size_t c = 0; c < H.cls[a].size(); c++) slot[(size_t)j * mN + c] = H.cls[a][c];
+      minnb = std::min(minnb, (int)cops[a].size());
+      j++;
+    }
+    P.m2l_split = split_for((int64_t)nj * (Mpad_ / GBM) * ((mN + GBN1 - 1) / GBN1), minnb);
+    P.m2l_slot.upload(slot);  // also for the autotuner's split candidates
+    reserve_part((size_t)std::min(64, 2 * P.m2l_split) * nj * mN * K_);
+  }
+  if (prec_ == 0) plan_m2l_pairs(P, H.cls, H.gv, cops, K_);
+  P.m2l_dense = true;
 }
 
 void Fmm::stats(int64_t *out) const {
@@ -1603,8 +1661,9 @@ void Fmm::launch_config(int level, int *split, int *depth) const {
       *depth = P.m2l_pair_on ? 10 + P.mx_pair_depth : P.mx_depth;
     }
   } else if (P.n_down) {
-    *split = P.m2l_pair_on ? 1 : P.m2l_split;
-    *depth = P.m2l_pair_on ? 1 : 0;
+    const bool one = P.m2l_spec_on || P.m2l_pair_on;
+    *split = one ? 1 : P.m2l_split;
+    *depth = one ? 1 : 0;
   }
 }
 
@@ -1613,6 +1672,13 @@ void Fmm::set_launch_config(int level, int split, int depth) {
   LevelPlan &P = plans_[level];
   const bool mixed = m16();
   if (mixed ? !P.mx_m2l_jobs : !P.n_down) throw Error(NNK_EARG, "launch config: level without M2L");
+  if (P.m2l_spec && depth == 1) {
+    if (split != 1) throw Error(NNK_EARG, "launch config: the frequency-space M2L takes split 1");
+    P.m2l_spec_on = true;
+    gop_.reset();
+    return;
+  }
+  if (P.m2l_spec && depth == 0) plan_m2l_dense(level);
   const size_t per_split = mixed ? (size_t)P.mx_m2l_jobs * P.mx_m2l_maxN * RP_
                                  : (size_t)P.m2l.njobs * P.m2l.maxN * m2l_ld();
   if (split < 1 || split > 64 || (split > 1 && ((size_t)split * per_split > part_elems_ ||
@@ -1625,7 +1691,7 @@ void Fmm::set_launch_config(int level, int split, int depth) {
       P.m2l_pair_on = true;
     } else if (depth == 0) {
       P.m2l_split = split;
-      P.m2l_pair_on = false;
+      P.m2l_pair_on = P.m2l_spec_on = false;
     } else {
       throw Error(NNK_EARG, "launch config: the FP64 forms take depth 0 or 1");
     }
@@ -1658,6 +1724,7 @@ void Fmm::autotune(hipStream_t s) {
       LevelPlan &P = plans_[l];
       const bool mixed = m16();
       if (mixed ? !P.mx_m2l_jobs : !P.n_down) continue;
+      if (P.m2l_spec_on) continue;   // one launch for every such level, nothing to choose
       const int s0 = mixed ? P.mx_split : P.m2l_split;
       const size_t per_split = mixed ? (size_t)P.mx_m2l_jobs * P.mx_m2l_maxN * RP_
                                      : (size_t)P.m2l.njobs * P.m2l.maxN * m2l_ld();
@@ -1801,13 +1868,20 @@ void Fmm::apply_impl(const double *d_f, double *d_u, hipStream_t s) {
                 xchk_.as<double>(), s);
     mark(5, false, s);
   }
+  if (spec_) {  // the M2L of every frequency-space level (chk of levels switched to dense is rewritten below)
+    mark(3, true, s);
+    spec_->run(up, chk, s);
+    mark(3, false, s);
+  }
   for (int l = 2; l <= maxlev_; l++) {
     LevelPlan &P = plans_[l];
     if (!P.n_down) continue;
-    mark(3, true, s);
-    if (P.m2l_pair_on) launch_m2l_pairs(P, up, K_, chk, K_, K_, Mpad_, Kpad_, s);
-    else gemm(P.m2l, up, K_, chk, K_, 0, s, 1, P.m2l_split, &P.m2l_slot);
-    mark(3, false, s);
+    if (!P.m2l_spec_on) {
+      mark(3, true, s);
+      if (P.m2l_pair_on) launch_m2l_pairs(P, up, K_, chk, K_, K_, Mpad_, Kpad_, s);
+      else gemm(P.m2l, up, K_, chk, K_, 0, s, 1, P.m2l_split, &P.m2l_slot);
+      mark(3, false, s);
+    }
     mark(4, true, s);
     gemm(P.l2l, dn, K_, chk, K_, 1, s);
     mark(4, false, s);

@@ -10,6 +10,7 @@
 
 #include "nnk_common.hpp"
 #include "nnk_graph.hpp"
+#include "nnk_spectral.hpp"
 #include "nnk_tree.hpp"
 
 namespace nnk {
@@ -131,6 +132,10 @@ struct LevelPlan {
   // pairs of one offset, each product into its own column of the pair
   // buffer, then a fixed-order sum per target (by offset slot).  Built
   // where the planner's work estimate favours it; m2l_pair_on selects it.
+  // FP64 form: the level's M2L runs in frequency space (with every other
+  // such level, in one set of launches before the level-by-level down pass);
+  // the dense batches below are then planned only if a caller selects them
+  bool m2l_spec = false, m2l_spec_on = false, m2l_dense = false;
   int m2l_npairs = 0;         // pairs of the per-offset plan (0: none built)
   bool m2l_pair_on = false;
   GemmBatch m2lp;             // one operator, <= 64 pairs per job
@@ -196,10 +201,16 @@ struct MixedOps {
 struct LevelOps {
   DBuf Wup, Vup, Wdn, Udn;    // check-to-equivalent factors, At layout
   DBuf M2M, L2L;              // 8 operators each (this level's child class)
-  DBuf T;                     // 316 translation operators (absent in the mixed forms)
-  std::vector<double *> tslot;  // host copy: slot -> device pointer or null
   std::vector<double> svdU, svdS, svdV;  // host SVD of K(up -> down), row-major
   size_t bytes() const;
+};
+
+// the 316 dense translation operators of one level (FP64 form, levels whose
+// M2L does not run in frequency space); read-only once built
+struct TransOps {
+  DBuf T;
+  std::vector<double *> tslot;  // offset slot (343) -> device pointer or null
+  size_t bytes() const { return T.bytes; }
 };
 
 // Process-wide cache of per-level operators.  The operators of a level
@@ -210,10 +221,12 @@ struct LevelOps {
 // entries are always shared; up to `limit` bytes of entries whose last
 // owner is gone are kept (least recently used first out).
 struct OpKey {
-  int dev, kind, res, shells, level, rank;  // kind: 0 FP64 (with T), 1 no T, 2+p mixed precision p
+  // kind: 0 FP64 (LevelOps), 2+p mixed precision p, kOpTrans, kOpSpec
+  int dev, kind, res, shells, level, rank;
   double eps, mu, w, tau;
   bool operator<(const OpKey &o) const;
 };
+constexpr int kOpTrans = 100, kOpSpec = 101;
 class OpCache {
  public:
   static OpCache &get();
@@ -297,10 +310,16 @@ class Fmm {
   // K(up -> down) of the canonical box of a level, and the level's
   // operators from that matrix's SVD (A = U diag(S) V^T, row-major)
   std::vector<double> up_to_down(int level) const;
-  std::shared_ptr<const LevelOps> build_ops(int level, bool with_T, std::vector<double> U, std::vector<double> S,
+  std::shared_ptr<const LevelOps> build_ops(int level, std::vector<double> U, std::vector<double> S,
                                             std::vector<double> V);
   // the 316 translation operators of a level into T (tslot: 343 pointers)
   void form_T(int level, DBuf &T, std::vector<double *> &tslot);
+  // FP64 form: the dense M2L of level l (class tiles and, where the planner
+  // favours them, per-offset pair jobs) and its translation operators
+  void plan_m2l_dense(int l);
+  // the cached translation operators of a level: dense, in frequency space
+  std::shared_ptr<const TransOps> trans_ops(int l);
+  std::shared_ptr<const SpecOps> spec_ops(int l);
   OpKey key(int kind, int level) const;
   void gemm(const GemmBatch &b, const double *X, int ldx, double *C, int ldc, int beta, hipStream_t s,
             int tag = 0, int nsplit = 1, const DBuf *slot = nullptr);
@@ -377,6 +396,8 @@ class Fmm {
   // work buffers
   DBuf chk_, uppot_, downpot_, tmp_;
   std::vector<std::shared_ptr<const LevelOps>> ops_;
+  std::vector<std::shared_ptr<const TransOps>> trans_;  // levels with a dense FP64 M2L
+  std::unique_ptr<SpectralM2L> spec_;                   // FP64 form: the levels with m2l_spec
   std::vector<LevelPlan> plans_;
   std::vector<HostLevel> hl_;
   int prec_ = 0;

@@ -301,8 +301,8 @@ void Fmm::build_mixed() {
     MixedOps &X = *fresh[l];
     // ---- M2L: C_o = Pdn T_o V_R, with T_o formed for this level only ----
     DBuf Ttmp;
-    std::vector<double *> tslot = O.tslot;
-    if (!O.T.p) form_T(l, Ttmp, tslot);
+    std::vector<double *> tslot;
+    form_T(l, Ttmp, tslot);
     std::vector<const double *> Ts;
     std::vector<int> slots;
     for (int sl = 0; sl < 343; sl++)
