@@ -25,7 +25,6 @@
 #include <map>
 #include <mutex>
 #include <tuple>
-#include <type_traits>
 
 #include "nnk_fmm.hpp"
 #include "nnk_gemm.hpp"
@@ -98,8 +97,8 @@ struct SurfArgs {
   double *chk;
 };
 
-// Check potential on a node surface from the sources of a set of leaves
-// (S2M: the leaf itself onto its down surface; P2L: the X list onto the up
+// FP32-math forms: check potential on a node surface from the sources of a
+// set of leaves (S2M: the leaf itself onto its down surface; P2L: the X list onto the up
 // surface).  One 512-thread block per node; sources staged in LDS 512 at a
 // time.  The nq surface points are taken in chunks of c, each point shared
 // by nsub = 512 / c lanes that split the sources; their partial sums are
@@ -110,14 +109,12 @@ struct SurfArgs {
 // than seven chunks of 56 points x 9 lanes.
 constexpr int kSurfThreads = 512;
 
-template <bool F32>
 __global__ __launch_bounds__(kSurfThreads) void k_surf_eval(SurfArgs a) {
   constexpr int T = kSurfThreads;
   const int n = a.nodes[blockIdx.x];
-  // FP32 math: positions as FP32 offsets from this node's centre (the
-  // smaller box of an X-list pair; S2M pairs share the box)
-  typedef typename std::conditional<F32, SrcStageRel<T>, SrcStage<false, T>>::type Stage;
-  __shared__ Stage st;
+  // positions as FP32 offsets from this node's centre (the smaller box of an
+  // X-list pair; S2M pairs share the box)
+  __shared__ SrcStageRel<T> st;
   __shared__ double red[T * 3];
   const double *box = a.corners + 6 * (size_t)(n - 1);
   double cx, cy, cz;
@@ -157,20 +154,11 @@ __global__ __launch_bounds__(kSurfThreads) void k_surf_eval(SurfArgs a) {
         const int cnt = min(T, se - s0);
         if (tid < cnt) {
           const size_t s = (size_t)(s0 + tid);
-          if constexpr (F32)
-            st.put(tid, a.src_pos[3 * s] - cx, a.src_pos[3 * s + 1] - cy, a.src_pos[3 * s + 2] - cz,
-                   a.src_q[3 * s], a.src_q[3 * s + 1], a.src_q[3 * s + 2]);
-          else
-            st.put(tid, a.src_pos[3 * s], a.src_pos[3 * s + 1], a.src_pos[3 * s + 2], a.src_q[3 * s],
-                   a.src_q[3 * s + 1], a.src_q[3 * s + 2]);
+          st.put(tid, a.src_pos[3 * s] - cx, a.src_pos[3 * s + 1] - cy, a.src_pos[3 * s + 2] - cz,
+                 a.src_q[3 * s], a.src_q[3 * s + 1], a.src_q[3 * s + 2]);
         }
         __syncthreads();
-        if (act) {
-          if constexpr (F32)
-            st.run(sub, nsub, cnt, (float)(tx - cx), (float)(ty - cy), (float)(tz - cz), e2f, ux, uy, uz);
-          else
-            st.run(sub, nsub, cnt, tx, ty, tz, a.e2, ux, uy, uz);
-        }
+        if (act) st.run(sub, nsub, cnt, (float)(tx - cx), (float)(ty - cy), (float)(tz - cz), e2f, ux, uy, uz);
         __syncthreads();
       }
     }
@@ -195,6 +183,206 @@ __global__ __launch_bounds__(kSurfThreads) void k_surf_eval(SurfArgs a) {
   }
 }
 
+// The FP64 form of S2M.  Surface points sit on lanes, one wavefront per 64
+// of them; a source is wavefront-uniform: its six doubles come through the
+// scalar cache into scalar registers, four sources at a time, so the loop
+// issues only the pairs' FP64 instructions, with no LDS staging and no
+// barrier.
+__global__ __launch_bounds__(512) void k_s2m64(SurfArgs a, const double *__restrict__ src_pos,
+                                               const double *__restrict__ src_q) {
+  const int n = a.nodes[blockIdx.x];
+  const double *box = a.corners + 6 * (size_t)(n - 1);
+  const int sb = a.src_ptr[n], se = a.src_ptr[n + 1];
+  for (int p = threadIdx.x; p < a.nq; p += blockDim.x) {
+    double tx, ty, tz;
+    surf_point(box, a.down, a.surf_idx[p], a.n1, tx, ty, tz);
+    double ux = 0, uy = 0, uz = 0;
+    int j = sb;
+    for (; j + 4 <= se; j += 4) {
+      double x[12], q[12];
+#pragma unroll
+      for (int k = 0; k < 12; k++) x[k] = src_pos[3 * (size_t)j + k];
+#pragma unroll
+      for (int k = 0; k < 12; k++) q[k] = src_q[3 * (size_t)j + k];
+#pragma unroll
+      for (int k = 0; k < 12; k += 3)
+        stokeslet_acc64(tx, ty, tz, x[k], x[k + 1], x[k + 2], q[k], q[k + 1], q[k + 2], a.e2, ux, uy, uz);
+    }
+    for (; j < se; j++) {
+      const double *x = src_pos + 3 * (size_t)j, *q = src_q + 3 * (size_t)j;
+      stokeslet_acc64(tx, ty, tz, x[0], x[1], x[2], q[0], q[1], q[2], a.e2, ux, uy, uz);
+    }
+    double *o = a.chk + (size_t)(n - 1) * a.K + 3 * p;
+    o[0] = a.c * ux;
+    o[1] = a.c * uy;
+    o[2] = a.c * uz;
+  }
+}
+
+// ---- FP64 sums with sources on lanes --------------------------------------
+// A wavefront sums a list of sources onto a block of NT targets: every lane
+// holds one source of a 64-source chunk in registers, the targets are
+// wavefront-uniform (scalar operands), and each lane keeps NT x 3 partial
+// sums, which a butterfly adds over the lanes at the end.  Per pair only
+// the 28 FP64 slots are issued; lanes are full whatever the number of
+// targets, where a target per lane would leave most of them idle (an
+// adaptive leaf holds about 10 targets).  The workgroup stages the sources
+// (list search, surface points) once for its wavefronts: each wavefront
+// fetching its own costs 25 % more on P2L and 50 % on the leaf kernel.
+// Measured before (targets on lanes, every source read from LDS per pair)
+// and now, res 6: leaf kernel of a 64-spheroid suspension 5.16 -> 2.33 ms
+// (0.99e9 pairs), its P2L 3.9 -> 3.2 ms (3.08e9 pairs, 0.96e12/s), leaf
+// kernel of 65,537 points 0.49 -> 0.23 ms, of 2^20 points 1.39 -> 1.28 ms.
+
+// one butterfly step: half of the C values move to the other lane of the
+// pair, the kept half is added; idx and cnt follow which values remain
+template <int C, int S, int N>
+__device__ __forceinline__ void wave_scatter_sum(double (&v)[N], int lane, int &idx, int &cnt) {
+  constexpr int H = C > 1 ? (C + 1) / 2 : 1;
+  if constexpr (C > 1) {
+    const bool hi = lane & S;
+#pragma unroll
+    for (int i = 0; i < H; i++) {
+      const double up = i + H < C ? v[i + H] : 0.0;
+      const double keep = hi ? up : v[i], send = hi ? v[i] : up;
+      v[i] = keep + __shfl_xor(send, S);
+    }
+    idx += hi ? H : 0;
+    cnt = hi ? cnt - H : min(cnt, H);
+  } else {
+    v[0] += __shfl_xor(v[0], S);
+  }
+  if constexpr (S > 1) wave_scatter_sum<H, S / 2>(v, lane, idx, cnt);
+}
+
+// prefix of the source counts of list[0 .. nu) (nu <= kLeafMaxU) into
+// pre[0 .. nu]; the whole workgroup calls it, with a barrier at the end
+constexpr int kLeafMaxU = 512;
+__device__ __forceinline__ void source_prefix(const int32_t *__restrict__ list, int nu,
+                                              const int32_t *__restrict__ src_ptr, int *pre) {
+  if (threadIdx.x < 64) {
+    int base = 0;
+    for (int e0 = 0; e0 < nu; e0 += 64) {
+      const int e = e0 + (int)threadIdx.x;
+      int c = 0;
+      if (e < nu) c = src_ptr[list[e] + 1] - src_ptr[list[e]];
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(c, d);
+        if ((int)threadIdx.x >= d) c += o;
+      }
+      if (e < nu) pre[e + 1] = base + c;
+      base += __shfl(c, 63);
+    }
+    if (threadIdx.x == 0) pre[0] = 0;
+  }
+  __syncthreads();
+}
+
+// source g of the concatenated list: leaf e with pre[e] <= g < pre[e + 1]
+// (empty leaves are skipped)
+__device__ __forceinline__ int source_index(const int32_t *__restrict__ list, int nu,
+                                            const int32_t *__restrict__ src_ptr, const int *pre, int g) {
+  int lo = 0, hi = nu;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (pre[mid] <= g) lo = mid;
+    else hi = mid;
+  }
+  return src_ptr[list[lo]] + (g - pre[lo]);
+}
+
+// lane k's value, in scalar registers
+__device__ __forceinline__ double lane_value(double v, int k) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                          __builtin_amdgcn_readlane(__double2loint(v), k));
+}
+
+struct Src6 { double x, y, z, qx, qy, qz; };
+// a batch of 256 staged sources, component by component, double-buffered
+typedef double SrcBatch[2][6][256];
+
+// the tot sources get(0 .. tot-1) onto the wavefront's NT targets: the
+// workgroup stages them 256 at a time (one per thread; the next batch is
+// fetched while the current one is summed), the wavefront takes the 64-source
+// chunks sp, sp + nsplit, ... of a batch.  Called by the whole workgroup.
+template <int NT, class Get>
+__device__ __forceinline__ void sum_sources(const double (&tx)[NT], const double (&ty)[NT], const double (&tz)[NT],
+                                            double e2, int sp, int nsplit, int tot, SrcBatch buf, Get &&get,
+                                            double (&u)[3 * NT]) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  // past the end: strength zero, one unit off a target
+  const Src6 none{tx[0] + 1.0, ty[0], tz[0], 0.0, 0.0, 0.0};
+  auto stage = [&](int b, const Src6 &s) {
+    buf[b][0][tid] = s.x;
+    buf[b][1][tid] = s.y;
+    buf[b][2][tid] = s.z;
+    buf[b][3][tid] = s.qx;
+    buf[b][4][tid] = s.qy;
+    buf[b][5][tid] = s.qz;
+  };
+  if (tot <= 0) return;
+  stage(0, tid < tot ? get(tid) : none);
+  __syncthreads();
+  for (int b = 0, g0 = 0; g0 < tot; b ^= 1, g0 += 256) {
+    const bool more = g0 + 256 < tot;
+    Src6 s = none;
+    if (g0 + 256 + tid < tot) s = get(g0 + 256 + tid);
+    const int nch = min(4, (tot - g0 + 63) >> 6);
+    for (int c = sp; c < nch; c += nsplit) {
+      const int i = 64 * c + lane;
+      const double x = buf[b][0][i], y = buf[b][1][i], z = buf[b][2][i];
+      const double qx = buf[b][3][i], qy = buf[b][4][i], qz = buf[b][5][i];
+#pragma unroll
+      for (int k = 0; k < NT; k++)
+        stokeslet_acc64(tx[k], ty[k], tz[k], x, y, z, qx, qy, qz, e2, u[3 * k], u[3 * k + 1], u[3 * k + 2]);
+    }
+    if (more) stage(b ^ 1, s);
+    __syncthreads();
+  }
+}
+
+// The FP64 form of P2L: a wavefront per NT surface points of a node, the
+// sources of its X list on lanes.
+template <int NT>
+__global__ __launch_bounds__(256) void k_p2l64(SurfArgs a, const double *__restrict__ src_pos,
+                                               const double *__restrict__ src_q) {
+  __shared__ int pre[kLeafMaxU + 1];
+  __shared__ SrcBatch buf;
+  const int n = a.nodes[blockIdx.x];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const double *box = a.corners + 6 * (size_t)(n - 1);
+  const int p0 = (blockIdx.y * 4 + w) * NT;
+  double lx = 0, ly = 0, lz = 0;
+  if (lane < NT) surf_point(box, a.down, a.surf_idx[min(p0 + lane, a.nq - 1)], a.n1, lx, ly, lz);
+  double tx[NT], ty[NT], tz[NT], u[3 * NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) {
+    tx[k] = lane_value(lx, k);
+    ty[k] = lane_value(ly, k);
+    tz[k] = lane_value(lz, k);
+    u[3 * k] = u[3 * k + 1] = u[3 * k + 2] = 0.0;
+  }
+  const int64_t lb = a.lptr[n], le = a.lptr[n + 1];
+  for (int64_t b0 = lb; b0 < le; b0 += kLeafMaxU) {
+    const int nu = (int)min((int64_t)kLeafMaxU, le - b0);
+    const int32_t *list = a.lidx + b0;
+    if (b0 > lb) __syncthreads();
+    source_prefix(list, nu, a.src_ptr, pre);
+    sum_sources<NT>(tx, ty, tz, a.e2, p0 < a.nq ? 0 : 4, 1, pre[nu], buf, [&](int g) {
+      const size_t j = 3 * (size_t)source_index(list, nu, a.src_ptr, pre, g);
+      return Src6{src_pos[j], src_pos[j + 1], src_pos[j + 2], src_q[j], src_q[j + 1], src_q[j + 2]};
+    }, u);
+  }
+  if (p0 >= a.nq) return;
+  int idx = 0, cnt = 3 * min(NT, a.nq - p0);
+  wave_scatter_sum<3 * NT, 32>(u, lane, idx, cnt);
+  if (cnt > 0) {
+    double *o = a.chk + (size_t)(n - 1) * a.K + 3 * p0 + idx;
+    *o = a.c * u[0];
+  }
+}
+
 struct LeafArgs {
   const int32_t *leaves;
   const double *corners;
@@ -214,7 +402,7 @@ struct LeafArgs {
   double *out;      // ntgt x 3
 };
 
-// Velocity at the targets of one leaf: L2T from its down density, P2P from
+// FP32-math forms: velocity at the targets of one leaf: L2T from its down density, P2P from
 // its U-list sources, M2T from its W-list up densities (Downleaf.m:37-40).
 // Each target is shared by nsub lanes that split the sources; partial sums
 // are combined in a fixed order.  T threads per workgroup (the autotuner
@@ -223,17 +411,15 @@ struct LeafArgs {
 // at a time (a leaf holds ~32: staging leaf by leaf would pay a load
 // latency and two barriers per leaf); lists longer than kLeafMaxU leaves
 // are staged leaf by leaf.
-constexpr int kLeafMaxU = 512;
-
-template <bool F32, int T>
+template <int T>
 __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
   const int n = a.leaves[blockIdx.x];
-  // FP32 math: the surface sources (L2T, M2T) go through the offset stage
+  // the surface sources (L2T, M2T) go through the offset stage
   // with the origin at the centre of the surface's node (this leaf for
   // L2T, the smaller W node for M2T); the U-list sources keep the FP64
   // separation
   __shared__ union {
-    SrcStage<F32, T> pts;
+    SrcStage<true, T> pts;
     SrcStageRel<T> srf;
   } st;
   __shared__ double red[T * 3];
@@ -273,7 +459,7 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
     auto surface = [&](int node, int down, const double *dens) {
       const double *box = a.corners + 6 * (size_t)(node - 1);
       double cx = 0, cy = 0, cz = 0;
-      if constexpr (F32) box_centre(box, cx, cy, cz);
+      box_centre(box, cx, cy, cz);
       const float txf = (float)(tx - cx), tyf = (float)(ty - cy), tzf = (float)(tz - cz);
       for (int p0 = 0; p0 < a.nq; p0 += T) {
         const int cnt = min(T, a.nq - p0);
@@ -281,15 +467,10 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
           double x, y, z;
           surf_point(box, down, a.surf_idx[p0 + tid], a.n1, x, y, z);
           const double *q = dens + (size_t)(node - 1) * a.K + 3 * (p0 + tid);
-          if constexpr (F32) st.srf.put(tid, x - cx, y - cy, z - cz, q[0], q[1], q[2]);
-          else st.pts.put(tid, x, y, z, q[0], q[1], q[2]);
+          st.srf.put(tid, x - cx, y - cy, z - cz, q[0], q[1], q[2]);
         }
         __syncthreads();
-        if constexpr (F32) {
-          if (act) st.srf.run(sub, nsub, cnt, txf, tyf, tzf, (float)a.e2, ux, uy, uz);
-        } else {
-          consume(cnt);
-        }
+        if (act) st.srf.run(sub, nsub, cnt, txf, tyf, tzf, (float)a.e2, ux, uy, uz);
         __syncthreads();
       }
     };
@@ -354,6 +535,96 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
       a.out[3 * (size_t)o + 2] = a.c * sz;
     }
     __syncthreads();
+  }
+}
+
+// The FP64 form of the leaf kernel: a workgroup takes up to 32 targets of a
+// leaf as 1, 2 or 4 blocks of at most 8 (as even as possible); its four
+// wavefronts are blocks x source shares.  The sources are one list: the
+// points of the leaf's down surface and of its W nodes' up surfaces (with
+// their densities), then the U-list sources.
+template <int NT>
+__device__ __forceinline__ void leaf_block64(const LeafArgs &a, const double *__restrict__ src_pos,
+                                             const double *__restrict__ src_q, const double *__restrict__ tgt_pos,
+                                             int n, int t0, int ntc, int blk, int sp, int nsplit, int *pre,
+                                             SrcBatch buf, double *red) {
+  double tx[NT], ty[NT], tz[NT], u[3 * NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) {
+    const double *p = tgt_pos + 3 * (size_t)(t0 + min(blk * NT + k, ntc - 1));
+    tx[k] = p[0];
+    ty[k] = p[1];
+    tz[k] = p[2];
+    u[3 * k] = u[3 * k + 1] = u[3 * k + 2] = 0.0;
+  }
+  auto point = [&](int s) {
+    const size_t j = 3 * (size_t)s;
+    return Src6{src_pos[j], src_pos[j + 1], src_pos[j + 2], src_q[j], src_q[j + 1], src_q[j + 2]};
+  };
+  if (a.far) {
+    const int64_t u0 = a.uptr[n], u1 = a.uptr[n + 1], w0 = a.wptr[n];
+    const int ns = a.nq * (1 + (int)(a.wptr[n + 1] - w0));
+    int64_t b0 = u0;
+    do {
+      const int nu = (int)min((int64_t)kLeafMaxU, u1 - b0), s0 = b0 == u0 ? ns : 0;
+      const int32_t *list = a.uidx + b0;
+      if (b0 > u0) __syncthreads();
+      source_prefix(list, nu, a.src_ptr, pre);
+      sum_sources<NT>(tx, ty, tz, a.e2, sp, nsplit, s0 + pre[nu], buf, [&](int g) {
+        if (g >= s0) return point(source_index(list, nu, a.src_ptr, pre, g - s0));
+        const int k = g / a.nq, p = g - k * a.nq;
+        const int node = k ? a.widx[w0 + k - 1] : n;
+        Src6 v;
+        surf_point(a.corners + 6 * (size_t)(node - 1), k == 0, a.surf_idx[p], a.n1, v.x, v.y, v.z);
+        const double *q = (k ? a.uppot : a.downpot) + (size_t)(node - 1) * a.K + 3 * p;
+        v.qx = q[0];
+        v.qy = q[1];
+        v.qz = q[2];
+        return v;
+      }, u);
+      b0 += kLeafMaxU;
+    } while (b0 < u1);
+  } else {  // reducedPass.m: the leaf's own sources
+    const int sb = a.src_ptr[n];
+    sum_sources<NT>(tx, ty, tz, a.e2, sp, nsplit, a.src_ptr[n + 1] - sb, buf, [&](int g) { return point(sb + g); }, u);
+  }
+  int idx = 0, cnt = 3 * NT;
+  wave_scatter_sum<3 * NT, 32>(u, threadIdx.x & 63, idx, cnt);
+  if (cnt > 0) red[idx] = u[0];
+}
+
+__global__ __launch_bounds__(256) void k_leaf64(LeafArgs a, const double *__restrict__ src_pos,
+                                                const double *__restrict__ src_q, const double *__restrict__ tgt_pos) {
+  __shared__ int pre[kLeafMaxU + 1];
+  __shared__ SrcBatch buf;
+  __shared__ double red[4][24];
+  const int n = a.leaves[blockIdx.x], tid = threadIdx.x;
+  const int tb = a.tgt_ptr[n], nt = a.tgt_ptr[n + 1] - tb, t0 = 32 * (int)blockIdx.y;
+  if (t0 >= nt) return;
+  const int ntc = min(32, nt - t0);
+  const int nblk = ntc <= 6 ? 1 : ntc <= 14 ? 2 : 4, per = (ntc + nblk - 1) / nblk;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), blk = w % nblk, sp = w / nblk, nsplit = 4 / nblk;
+#define NNK_LEAF_CASE(NT)                                                                                       \
+  case NT:                                                                                                      \
+    leaf_block64<NT>(a, src_pos, src_q, tgt_pos, n, tb + t0, ntc, blk, sp, nsplit, pre, buf, red[w]);           \
+    break
+  switch (per) {
+    NNK_LEAF_CASE(1);
+    NNK_LEAF_CASE(2);
+    NNK_LEAF_CASE(3);
+    NNK_LEAF_CASE(4);
+    NNK_LEAF_CASE(5);
+    NNK_LEAF_CASE(6);
+    NNK_LEAF_CASE(7);
+    NNK_LEAF_CASE(8);
+  }
+#undef NNK_LEAF_CASE
+  __syncthreads();
+  if (tid < 3 * ntc) {
+    const int t = tid / 3, d = tid - 3 * t, b = t / per;
+    double v = 0.0;
+    for (int s = 0; s < nsplit; s++) v += red[s * nblk + b][3 * (t - b * per) + d];
+    a.out[3 * (size_t)a.tgt_out[tb + t0 + t] + d] = a.c * v;
   }
 }
 
@@ -1593,8 +1864,11 @@ void Fmm::launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const in
   a.e2 = eps_ * eps_;
   a.c = 1.0 / (8.0 * kPi * mu_);
   a.chk = chk;
-  if (fp32_math()) hipLaunchKernelGGL(k_surf_eval<true>, dim3(n), dim3(kSurfThreads), 0, s, a);
-  else hipLaunchKernelGGL(k_surf_eval<false>, dim3(n), dim3(kSurfThreads), 0, s, a);
+  if (fp32_math()) hipLaunchKernelGGL(k_surf_eval, dim3(n), dim3(kSurfThreads), 0, s, a);
+  else if (lptr)
+    hipLaunchKernelGGL(k_p2l64<8>, dim3(n, (nq_ + 31) / 32), dim3(256), 0, s, a, a.src_pos, a.src_q);
+  else
+    hipLaunchKernelGGL(k_s2m64, dim3(n), dim3(64 * std::min((nq_ + 63) / 64, 8)), 0, s, a, a.src_pos, a.src_q);
   NNK_HIP(hipGetLastError());
 }
 
@@ -1629,13 +1903,12 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   const dim3 grid((unsigned)n_tleaves_, (unsigned)std::max(1, (max_leaf_tgt_ + a.tc - 1) / a.tc));
   auto go = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, grid, dim3(threads), 0, s, a); };
   if (fp32_math()) {
-    if (T == 128) go(k_leaf<true, 128>, 128);
-    else if (T == 512) go(k_leaf<true, 512>, 512);
-    else go(k_leaf<true, 256>, 256);
+    if (T == 128) go(k_leaf<128>, 128);
+    else if (T == 512) go(k_leaf<512>, 512);
+    else go(k_leaf<256>, 256);
   } else {
-    if (T == 128) go(k_leaf<false, 128>, 128);
-    else if (T == 512) go(k_leaf<false, 512>, 512);
-    else go(k_leaf<false, 256>, 256);
+    hipLaunchKernelGGL(k_leaf64, dim3((unsigned)n_tleaves_, (unsigned)std::max(1, (max_leaf_tgt_ + 31) / 32)), dim3(256),
+                       0, s, a, a.src_pos, a.src_q, a.tgt_pos);
   }
   NNK_HIP(hipGetLastError());
 }
@@ -1807,7 +2080,7 @@ void Fmm::autotune(hipStream_t s) {
 // time the leaf kernel (L2T + P2P + M2T) at 128, 256 and 512 threads per
 // target leaf on the current densities and keep the fastest
 void Fmm::autotune_leaf(hipStream_t s) {
-  if (!n_tleaves_) return;
+  if (!n_tleaves_ || !fp32_math()) return;   // k_leaf64 has one shape
   DBuf out;
   out.alloc(sizeof(double) * 3 * std::max<int64_t>(ntgt_, 1));
   hipEvent_t a, b;

@@ -54,6 +54,35 @@ __device__ __forceinline__ void stokeslet_acc(double tx, double ty, double tz, d
   uz += iso * qz + rq * rz;
 }
 
+// 1 / sqrt(x) for x > 0: the hardware estimate (relative error below 2^-22)
+// and one third-order step, y (1 + e/2 + 3 e^2 / 8) with e = 1 - x y^2, whose
+// own error is of order e^3.  (x = 0 and x = inf give NaN: the kernel's sums
+// are NaN there with any reciprocal square root.)
+__device__ __forceinline__ double rsqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
+// stokeslet_acc in 28 FP64 instruction slots (the hardware estimate counts
+// four): r^2 + eps^2 as one chain, the isotropic factor
+// (r^2 + 2 eps^2) / (r^2 + eps^2)^{3/2} as 1/s + eps^2 / s^3.  For the FP64
+// kernels whose sources or targets are wavefront-uniform (scalar operands),
+// so that nothing but these slots is issued per pair.
+__device__ __forceinline__ void stokeslet_acc64(double tx, double ty, double tz, double sx, double sy, double sz,
+                                                double qx, double qy, double qz, double e2, double &ux, double &uy,
+                                                double &uz) {
+  const double rx = tx - sx, ry = ty - sy, rz = tz - sz;
+  const double re = __builtin_fma(rx, rx, __builtin_fma(ry, ry, __builtin_fma(rz, rz, e2)));
+  const double inv = rsqrt_pos(re);
+  const double inv3 = inv * inv * inv;
+  const double iso = __builtin_fma(e2, inv3, inv);
+  const double rq = __builtin_fma(rx, qx, __builtin_fma(ry, qy, rz * qz)) * inv3;
+  ux = __builtin_fma(iso, qx, __builtin_fma(rq, rx, ux));
+  uy = __builtin_fma(iso, qy, __builtin_fma(rq, ry, uy));
+  uz = __builtin_fma(iso, qz, __builtin_fma(rq, rz, uz));
+}
+
 // Mixed form: the separation r = t - s is formed in FP64 (so near pairs keep
 // their digits), the kernel is evaluated in FP32 with the hardware reciprocal
 // square root, and the result is accumulated in FP64.  The strength comes in
