@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "nnk_batch.hpp"
@@ -66,11 +67,41 @@ __device__ __forceinline__ void grad_acc(double rxd, double ryd, double rzd, dou
 
 }  // namespace
 
+// The pair sums read a problem's sources as 48 B records: position in FP64,
+// strength in FP64 or, for the FP32-math operators, rounded to FP32.  They
+// lie in kRuns runs (sources w, w + kRuns, ...).  First record of run w of
+// problem p, whose n sources start at source sb (kRuns spare records a
+// problem):
+constexpr int kRuns = 4;
+__device__ __forceinline__ int64_t rec_run(int64_t sb, int p, int w, int64_t n) {
+  return sb + (int64_t)kRuns * p + w * ((n + kRuns - 1) / kRuns);
+}
+__device__ __forceinline__ void put_record(double *rec, bool f32, int64_t sb, int p, int64_t n, int64_t loc,
+                                           const double *x, double gx, double gy, double gz) {
+  double *o = rec + 6 * (rec_run(sb, p, (int)(loc % kRuns), n) + loc / kRuns);
+  o[0] = x[0];
+  o[1] = x[1];
+  o[2] = x[2];
+  if (f32) {
+    float *f = reinterpret_cast<float *>(o + 3);
+    f[0] = (float)gx;
+    f[1] = (float)gy;
+    f[2] = (float)gz;
+  } else {
+    o[3] = gx;
+    o[4] = gy;
+    o[5] = gz;
+  }
+}
+
 // g[q] = sum_e NN(q, col e) f(col e)    (the quadrature strengths, 3 each)
+// and, unless null, the sources' records
 __global__ void k_bgather(int64_t qtot, const int64_t *__restrict__ ptr, const int32_t *__restrict__ col,
                           const double *__restrict__ val, const double *__restrict__ x,
                           const int64_t *__restrict__ xbase, const int64_t *__restrict__ xstride,
-                          double *__restrict__ g) {
+                          double *__restrict__ g, double *__restrict__ rec, bool f32,
+                          const int32_t *__restrict__ fpid, const int64_t *__restrict__ foff,
+                          const double *__restrict__ fine) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= qtot) return;
   double gx = 0, gy = 0, gz = 0;
@@ -85,6 +116,25 @@ __global__ void k_bgather(int64_t qtot, const int64_t *__restrict__ ptr, const i
   g[3 * q] = gx;
   g[3 * q + 1] = gy;
   g[3 * q + 2] = gz;
+  if (rec) {
+    const int p = fpid[q];
+    const int64_t sb = foff[p];
+    put_record(rec, f32, sb, p, foff[p + 1] - sb, q - sb, fine + 3 * q, gx, gy, gz);
+  }
+}
+
+// the force points' records for the transpose sums, strengths from the three
+// component blocks of a batched vector
+__global__ void k_brecordT(int64_t ntot, const double *__restrict__ x, const int64_t *__restrict__ xbase,
+                           const int64_t *__restrict__ xstride, double *__restrict__ rec, bool f32,
+                           const int32_t *__restrict__ ppid, const int64_t *__restrict__ poff,
+                           const double *__restrict__ pts) {
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= ntot) return;
+  const int64_t b = xbase[j], st = xstride[j];
+  const int p = ppid[j];
+  const int64_t sb = poff[p];
+  put_record(rec, f32, sb, p, poff[p + 1] - sb, j - sb, pts + 3 * j, x[b], x[b + st], x[b + 2 * st]);
 }
 
 __global__ void k_bcounter_reset(int *c) {
@@ -109,72 +159,165 @@ __global__ void k_bcounter_reset(int *c) {
   __syncthreads();              \
   }
 
-// forward P2P: u_i = c sum_q S(x_i - y_q) g_q, then + BT (U; W) on body
-// points.  NW wavefronts per workgroup split the sources of a tile (the
-// autotuner picks 1, 2 or 4); their partial sums are added in wave order.
-template <bool F32, int NW>
-__global__ __launch_bounds__(64 * NW) void k_bp2p(int nitems, const int2 *__restrict__ items, int *counter,
-                                              const int64_t *__restrict__ poff, const int64_t *__restrict__ foff,
-                                              const int64_t *__restrict__ voff, const int32_t *__restrict__ nsw,
-                                              const double *__restrict__ pts, const double *__restrict__ fine,
-                                              const double *__restrict__ g, const double *__restrict__ rot,
-                                              const int32_t *__restrict__ pbody, const double *__restrict__ eps,
-                                              const int32_t *__restrict__ active, double c,
-                                              const double *__restrict__ x, double *__restrict__ y) {
-  constexpr int T = 64 * NW;
-  __shared__ SrcStage<F32, T> st;
-  __shared__ double red[NW][kTile * 3];
-  __shared__ int item_s;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  NNK_PERSISTENT_LOOP_BEGIN
-  const int64_t pb = poff[p], Np = poff[p + 1] - pb;
-  const int64_t i0 = pb + (int64_t)kTile * tile;
-  const int nt = (int)min((int64_t)kTile, Np - (int64_t)kTile * tile);
-  double tx = 0, ty = 0, tz = 0;
-  if (lane < nt) {
-    tx = pts[3 * (i0 + lane)];
-    ty = pts[3 * (i0 + lane) + 1];
-    tz = pts[3 * (i0 + lane) + 2];
-  }
-  const double e2 = eps[p] * eps[p];
-  double ux = 0, uy = 0, uz = 0;
-  const int64_t qb = foff[p], qe = foff[p + 1];
-  for (int64_t q0 = qb; q0 < qe; q0 += T) {
-    const int cnt = (int)min((int64_t)T, qe - q0);
-    if (tid < cnt) {
-      const int64_t q = q0 + tid;
-      st.put(tid, fine[3 * q], fine[3 * q + 1], fine[3 * q + 2], g[3 * q], g[3 * q + 1], g[3 * q + 2]);
-    }
-    __syncthreads();
-    if (lane < nt)
-      st.run(wv, NW, cnt, tx, ty, tz, e2, ux, uy, uz);
-    __syncthreads();
-  }
-  red[wv][3 * lane] = ux;
-  red[wv][3 * lane + 1] = uy;
-  red[wv][3 * lane + 2] = uz;
-  __syncthreads();
-  if (wv == 0 && lane < nt) {
-    double u[3];
-    for (int d = 0; d < 3; d++) {
-      double t = red[0][3 * lane + d];
+// Pair sums of one work item: a 64-target tile of a problem and one of the
+// kRuns runs of its sources (forward: quadrature points onto force points;
+// transpose: the other way round); run w's sums go to P[slot][component][64].
+// The order of a target's FP64 additions is fixed, one after the other over
+// the run (GMRES on these first-kind systems turns a reordered sum, 1e-16,
+// into 1e-8 of the solution), which would leave a large problem's run,
+// 18,816 sources for 4,704 points, to one wavefront.  Only the additions
+// are serial: the wavefronts of a workgroup evaluate the terms of the next
+// sources (FP64: 8 wavefronts, two sources each; FP32 math: 16, the FP32 sum
+// of four each) and leave them in LDS, from which three of them add one
+// component each, in order, while the others go on with the next batch.
+// Targets sit on lanes; a wavefront's records come through the scalar cache
+// into scalar registers.
+// Measured, one workgroup of four wavefronts per tile with the sources staged
+// in LDS -> now: 24 problems of 200 to 4,704 points, FP64, 3.26 -> 1.41 ms a
+// forward application (0.65e12 pairs/s; the FP64 units allow ~1.0e12);
+// squirmer pair (1,728 x 27,648 points, 27 tiles), FP32 math, forward
+// 0.575 -> 0.10 ms.  16 wavefronts of two FP64 sources took 1.66 ms, of one
+// 1.43 ms, 8 of four 1.91 ms (LDS for one workgroup a CU); a tile's runs
+// summed by one wavefront each 1.63 ms.
+template <bool F32> constexpr int kSumWaves = F32 ? 16 : 8;
+
+// the FP32 strength of a record, at the doubles q[0], q[1]
+__device__ __forceinline__ float4 rec_strength(const double *q) {
+  return float4{__int_as_float(__double2loint(q[0])), __int_as_float(__double2hiint(q[0])),
+                __int_as_float(__double2loint(q[1])), 0.f};
+}
+
+template <bool F32>
+__global__ __launch_bounds__(64 * kSumWaves<F32>) void k_bsum(const BatchItem *__restrict__ items,
+                                                              const int64_t *__restrict__ toff,
+                                                              const int64_t *__restrict__ soff,
+                                                              const double *__restrict__ tgt,
+                                                              const double *__restrict__ rec,
+                                                              const double *__restrict__ eps,
+                                                              const int32_t *__restrict__ active,
+                                                              double *__restrict__ P) {
+  // entries a wavefront evaluates per batch, records of an entry, terms of a
+  // batch ([2][entry][component][lane])
+  constexpr int PER = F32 ? 1 : 2, RE = F32 ? 4 : 1, NE = PER * kSumWaves<F32>, NV = 6 * PER * RE;
+  typedef typename std::conditional<F32, float, double>::type Term;
+  __shared__ Term term[2][NE][3][64];
+  const BatchItem it = items[blockIdx.x];
+  if (!active[it.p]) return;
+  const int lane = threadIdx.x & 63, v = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int64_t i = min(toff[it.p] + (int64_t)kTile * it.tile + lane, toff[it.p + 1] - 1);
+  const double tx = tgt[3 * i], ty = tgt[3 * i + 1], tz = tgt[3 * i + 2];
+  const double e2 = eps[it.p] * eps[it.p];
+  const int64_t sb = soff[it.p], ns = soff[it.p + 1] - sb;
+  const int n = (int)((ns - it.run + kRuns - 1) / kRuns);
+  const double *__restrict__ r = rec + 6 * rec_run(sb, it.p, it.run, ns);
+  const int entries = n / RE;
+  double u = 0.0;   // wavefront c < 3: component c
+  double s[NV];
+  // this wavefront's records of the batch at b (past the run's end: its
+  // first; a run's last record may bring the one after it, whose term is not
+  // used)
+  auto load = [&](int b) {
+    const int e = b + PER * v;
+    const double *q = r + 6 * RE * (size_t)(e < entries ? e : 0);
 #pragma unroll
-      for (int w2 = 1; w2 < NW; w2++) t += red[w2][3 * lane + d];
-      u[d] = c * t;
+    for (int k = 0; k < NV; k++) s[k] = q[k];
+  };
+  for (int b0 = 0, buf = 0; b0 < entries; b0 += NE, buf ^= 1) {
+    load(b0);
+    if constexpr (F32) {
+      float g[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float4 f = rec_strength(s + 6 * k + 3);
+        float a[3];
+        stokeslet_term_f32_fixed(tx, ty, tz, s[6 * k], s[6 * k + 1], s[6 * k + 2], f.x, f.y, f.z, (float)e2, a[0],
+                                 a[1], a[2]);
+        for (int d = 0; d < 3; d++) g[d] = k == 0 ? a[d] : g[d] + a[d];
+      }
+      for (int d = 0; d < 3; d++) term[buf][v][d][lane] = g[d];
+    } else {
+      double ax[PER], ay[PER], az[PER];
+      stokeslet_terms_fixed<PER>(tx, ty, tz, s, e2, ax, ay, az);
+#pragma unroll
+      for (int k = 0; k < PER; k++) {
+        term[buf][PER * v + k][0][lane] = ax[k];
+        term[buf][PER * v + k][1][lane] = ay[k];
+        term[buf][PER * v + k][2][lane] = az[k];
+      }
     }
-    const Slots S = slots(p, poff, voff, nsw);
-    const int64_t i = i0 + lane, loc = i - pb;
-    const int b = pbody[i];
-    if (b >= 0) {
-      const double rx = rot[3 * i], ry = rot[3 * i + 1], rz = rot[3 * i + 2];
-      const double wx = x[S.w(0, b)], wy = x[S.w(1, b)], wz = x[S.w(2, b)];
-      u[0] -= x[S.u(0, b)] + (wy * rz - wz * ry);
-      u[1] -= x[S.u(1, b)] + (wz * rx - wx * rz);
-      u[2] -= x[S.u(2, b)] + (wx * ry - wy * rx);
+    __syncthreads();
+    if (v < 3) {
+      const int cnt = min(NE, entries - b0);
+      if (cnt == NE) {
+#pragma unroll
+        for (int k = 0; k < NE; k++) u += (double)term[buf][k][v][lane];
+      } else {
+        for (int k = 0; k < cnt; k++) u += (double)term[buf][k][v][lane];
+      }
     }
-    for (int d = 0; d < 3; d++) y[S.f(d, loc)] = u[d];
   }
-  NNK_PERSISTENT_LOOP_END
+  if (v >= 3) return;
+  if constexpr (F32) {   // up to three sources left over: one FP64 addition each
+    for (int j = 4 * entries; j < n; j++) {
+      const double *q = r + 6 * (size_t)j;
+      const float4 f = rec_strength(q + 3);
+      float a[3];
+      stokeslet_term_f32_fixed(tx, ty, tz, q[0], q[1], q[2], f.x, f.y, f.z, (float)e2, a[0], a[1], a[2]);
+      u += (double)(v == 0 ? a[0] : v == 1 ? a[1] : a[2]);
+    }
+  }
+  P[((size_t)it.slot * 3 + v) * kTile + lane] = u;
+}
+
+// a point's pair sum: its tile's runs in order (slot0: the problem's first)
+__device__ __forceinline__ void run_sum(const double *__restrict__ P, int32_t slot0, int64_t loc, double u[3]) {
+  const double *q = P + ((size_t)slot0 + (size_t)(loc / kTile) * kRuns) * (3 * kTile) + loc % kTile;
+  for (int d = 0; d < 3; d++) u[d] = q[kTile * d];
+#pragma unroll
+  for (int k = 1; k < kRuns; k++) {
+    q += 3 * kTile;
+    for (int d = 0; d < 3; d++) u[d] += q[kTile * d];
+  }
+}
+
+// forward: u_i = c sum_q S(x_i - y_q) g_q, then + BT (U; W) on body points
+__global__ void k_bfinish(int64_t ntot, const int32_t *__restrict__ ppid, const int32_t *__restrict__ slot0,
+                          const double *__restrict__ P, const int64_t *__restrict__ poff,
+                          const int64_t *__restrict__ voff, const int32_t *__restrict__ nsw,
+                          const double *__restrict__ rot, const int32_t *__restrict__ pbody,
+                          const int32_t *__restrict__ active, double c, const double *__restrict__ x,
+                          double *__restrict__ y) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ntot) return;
+  const int p = ppid[i];
+  if (!active[p]) return;
+  const int64_t loc = i - poff[p];
+  double u[3];
+  run_sum(P, slot0[p], loc, u);
+  for (int d = 0; d < 3; d++) u[d] *= c;
+  const Slots S = slots(p, poff, voff, nsw);
+  const int b = pbody[i];
+  if (b >= 0) {
+    const double rx = rot[3 * i], ry = rot[3 * i + 1], rz = rot[3 * i + 2];
+    const double wx = x[S.w(0, b)], wy = x[S.w(1, b)], wz = x[S.w(2, b)];
+    u[0] -= x[S.u(0, b)] + (wy * rz - wz * ry);
+    u[1] -= x[S.u(1, b)] + (wz * rx - wx * rz);
+    u[2] -= x[S.u(2, b)] + (wx * ry - wy * rx);
+  }
+  for (int d = 0; d < 3; d++) y[S.f(d, loc)] = u[d];
+}
+
+// transpose: v_q = c sum_i S(y_q - x_i) l_i over the problem's force points
+__global__ void k_bfinishT(int64_t qtot, const int32_t *__restrict__ fpid, const int32_t *__restrict__ slot0,
+                           const double *__restrict__ P, const int64_t *__restrict__ foff,
+                           const int32_t *__restrict__ active, double c, double *__restrict__ v) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= qtot) return;
+  const int p = fpid[q];
+  if (!active[p]) return;
+  double u[3];
+  run_sum(P, slot0[p], q - foff[p], u);
+  for (int d = 0; d < 3; d++) v[3 * q + d] = c * u[d];
 }
 
 // B f per body: [sum_j w_j f_j ; sum_j pm_j x f_j] into the body's rows
@@ -210,55 +353,6 @@ __global__ __launch_bounds__(256) void k_bB(const int32_t *__restrict__ bprob, c
   }
   if (threadIdx.x < 3) y[S.u(threadIdx.x, lb)] = red[threadIdx.x][0];
   else if (threadIdx.x < 6) y[S.w(threadIdx.x - 3, lb)] = red[threadIdx.x][0];
-}
-
-// transpose P2P: v_q = c sum_i S(y_q - x_i) l_i over the problem's force
-// points (l = the force-point block of the adjoint vector)
-template <bool F32>
-__global__ __launch_bounds__(256) void k_bp2pT(int nitems, const int2 *__restrict__ items, int *counter,
-                                               const int64_t *__restrict__ poff, const int64_t *__restrict__ foff,
-                                               const int64_t *__restrict__ voff, const double *__restrict__ pts,
-                                               const double *__restrict__ fine, const double *__restrict__ eps,
-                                               const int32_t *__restrict__ active, double c,
-                                               const double *__restrict__ x, double *__restrict__ v) {
-  __shared__ SrcStage<F32, 256> st;
-  __shared__ double red[4][kTile * 3];
-  __shared__ int item_s;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  NNK_PERSISTENT_LOOP_BEGIN
-  const int64_t qb = foff[p], Qp = foff[p + 1] - qb;
-  const int64_t q0t = qb + (int64_t)kTile * tile;
-  const int nt = (int)min((int64_t)kTile, Qp - (int64_t)kTile * tile);
-  double tx = 0, ty = 0, tz = 0;
-  if (lane < nt) {
-    tx = fine[3 * (q0t + lane)];
-    ty = fine[3 * (q0t + lane) + 1];
-    tz = fine[3 * (q0t + lane) + 2];
-  }
-  const double e2 = eps[p] * eps[p];
-  const int64_t pb = poff[p], Np = poff[p + 1] - pb, base = voff[p];
-  double ux = 0, uy = 0, uz = 0;
-  for (int64_t s0 = 0; s0 < Np; s0 += 256) {
-    const int cnt = (int)min((int64_t)256, Np - s0);
-    if (tid < cnt) {
-      const int64_t i = pb + s0 + tid;
-      st.put(tid, pts[3 * i], pts[3 * i + 1], pts[3 * i + 2], x[base + s0 + tid], x[base + Np + s0 + tid],
-             x[base + 2 * Np + s0 + tid]);
-    }
-    __syncthreads();
-    if (lane < nt)
-      st.run(wv, 4, cnt, tx, ty, tz, e2, ux, uy, uz);
-    __syncthreads();
-  }
-  red[wv][3 * lane] = ux;
-  red[wv][3 * lane + 1] = uy;
-  red[wv][3 * lane + 2] = uz;
-  __syncthreads();
-  if (wv == 0 && lane < nt)
-    for (int d = 0; d < 3; d++)
-      v[3 * (q0t + lane) + d] =
-          c * (((red[0][3 * lane + d] + red[1][3 * lane + d]) + red[2][3 * lane + d]) + red[3][3 * lane + d]);
-  NNK_PERSISTENT_LOOP_END
 }
 
 // transpose force-point rows: mu_j = sum_q NN(q,j) v_q + [body b] (w_j lF_b + lM_b x pm_j)
@@ -624,6 +718,21 @@ Batch::Batch(int nprob, const int64_t *pt_off, const double *pts, const int64_t 
     return sorted;
   };
   auto it_f = make_items(false), it_t = make_items(true);
+  std::vector<BatchItem> sum_f, sum_t;
+  std::vector<int32_t> slot_f, slot_t;
+  hfoff_ = hfoff;
+  const int64_t slots = std::max(pair_items(false, sum_f, slot_f), pair_items(true, sum_t, slot_t));
+  nsums_ = (int)sum_f.size();
+  nsumsT_ = (int)sum_t.size();
+  sums_.upload(sum_f);
+  sumsT_.upload(sum_t);
+  slot0_.upload(slot_f);
+  slot0T_.upload(slot_t);
+  sumbuf_.alloc(sizeof(double) * 3 * kTile * (size_t)std::max<int64_t>(slots, 1));
+  std::vector<int32_t> fpid(qtot_);
+  for (int p = 0; p < nprob; p++)
+    for (int64_t q = hfoff[p]; q < hfoff[p + 1]; q++) fpid[q] = p;
+  fpid_.upload(fpid);
   nitems_ = (int)it_f.size();
   nitemsT_ = (int)it_t.size();
   poff_.upload(hpoff_);
@@ -656,35 +765,51 @@ Batch::Batch(int nprob, const int64_t *pt_off, const double *pts, const int64_t 
   counter_.alloc(sizeof(int));
   g_.alloc(sizeof(double) * 3 * std::max<int64_t>(qtot_, 1));
   v_.alloc(sizeof(double) * 3 * std::max<int64_t>(qtot_, 1));
+  // one record more: the FP64 sums read records in pairs
+  rec_.alloc(sizeof(double) * 6 * (size_t)(std::max(qtot_, ntot_) + kRuns * (int64_t)nprob + 1));
   active_.upload(std::vector<int32_t>(nprob, 1));
   pidf_.upload(ppid);
+}
+
+// pair-sum items, most expensive first; slots number (problem, tile, run) in
+// order
+int64_t Batch::pair_items(bool transpose, std::vector<BatchItem> &items, std::vector<int32_t> &slot0) const {
+  const std::vector<int64_t> &to = transpose ? hfoff_ : hpoff_, &so = transpose ? hpoff_ : hfoff_;
+  int64_t slot = 0;
+  for (int p = 0; p < np_; p++) {
+    slot0.push_back((int32_t)slot);
+    for (int64_t t = 0; t * kTile < to[p + 1] - to[p]; t++)
+      for (int w = 0; w < kRuns; w++) items.push_back({p, (int)t, w, (int)slot++});
+    if (slot > INT32_MAX) throw Error(NNK_EARG, "batch: too many points");
+  }
+  std::stable_sort(items.begin(), items.end(), [&](const BatchItem &a, const BatchItem &b) {
+    return so[a.p + 1] - so[a.p] > so[b.p + 1] - so[b.p];
+  });
+  return slot;
+}
+
+void Batch::pair_sums(const DBuf &items, int n, bool transpose, hipStream_t s) {
+  if (!n) return;
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * (f32_ ? kSumWaves<true> : kSumWaves<false>)), 0, s, items.as<BatchItem>(),
+                       (transpose ? foff_ : poff_).as<int64_t>(), (transpose ? poff_ : foff_).as<int64_t>(),
+                       (transpose ? fine_ : pts_).as<double>(), rec_.as<double>(), eps_.as<double>(),
+                       active_.as<int32_t>(), sumbuf_.as<double>());
+  };
+  if (f32_) launch(k_bsum<true>);
+  else launch(k_bsum<false>);
 }
 
 void Batch::op(const double *x, double *y, hipStream_t s) {
   if (qtot_)
     hipLaunchKernelGGL(k_bgather, dim3(nblk(qtot_)), dim3(256), 0, s, qtot_, nnptr_.as<int64_t>(),
                        nncol_.as<int32_t>(), nnval_.as<double>(), x, xbase_.as<int64_t>(),
-                       xstride_.as<int64_t>(), g_.as<double>());
-  hipLaunchKernelGGL(k_bcounter_reset, dim3(1), dim3(64), 0, s, counter_.as<int>());
-  // persistent grid: about 256k threads whatever the workgroup size
-  const int NW = p2p_waves_;
-  const unsigned grid = (unsigned)std::max(1, std::min(nitems_, 1024 * 4 / NW));
-  const double c = 1.0 / (8.0 * kPi * mu_);
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), 0, s, nitems_, items_.as<int2>(), counter_.as<int>(),
-                       poff_.as<int64_t>(), foff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(),
-                       pts_.as<double>(), fine_.as<double>(), g_.as<double>(), rot_.as<double>(),
-                       pbody_.as<int32_t>(), eps_.as<double>(), active_.as<int32_t>(), c, x, y);
-  };
-  if (f32_) {
-    if (NW == 1) launch(k_bp2p<true, 1>);
-    else if (NW == 2) launch(k_bp2p<true, 2>);
-    else launch(k_bp2p<true, 4>);
-  } else {
-    if (NW == 1) launch(k_bp2p<false, 1>);
-    else if (NW == 2) launch(k_bp2p<false, 2>);
-    else launch(k_bp2p<false, 4>);
-  }
+                       xstride_.as<int64_t>(), g_.as<double>(), rec_.as<double>(), f32_ != 0, fpid_.as<int32_t>(),
+                       foff_.as<int64_t>(), fine_.as<double>());
+  pair_sums(sums_, nsums_, false, s);
+  hipLaunchKernelGGL(k_bfinish, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, pidf_.as<int32_t>(), slot0_.as<int32_t>(),
+                     sumbuf_.as<double>(), poff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(),
+                     rot_.as<double>(), pbody_.as<int32_t>(), active_.as<int32_t>(), 1.0 / (8.0 * kPi * mu_), x, y);
   if (nbody_)
     hipLaunchKernelGGL(k_bB, dim3(nbody_), dim3(256), 0, s, bprob_.as<int32_t>(), blocal_.as<int32_t>(),
                        bpt_.as<int64_t>(), poff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(),
@@ -693,18 +818,14 @@ void Batch::op(const double *x, double *y, hipStream_t s) {
 }
 
 void Batch::opT(const double *x, double *y, hipStream_t s) {
-  const double c = 1.0 / (8.0 * kPi * mu_);
-  if (nitemsT_) {
-    hipLaunchKernelGGL(k_bcounter_reset, dim3(1), dim3(64), 0, s, counter_.as<int>());
-    const unsigned grid = (unsigned)std::max(1, std::min(nitemsT_, 1024));
-    auto launch = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, nitemsT_, itemsT_.as<int2>(), counter_.as<int>(),
-                         poff_.as<int64_t>(), foff_.as<int64_t>(), voff_.as<int64_t>(), pts_.as<double>(),
-                         fine_.as<double>(), eps_.as<double>(), active_.as<int32_t>(), c, x, v_.as<double>());
-    };
-    if (f32_) launch(k_bp2pT<true>);
-    else launch(k_bp2pT<false>);
-  }
+  hipLaunchKernelGGL(k_brecordT, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, x, xbase_.as<int64_t>(),
+                     xstride_.as<int64_t>(), rec_.as<double>(), f32_ != 0, pidf_.as<int32_t>(), poff_.as<int64_t>(),
+                     pts_.as<double>());
+  pair_sums(sumsT_, nsumsT_, true, s);
+  if (qtot_)
+    hipLaunchKernelGGL(k_bfinishT, dim3(nblk(qtot_)), dim3(256), 0, s, qtot_, fpid_.as<int32_t>(),
+                       slot0T_.as<int32_t>(), sumbuf_.as<double>(), foff_.as<int64_t>(), active_.as<int32_t>(),
+                       1.0 / (8.0 * kPi * mu_), v_.as<double>());
   hipLaunchKernelGGL(k_bgatherT, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, pidf_.as<int32_t>(),
                      nntptr_.as<int64_t>(), nntrow_.as<int32_t>(), nntval_.as<double>(), v_.as<double>(),
                      poff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(), w_.as<double>(), pm_.as<double>(),
@@ -716,50 +837,7 @@ void Batch::opT(const double *x, double *y, hipStream_t s) {
   NNK_HIP(hipGetLastError());
 }
 
-// time the forward operator with 1, 2 and 4 wavefronts per P2P workgroup
-// (on the caller's vectors; y is overwritten) and keep the fastest
-void Batch::autotune_p2p(const double *x, double *y, hipStream_t s) {
-  // time every problem, then restore the caller's active flags
-  std::vector<int32_t> saved(np_), act(np_, 1);
-  NNK_HIP(hipMemcpyAsync(saved.data(), active_.p, sizeof(int32_t) * np_, hipMemcpyDeviceToHost, s));
-  NNK_HIP(hipStreamSynchronize(s));
-  NNK_HIP(hipMemcpyAsync(active_.p, act.data(), sizeof(int32_t) * np_, hipMemcpyHostToDevice, s));
-  hipEvent_t a, b;
-  NNK_HIP(hipEventCreate(&a));
-  NNK_HIP(hipEventCreate(&b));
-  float best = 1e30f;
-  int bw = p2p_waves_;
-  try {
-    for (int nw : {1, 2, 4}) {
-      p2p_waves_ = nw;
-      op(x, y, s);  // warm
-      NNK_HIP(hipEventRecord(a, s));
-      op(x, y, s);
-      op(x, y, s);
-      NNK_HIP(hipEventRecord(b, s));
-      NNK_HIP(hipEventSynchronize(b));
-      float ms = 0;
-      NNK_HIP(hipEventElapsedTime(&ms, a, b));
-      if (ms < best) { best = ms; bw = nw; }
-    }
-  } catch (...) {
-    p2p_waves_ = bw;
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
-    throw;
-  }
-  p2p_waves_ = bw;
-  NNK_HIP(hipMemcpyAsync(active_.p, saved.data(), sizeof(int32_t) * np_, hipMemcpyHostToDevice, s));
-  NNK_HIP(hipStreamSynchronize(s));
-  NNK_HIP(hipEventDestroy(a));
-  NNK_HIP(hipEventDestroy(b));
-}
-
 void Batch::apply(const double *x, double *y, bool transpose, hipStream_t s) {
-  if (tune_ && !tuned_) {  // outside any graph capture
-    autotune_p2p(x, y, s);
-    tuned_ = true;
-  }
   if (!graph_) {
     if (transpose) opT(x, y, s);
     else op(x, y, s);
@@ -918,7 +996,7 @@ void Batch::gradient(const double *z, const double *lambda, double *gx, double *
   if (qtot_)
     hipLaunchKernelGGL(k_bgather, dim3(nblk(qtot_)), dim3(256), 0, s, qtot_, nnptr_.as<int64_t>(),
                        nncol_.as<int32_t>(), nnval_.as<double>(), z, xbase_.as<int64_t>(),
-                       xstride_.as<int64_t>(), g_.as<double>());
+                       xstride_.as<int64_t>(), g_.as<double>(), nullptr, false, nullptr, nullptr, nullptr);
   const double c = 1.0 / (8.0 * kPi * mu_);
   DBuf ge;
   ge.alloc(sizeof(double) * ntot_);

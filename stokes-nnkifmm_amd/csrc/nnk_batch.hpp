@@ -13,10 +13,10 @@
 //
 // All problems share one device vector [x_0; x_1; ...], x_p =
 // [f (3 N_p, all x, all y, all z); U (3 nsw_p: all x, all y, all z);
-// Omega (3 nsw_p)].  The operator is three launches: the quadrature
-// strengths g = (NN (x) I3) f, a persistent P2P kernel that walks
-// (problem, 64-target tile) work items largest first and adds BT (U; W),
-// and one workgroup per body for B f.  The transpose (adjoint) operator
+// Omega (3 nsw_p)].  The operator is four launches: the quadrature
+// strengths g = (NN (x) I3) f, the pair sums of (problem, 64-target tile,
+// source part) work items largest first, the sums of their parts plus
+// BT (U; W), and one workgroup per body for B f.  The transpose (adjoint) operator
 // runs the P2P from force points onto quadrature points and gathers with
 // NN^T.  GMRES runs all problems in lockstep (segmented dot products,
 // per-problem Givens on the host) and retires each problem as it converges.
@@ -36,6 +36,12 @@
 
 namespace nnk {
 
+// one workgroup of the pair sums: run `run` of problem p's sources onto its
+// 64-target tile `tile`, sums to slot `slot`
+struct BatchItem {
+  int32_t p, tile, run, slot;
+};
+
 class Batch {
  public:
   // pt_body: body of each force point, local to its problem (0..nsw_p-1)
@@ -50,9 +56,8 @@ class Batch {
   // y = A x (transpose: y = A^T x) for every problem (device vectors)
   void apply(const double *x, double *y, bool transpose, hipStream_t s);
   void set_graph(bool on) { graph_ = on; }
-  // time the P2P workgroup size (1, 2, 4 wavefronts) on the first apply
-  void set_autotune(bool on) { tune_ = on; }
-  int p2p_waves() const { return p2p_waves_; }
+  // runs a tile's sources are summed in (wavefronts that used to share them)
+  int p2p_waves() const { return 4; }
   // unrestarted GMRES from x = 0 per problem on A (or A^T); per-problem
   // flag (0 when the recomputed relative residual is <= tol), that residual
   // and the iteration count.  With FP32-math operators the Arnoldi
@@ -66,23 +71,29 @@ class Batch {
 
  private:
   void op(const double *x, double *y, hipStream_t s);
-  void autotune_p2p(const double *x, double *y, hipStream_t s);
   void opT(const double *x, double *y, hipStream_t s);
+  // work items of the pair sums and the problems' first slots (returns the
+  // slots in all); the sums of a list of items into sumbuf_ (transpose: force
+  // points onto quadrature points)
+  int64_t pair_items(bool transpose, std::vector<BatchItem> &items, std::vector<int32_t> &slot0) const;
+  void pair_sums(const DBuf &items, int n, bool transpose, hipStream_t s);
   void segdots(int k, const double *V, const double *w, double *host_out, hipStream_t s);
 
   int np_ = 0, nbody_ = 0;
   int64_t ntot_ = 0, qtot_ = 0, n_ = 0;
   double mu_ = 1.0;
   int f32_ = 0;
-  std::vector<int64_t> hpoff_, hvoff_;
+  std::vector<int64_t> hpoff_, hfoff_, hvoff_;
   DBuf poff_, foff_, voff_, pts_, fine_, nnptr_, nncol_, nnval_, nntptr_, nntrow_, nntval_;
   DBuf w_, pm_, rot_, eps_, pbody_, fbody_, nsw_;
   DBuf bprob_, blocal_, bpt_;  // per body: problem, local index, point range
   DBuf xbase_, xstride_, pid_, pidf_, items_, itemsT_, counter_, g_, v_, active_, part_;
   int nitems_ = 0, nitemsT_ = 0;
+  // pair sums: items, problems' first slots, sums, quadrature points'
+  // problems, source records
+  DBuf sums_, sumsT_, slot0_, slot0T_, sumbuf_, fpid_, rec_;
+  int nsums_ = 0, nsumsT_ = 0;
   bool graph_ = false;
-  bool tune_ = false, tuned_ = false;
-  int p2p_waves_ = 4;
   GraphOp gop_[2];
 };
 

@@ -589,7 +589,7 @@ int32_t nnk_batch_set_graph(nnk_batch *h, int32_t on) {
 int32_t nnk_batch_set_autotune(nnk_batch *h, int32_t on) {
   return guard([&]() -> int32_t {
     if (!h) return fail(NNK_EARG, "nnk_batch_set_autotune: null handle");
-    h->b->set_autotune(on != 0);
+    (void)on;   // the pair sums have one launch shape
     return NNK_OK;
   });
 }

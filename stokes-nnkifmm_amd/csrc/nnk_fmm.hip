@@ -419,7 +419,7 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
   // L2T, the smaller W node for M2T); the U-list sources keep the FP64
   // separation
   __shared__ union {
-    SrcStage<true, T> pts;
+    SrcStage<T> pts;
     SrcStageRel<T> srf;
   } st;
   __shared__ double red[T * 3];

@@ -83,6 +83,67 @@ __device__ __forceinline__ void stokeslet_acc64(double tx, double ty, double tz,
   uz = __builtin_fma(iso, qz, __builtin_fma(rq, rz, uz));
 }
 
+// The terms of stokeslet_acc of the N sources v[6 k ..] (position, strength),
+// stage by stage so that their dependent chains overlap, every rounding
+// written out: the sums of batched solves keep the roundings they were
+// defined with (their GMRES turns a last-bit change into 1e-8 of the
+// solution), whatever the compiler contracts elsewhere.
+template <int N>
+__device__ __forceinline__ void stokeslet_terms_fixed(double tx, double ty, double tz, const double (&v)[6 * N],
+                                                      double e2, double (&rx)[N], double (&ry)[N], double (&rz)[N]) {
+#pragma clang fp contract(off)
+  double re[N], y[N], e[N], rq[N], iso[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    rx[k] = tx - v[6 * k];
+    ry[k] = ty - v[6 * k + 1];
+    rz[k] = tz - v[6 * k + 2];
+  }
+#pragma unroll
+  for (int k = 0; k < N; k++) re[k] = ry[k] * ry[k];
+#pragma unroll
+  for (int k = 0; k < N; k++) re[k] = __builtin_fma(rx[k], rx[k], re[k]);
+#pragma unroll
+  for (int k = 0; k < N; k++) re[k] = __builtin_fma(rz[k], rz[k], re[k]);
+#pragma unroll
+  for (int k = 0; k < N; k++) re[k] = re[k] + e2;
+#pragma unroll
+  for (int k = 0; k < N; k++) y[k] = __builtin_amdgcn_rsq(re[k]);
+#pragma unroll
+  for (int k = 0; k < N; k++) rq[k] = ry[k] * v[6 * k + 4];
+#pragma unroll
+  for (int k = 0; k < N; k++) rq[k] = __builtin_fma(rx[k], v[6 * k + 3], rq[k]);
+#pragma unroll
+  for (int k = 0; k < N; k++) rq[k] = __builtin_fma(rz[k], v[6 * k + 5], rq[k]);
+#pragma unroll
+  for (int k = 0; k < N; k++) e[k] = re[k] * y[k];
+#pragma unroll
+  for (int k = 0; k < N; k++) e[k] = __builtin_fma(-e[k], y[k], 1.0);
+#pragma unroll
+  for (int k = 0; k < N; k++) iso[k] = re[k] + e2;
+#pragma unroll
+  for (int k = 0; k < N; k++) re[k] = __builtin_fma(e[k], 0.375, 0.5);
+#pragma unroll
+  for (int k = 0; k < N; k++) e[k] = y[k] * e[k];
+#pragma unroll
+  for (int k = 0; k < N; k++) y[k] = __builtin_fma(e[k], re[k], y[k]);
+#pragma unroll
+  for (int k = 0; k < N; k++) re[k] = y[k] * y[k];
+#pragma unroll
+  for (int k = 0; k < N; k++) y[k] = y[k] * re[k];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    iso[k] = iso[k] * y[k];
+    rq[k] = rq[k] * y[k];
+  }
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    rx[k] = __builtin_fma(v[6 * k + 3], iso[k], rx[k] * rq[k]);
+    ry[k] = __builtin_fma(v[6 * k + 4], iso[k], ry[k] * rq[k]);
+    rz[k] = __builtin_fma(v[6 * k + 5], iso[k], rz[k] * rq[k]);
+  }
+}
+
 // Mixed form: the separation r = t - s is formed in FP64 (so near pairs keep
 // their digits), the kernel is evaluated in FP32 with the hardware reciprocal
 // square root, and the result is accumulated in FP64.  The strength comes in
@@ -104,41 +165,27 @@ __device__ __forceinline__ void stokeslet_acc_f32q(double tx, double ty, double 
   uz += (double)(iso * fz + rq * rz);
 }
 
-__device__ __forceinline__ void stokeslet_acc_f32(double tx, double ty, double tz, double sx,
-                                                  double sy, double sz, double qx, double qy,
-                                                  double qz, double e2, double &ux, double &uy,
-                                                  double &uz) {
-  stokeslet_acc_f32q(tx, ty, tz, sx, sy, sz, (float)qx, (float)qy, (float)qz, e2, ux, uy, uz);
+// the FP32 term of one source (stokeslet_acc_f32q before its FP64 addition),
+// every rounding written out
+__device__ __forceinline__ void stokeslet_term_f32_fixed(double tx, double ty, double tz, double sx, double sy,
+                                                         double sz, float fx, float fy, float fz, float e2f, float &gx,
+                                                         float &gy, float &gz) {
+#pragma clang fp contract(off)
+  const float rx = (float)(tx - sx), ry = (float)(ty - sy), rz = (float)(tz - sz);
+  const float re = __builtin_fmaf(rz, rz, __builtin_fmaf(rx, rx, ry * ry)) + e2f;
+  const float inv = __builtin_amdgcn_rsqf(re);
+  const float inv3 = inv * (inv * inv);
+  const float iso = __builtin_fmaf(e2f, inv3, inv);  // (re + e2) / re^1.5
+  const float rq = __builtin_fmaf(rz, fz, __builtin_fmaf(rx, fx, ry * fy)) * inv3;
+  gx = __builtin_fmaf(fx, iso, rq * rx);
+  gy = __builtin_fmaf(fy, iso, rq * ry);
+  gz = __builtin_fmaf(fz, iso, rq * rz);
 }
 
-// LDS stage of up to T sources: positions in FP64; strengths in FP64, or,
-// for the FP32-math form, rounded to FP32 once when staged (the values the
-// pair routine would otherwise round per pair).  acc(j, ...) adds source j.
-template <bool F32, int T> struct SrcStage;
-template <int T> struct SrcStage<false, T> {
-  double p[3 * T], q[3 * T];
-  __device__ __forceinline__ void put(int i, double x, double y, double z, double qx, double qy, double qz) {
-    p[3 * i] = x; p[3 * i + 1] = y; p[3 * i + 2] = z;
-    q[3 * i] = qx; q[3 * i + 1] = qy; q[3 * i + 2] = qz;
-  }
-  __device__ __forceinline__ void acc(int j, double tx, double ty, double tz, double e2, double &ux,
-                                      double &uy, double &uz) const {
-    stokeslet_acc(tx, ty, tz, p[3 * j], p[3 * j + 1], p[3 * j + 2], q[3 * j], q[3 * j + 1], q[3 * j + 2], e2,
-                  ux, uy, uz);
-  }
-  // sources j = j0, j0 + step, ... < cnt, four per iteration (the same
-  // sequence of FP64 accumulations as one at a time)
-  __device__ __forceinline__ void run(int j0, int step, int cnt, double tx, double ty, double tz, double e2,
-                                      double &ux, double &uy, double &uz) const {
-    int j = j0;
-    for (; j + 3 * step < cnt; j += 4 * step) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) acc(j + k * step, tx, ty, tz, e2, ux, uy, uz);
-    }
-    for (; j < cnt; j += step) acc(j, tx, ty, tz, e2, ux, uy, uz);
-  }
-};
-template <int T> struct SrcStage<true, T> {
+// FP32-math forms: LDS stage of up to T sources, positions in FP64, strengths
+// rounded to FP32 once when staged (the values the pair routine would
+// otherwise round per pair).  acc(j, ...) adds source j.
+template <int T> struct SrcStage {
   double p[3 * T];
   __attribute__((aligned(16))) float q[4 * T];
   __device__ __forceinline__ void put(int i, double x, double y, double z, double qx, double qy, double qz) {
@@ -242,14 +289,6 @@ __device__ __forceinline__ void box_centre(const double *__restrict__ box, doubl
   cx = 0.5 * (box[0] + box[3]);
   cy = 0.5 * (box[1] + box[4]);
   cz = 0.5 * (box[2] + box[5]);
-}
-
-template <bool F32>
-__device__ __forceinline__ void stk(double tx, double ty, double tz, double sx, double sy, double sz,
-                                    double qx, double qy, double qz, double e2, double &ux, double &uy,
-                                    double &uz) {
-  if constexpr (F32) stokeslet_acc_f32(tx, ty, tz, sx, sy, sz, qx, qy, qz, e2, ux, uy, uz);
-  else stokeslet_acc(tx, ty, tz, sx, sy, sz, qx, qy, qz, e2, ux, uy, uz);
 }
 
 }  // namespace nnk
