@@ -342,10 +342,10 @@ __device__ __forceinline__ void sum_sources(const double (&tx)[NT], const double
   }
 }
 
-// The FP64 form of P2L: a wavefront per NT surface points of a node, the
-// sources of its X list on lanes.
+// The FP64 form of P2L, and of S2M for leaves of many sources: a wavefront per
+// NT surface points of a node, the sources of its X list, or its own, on lanes.
 template <int NT>
-__global__ __launch_bounds__(256) void k_p2l64(SurfArgs a, const double *__restrict__ src_pos,
+__global__ __launch_bounds__(256) void k_surf64(SurfArgs a, const double *__restrict__ src_pos,
                                                const double *__restrict__ src_q) {
   __shared__ int pre[kLeafMaxU + 1];
   __shared__ SrcBatch buf;
@@ -363,16 +363,24 @@ __global__ __launch_bounds__(256) void k_p2l64(SurfArgs a, const double *__restr
     tz[k] = lane_value(lz, k);
     u[3 * k] = u[3 * k + 1] = u[3 * k + 2] = 0.0;
   }
-  const int64_t lb = a.lptr[n], le = a.lptr[n + 1];
-  for (int64_t b0 = lb; b0 < le; b0 += kLeafMaxU) {
-    const int nu = (int)min((int64_t)kLeafMaxU, le - b0);
-    const int32_t *list = a.lidx + b0;
-    if (b0 > lb) __syncthreads();
-    source_prefix(list, nu, a.src_ptr, pre);
-    sum_sources<NT>(tx, ty, tz, a.e2, p0 < a.nq ? 0 : 4, 1, pre[nu], buf, [&](int g) {
-      const size_t j = 3 * (size_t)source_index(list, nu, a.src_ptr, pre, g);
-      return Src6{src_pos[j], src_pos[j + 1], src_pos[j + 2], src_q[j], src_q[j + 1], src_q[j + 2]};
-    }, u);
+  auto source = [&](int s) {
+    const size_t j = 3 * (size_t)s;
+    return Src6{src_pos[j], src_pos[j + 1], src_pos[j + 2], src_q[j], src_q[j + 1], src_q[j + 2]};
+  };
+  const int sp = p0 < a.nq ? 0 : 4;   // a wavefront past the last point takes no chunk
+  if (a.lptr) {
+    const int64_t lb = a.lptr[n], le = a.lptr[n + 1];
+    for (int64_t b0 = lb; b0 < le; b0 += kLeafMaxU) {
+      const int nu = (int)min((int64_t)kLeafMaxU, le - b0);
+      const int32_t *list = a.lidx + b0;
+      if (b0 > lb) __syncthreads();
+      source_prefix(list, nu, a.src_ptr, pre);
+      sum_sources<NT>(tx, ty, tz, a.e2, sp, 1, pre[nu], buf,
+                      [&](int g) { return source(source_index(list, nu, a.src_ptr, pre, g)); }, u);
+    }
+  } else {
+    const int sb = a.src_ptr[n];
+    sum_sources<NT>(tx, ty, tz, a.e2, sp, 1, a.src_ptr[n + 1] - sb, buf, [&](int g) { return source(sb + g); }, u);
   }
   if (p0 >= a.nq) return;
   int idx = 0, cnt = 3 * min(NT, a.nq - p0);
@@ -1864,9 +1872,15 @@ void Fmm::launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const in
   a.e2 = eps_ * eps_;
   a.c = 1.0 / (8.0 * kPi * mu_);
   a.chk = chk;
+  // FP64 S2M: k_s2m64 walks a leaf's sources one after the other on three
+  // wavefronts; from 64 sources per leaf on average a chunk of k_surf64 is
+  // full and the leaf's sources are read by all its wavefronts.  Both sides
+  // at res 6: ten bodies over a wall, capacity 500, 68 -> 7.9 us; 128 sources
+  // in each of 512 leaves 30 -> 22.6 us; 32 in each of 32,768 0.19 against
+  // 0.50 ms.
   if (fp32_math()) hipLaunchKernelGGL(k_surf_eval, dim3(n), dim3(kSurfThreads), 0, s, a);
-  else if (lptr)
-    hipLaunchKernelGGL(k_p2l64<8>, dim3(n, (nq_ + 31) / 32), dim3(256), 0, s, a, a.src_pos, a.src_q);
+  else if (lptr || nsrc_ >= 64 * (int64_t)n)
+    hipLaunchKernelGGL(k_surf64<8>, dim3(n, (nq_ + 31) / 32), dim3(256), 0, s, a, a.src_pos, a.src_q);
   else
     hipLaunchKernelGGL(k_s2m64, dim3(n), dim3(64 * std::min((nq_ + 63) / 64, 8)), 0, s, a, a.src_pos, a.src_q);
   NNK_HIP(hipGetLastError());

@@ -85,3 +85,17 @@ def test_surface_point_counts(oracle, nnk, res):
     u = nnk.KIFMM(tree, [1e-3, 1.0], "coronaRes", res).computeVel(q)
     uo = oracle.Tree(p, p, nodeCapacity=16).matvec(q, 1e-3, 1.0, res, 1)
     assert np.linalg.norm(u - uo) <= 1e-10 * np.linalg.norm(uo)
+
+
+@pytest.mark.parametrize("cap,n", [(100, 4500), (180, 9000), (400, 20000)])
+def test_s2m_of_large_leaves(oracle, nnk, cap, n):
+    """Leaves of 64 sources and more on average take their sources on lanes:
+    chunks of 64 and batches of 256, with remainders."""
+    rng = np.random.default_rng(n + cap)
+    p = np.concatenate([[[0, 0, 0], [1, 1, 1.0]], rng.random((n, 3))])
+    tree = nnk.OcTree(p, p, "nodeCapacity", cap)
+    assert tree.nodeCount == 73   # 64 leaves
+    q = rng.standard_normal(p.shape)
+    u = nnk.KIFMM(tree, [1e-3, 1.0], "coronaRes", 4).computeVel(q)
+    uo = oracle.Tree(p, p, nodeCapacity=cap).matvec(q, 1e-3, 1.0, 4, 1)
+    assert np.linalg.norm(u - uo) <= 1e-10 * np.linalg.norm(uo)
