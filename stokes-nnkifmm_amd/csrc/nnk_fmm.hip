@@ -1055,6 +1055,9 @@ void Fmm::split_reduce(const DBuf &slot, int ncols, int M, int ldc, int nsplit, 
   NNK_HIP(hipGetLastError());
 }
 
+// The truncated forms keep one summation order: what they compute here is
+// rounded to 16-bit parts next, and a value moved by one FP64 rounding can move
+// its parts (5e-9 to 6e-8 of the velocities).
 void Fmm::gemm_dims(const GemmBatch &b, const double *X, int ldx, double *C, int ldc, int beta,
                     hipStream_t s, int M, int K, int Mpad, int Kpad, int nsplit, const DBuf *slot, int tag) {
   if (b.njobs == 0 || b.maxN == 0) return;
@@ -1077,21 +1080,9 @@ void Fmm::gemm_dims(const GemmBatch &b, const double *X, int ldx, double *C, int
 void Fmm::gemm(const GemmBatch &b, const double *X, int ldx, double *C, int ldc, int beta,
                hipStream_t s, int tag, int nsplit, const DBuf *slot) {
   if (b.njobs == 0 || b.maxN == 0) return;
-  const int nrb = Mpad_ / GBM;
-  if (nsplit > 1) {
-    // partial tiles, then the fixed-order reduction (stores: beta must be 0)
-    if (beta != 0 || !slot) throw Error(NNK_ESTATE, "split GEMM needs beta = 0 and a slot list");
-    if ((size_t)nsplit * b.njobs * b.maxN * ldc > part_elems_) throw Error(NNK_ESTATE, "split buffer too small");
-    if (tag == 1) launch_gemm<GBN1, 1>(nrb, K_, K_, Mpad_, Kpad_, X, ldx, C, ldc, 0, b, s, nsplit, part_.as<double>());
-    else launch_gemm<GBN0, 0>(nrb, K_, K_, Mpad_, Kpad_, X, ldx, C, ldc, 0, b, s, nsplit, part_.as<double>());
-    split_reduce(*slot, b.njobs * b.maxN, K_, ldc, nsplit, C, s);
-    return;
-  }
-  if (tag == 1) {
-    launch_gemm<GBN1, 1>(nrb, K_, K_, Mpad_, Kpad_, X, ldx, C, ldc, beta, b, s);
-  } else {
-    launch_gemm<GBN0, 0>(nrb, K_, K_, Mpad_, Kpad_, X, ldx, C, ldc, beta, b, s);
-  }
+  if (tag == 1) gemm_dims(b, X, ldx, C, ldc, beta, s, K_, K_, Mpad_, Kpad_, nsplit, slot, 1);
+  else
+    launch_gemm_direct(K_, K_, Mpad_, Kpad_, X, ldx, C, ldc, beta, b.jobs.as<GemmJob>(), b.njobs, b.maxN, s);
 }
 
 Fmm::~Fmm() {
@@ -1613,12 +1604,6 @@ void Fmm::plan() {
       add_job(P.m2m, jobs, A, &g, &nl, (int)nl.size());
       finish(P.m2m, jobs);
       hl_[l].m2m_g = g;
-      const int64_t tiles = (int64_t)(Mpad_ / GBM) * (((int64_t)nl.size() + GBN0 - 1) / GBN0);
-      P.m2m_split = split_m2m(tiles, nl.size() * (size_t)K_);
-      if (P.m2m_split > 1) {
-        P.m2m_slot.upload(nl);
-        reserve_part((size_t)P.m2m_split * nl.size() * K_);
-      }
     }
     hl_[l].up_leaves = up;
     hl_[l].up_nonleaves = nl;
@@ -2144,7 +2129,7 @@ void Fmm::apply_impl(const double *d_f, double *d_u, hipStream_t s) {
   for (int l = maxlev_; l >= 2; l--) {
     LevelPlan &P = plans_[l];
     if (!P.n_up) continue;
-    gemm(P.m2m, up, K_, chk, K_, 0, s, 0, P.m2m_split, &P.m2m_slot);
+    gemm(P.m2m, up, K_, chk, K_, 0, s);
     gemm(P.up_solve1, chk, K_, tmp, K_, 0, s);
     gemm(P.up_solve2, tmp, K_, up, K_, 0, s);
   }

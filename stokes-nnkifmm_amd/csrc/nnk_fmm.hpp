@@ -17,9 +17,9 @@ namespace nnk {
 
 struct RedArgs;
 
-// rows per workgroup tile and k depth per chunk of the FP64 gather GEMM;
-// columns per tile of its M2L launches (GBN1) and of the others (GBN0:
-// expansions, M2M, L2L, check-to-equivalent solves)
+// rows per workgroup tile and k depth per chunk of the FP64 gather GEMM (the
+// operators' padding); columns per tile of its M2L launches (GBN1) and of the
+// truncated forms' expansions, M2M and L2L (GBN0)
 constexpr int GBM = 160, GBK = 16, GBN1 = 64, GBN0 = 32;
 
 struct GemmJob {
@@ -117,8 +117,6 @@ struct LevelPlan {
   int n_up = 0;
   DBuf up_nodes;              // slots (id-1)
   GemmBatch m2m;              // children -> parent check surface
-  int m2m_split = 1;          // split-K factor of the M2M launch (one or two children per part)
-  DBuf m2m_slot;              // column -> parent slot, for its split reduction
   GemmBatch up_solve1, up_solve2;
   // downward
   int n_down = 0;
@@ -149,8 +147,8 @@ struct LevelPlan {
   DBuf x_nodes;               // nodes with a non-empty X list
   // mixed form
   GemmBatch mx_m2m, mx_l2l, mx_xP;
-  int mx_m2m_split = 1;       // as m2m_split, for the mixed form's M2M
-  DBuf mx_m2m_slot;
+  int mx_m2m_split = 1;       // split-K factor of the mixed form's M2M launch (one or two children per part)
+  DBuf mx_m2m_slot;           // column -> parent slot, for its split reduction
   DBuf mx_m2l;                // GemmJobBf16[8]
   int mx_split = 1, mx_depth = 3;  // split-K factor and register-ring depth of the M2L launch
                                    // (depth 4: the DMA-staged kernel; 5: the same with

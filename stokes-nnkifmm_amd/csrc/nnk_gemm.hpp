@@ -3,9 +3,10 @@
 //   C[:, cidx[n]] (+)= sum_b A_b X[:, gidx[b][n]]
 //
 // A_b are (3Nq x 3Nq) operators stored k-major (At[k][m], Kpad x Mpad, zero
-// padded); X and C hold one density vector of length K per node.  Used for
-// M2L (189 translation operators per child class), M2M (8 child
-// operators), L2L and the two-factor check-to-equivalent solves.
+// padded); X and C hold one density vector of length K per node.
+// k_gemm_gather serves the dense M2L (189 translation operators per child
+// class) and the truncated forms; k_gemm_direct below the FP64 form's M2M (8
+// child operators), L2L and two-factor check-to-equivalent solves.
 //
 // Work decomposition: the flattened grid is walked job-fastest, so with the
 // hardware's round-robin dispatch of workgroups to the 8 XCDs the 8 M2L jobs
@@ -30,6 +31,9 @@ namespace nnk {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2v __attribute__((ext_vector_type(2)));
+// pointers read out of a job: global, not flat, loads
+typedef const double __attribute__((address_space(1))) *gcd;
+typedef const int32_t __attribute__((address_space(1))) *gci;
 
 // TAG only separates launches by role in profiles (1 = M2L translations).
 template <int BM, int BN, int BK, int TAG>
@@ -211,6 +215,187 @@ __global__ __launch_bounds__(256, 2) void k_gemm_gather(int M, int K, int Mpad, 
         }
       }
     }
+}
+
+// The same product for the FP64 form's M2M, L2L and check-to-equivalent
+// solves (jobs of at most 16 operator blocks), without LDS staging.  An FP64
+// MFMA holds the matrix core for 64 cycles, so a wavefront of TM x TN tiles of
+// 16 x 16 needs one fragment load per TM TN / (TM + TN) products: little
+// enough to load the fragments straight from memory, one 16-deep K chunk
+// ahead, with no barrier to wait at.  Within a chunk lane group lk = lane / 16
+// takes k = 4 lk .. 4 lk + 3 (32 contiguous bytes of a column); product s
+// takes the s-th of each group.  KS = 1: the four wavefronts of a workgroup
+// take the same rows of neighbouring column tiles (three of them read A from
+// L1).  KS > 1: KS wavefronts share one tile and split its (block, chunk)
+// sequence, their sums added in wavefront order through LDS: for launches of
+// few tiles, which are bound by the latency of the chunks in a row.
+// The row blocks of a column tile are 8 workgroups apart, on one XCD, so its
+// columns come from one L2.
+template <int TM, int TN, int KS>
+__global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
+    int M, int K, int Mpad, int Kpad, const double *__restrict__ X, int ldx, double *__restrict__ C, int ldc, int beta,
+    const GemmJob *__restrict__ jobs, int njobs, int nrb, int nct) {
+  constexpr int WAVES = KS > 4 ? KS : 4, CW = WAVES / KS;   // wavefronts, column tiles of a workgroup
+  __shared__ double red[KS > 1 ? (WAVES - CW) * TM * TN * 256 : 1];
+  __shared__ int act[16], nact_s;
+  const int q = blockIdx.x >> 3, u = (q / nrb) * 8 + (blockIdx.x & 7), rb = q % nrb;
+  if (u >= njobs * nct) return;
+  const GemmJob J = jobs[u % njobs];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
+  const int ks = wave / CW, wc = wave % CW;
+  const int wg0 = (u / njobs) * CW * TN * 16;    // first column of the workgroup
+  if (wg0 >= J.N) return;
+  // operator blocks with a source in the workgroup's columns, in order
+  if (wave == 0) {
+    int n = 0;
+    for (int b = 0; b < J.nb; b++) {
+      bool any = true;
+      if (J.gidx) {
+        any = false;
+        for (int c = lane; c < CW * TN * 16; c += 64) any |= wg0 + c < J.N && ((gci)J.gidx)[(size_t)b * J.N + wg0 + c] >= 0;
+        any = __ballot(any) != 0;
+      }
+      if (any) {
+        if (lane == 0) act[n] = b;
+        n++;
+      }
+    }
+    if (lane == 0) nact_s = n;
+  }
+  __syncthreads();
+  const int KC = Kpad / 16, total = nact_s * KC;
+  const int col0 = wg0 + wc * TN * 16;
+  const int rt0 = rb * TM;                       // first row tile; past the last: its rows are not stored
+  d4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = d4{0, 0, 0, 0};
+  int cur = -1;
+  gcd Ab = nullptr;
+  gcd xc[TN];
+  bool on[TN];
+  // Branch-free: a lane without a source loads node 0's values and a lane past
+  // the columns' end the last four; lo is the first product that counts.
+  auto fetch = [&](int c, double (&a)[4][TM], double (&x)[TN][4], int (&lo)[TN]) {
+    const int qb = c / KC, k0 = (c - qb * KC) * 16 + 4 * lk;
+    if (qb != cur) {
+      cur = qb;
+      const int b = act[qb];
+      Ab = (gcd)((const uint64_t __attribute__((address_space(1))) *)J.A)[b];
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const int col = col0 + j * 16 + lr;
+        int g = -1;
+        if (col < J.N) g = J.gidx ? ((gci)J.gidx)[(size_t)b * J.N + col] : col;
+        on[j] = g >= 0;
+        xc[j] = (gcd)X + (size_t)(g < 0 ? 0 : g) * ldx;
+      }
+    }
+    const int kb = max(min(k0, K - 4), 0);
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int i = 0; i < TM; i++) a[s][i] = Ab[(size_t)(kb + s) * Mpad + min((rt0 + i) * 16, Mpad - 16) + lr];
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+#pragma unroll
+      for (int s = 0; s < 4; s++) x[j][s] = xc[j][kb + s];
+      lo[j] = on[j] ? k0 - kb : 4;
+    }
+  };
+  auto product = [&](const double (&a)[4][TM], const double (&x)[TN][4], const int (&lo)[TN]) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      double v[TN];
+#pragma unroll
+      for (int j = 0; j < TN; j++) v[j] = s >= lo[j] && s < K ? x[j][s] : 0.0;
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][i], v[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  double a0[4][TM], a1[4][TM], x0[TN][4], x1[TN][4];
+  int l0[TN], l1[TN];
+  // the wavefront's chunks: a contiguous share of the sequence, in pairs; a
+  // chunk past the end counts for nothing
+  const int c0 = (int)((int64_t)total * ks / KS), c1 = (int)((int64_t)total * (ks + 1) / KS);
+  if (c0 < c1) {
+    fetch(c0, a0, x0, l0);
+#pragma unroll 1
+    for (int c = c0; c < c1; c += 2) {
+      fetch(min(c + 1, c1 - 1), a1, x1, l1);
+      if (c + 1 == c1)
+#pragma unroll
+        for (int j = 0; j < TN; j++) l1[j] = 4;
+      __builtin_amdgcn_sched_barrier(0);   // the loads go out before the products, not among them
+      product(a0, x0, l0);
+      fetch(min(c + 2, c1 - 1), a0, x0, l0);
+      __builtin_amdgcn_sched_barrier(0);
+      product(a1, x1, l1);
+    }
+  }
+  if constexpr (KS > 1) {
+    auto slot = [&](int k, int e) { return ((((k - 1) * CW + wc) * TM * TN * 4) + e) * 64 + lane; };
+    if (ks > 0)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) red[slot(ks, (i * TN + j) * 4 + r)] = acc[i][j][r];
+    __syncthreads();
+    if (ks > 0) return;
+    for (int k = 1; k < KS; k++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][j][r] += red[slot(k, (i * TN + j) * 4 + r)];
+  }
+#pragma unroll
+  for (int j = 0; j < TN; j++) {
+    const int col = col0 + j * 16 + lr;
+    if (col >= J.N) continue;
+    double *p = C + (size_t)(J.cidx ? J.cidx[col] : col) * ldc;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int row = (rt0 + i) * 16 + lk + 4 * r;
+        if (row < M) p[row] = beta ? p[row] + acc[i][j][r] : acc[i][j][r];
+      }
+  }
+}
+
+// Launches the product by its number of workgroups: one wavefront per tile
+// (48 x 128 per workgroup) from two workgroups per CU, 48 x 32 shared by four
+// wavefronts from one per CU, else 32 x 16 shared by eight.  Both sides of the
+// lines at K = 456: 4,096 columns (320 workgroups of 48 x 128) take 0.16 ms
+// less over a matvec's up pass with the shared tiles; 512 columns 36 against
+// 23 us for an L2L.
+// FP64 matvecs before (160 x 32 tiles staged through LDS, M2M split over the
+// children where columns are few) and now, res 6: up pass 198 -> 76 us, solves
+// 155 -> 46 us, L2L 49 -> 23 us with 64 and 512 leaves; 2^20 points 1.42 ->
+// 1.11 ms, 0.91 -> 0.71 ms, 0.46 -> 0.40 ms.
+inline void launch_gemm_direct(int M, int K, int Mpad, int Kpad, const double *X, int ldx, double *C, int ldc,
+                               int beta, const GemmJob *jobs, int njobs, int maxN, hipStream_t s) {
+  auto wgs = [&](int rows, int cols) {
+    return (int64_t)njobs * ((M + rows - 1) / rows) * ((maxN + cols - 1) / cols);
+  };
+  auto go = [&](auto kern, int threads, int rows, int cols) {
+    const int nrb = (M + rows - 1) / rows, nct = (maxN + cols - 1) / cols;
+    const int64_t units = ((int64_t)njobs * nct + 7) / 8 * 8;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(units * nrb)), dim3(threads), 0, s, M, K, Mpad, Kpad, X, ldx, C, ldc,
+                       beta, jobs, njobs, nrb, nct);
+    NNK_HIP(hipGetLastError());
+  };
+  if (wgs(48, 128) >= 512) go(k_gemm_direct<3, 2, 1>, 256, 48, 128);
+  else if (wgs(48, 32) >= 256) go(k_gemm_direct<3, 2, 4>, 256, 48, 32);
+  else go(k_gemm_direct<2, 1, 8>, 512, 32, 16);
 }
 
 // C[slot[c]][row] = sum over splits of P[split][c][row], splits in order
