@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "nnk_fmm.hpp"
@@ -78,15 +79,19 @@ __global__ __launch_bounds__(256) void k_red_form(RedArgs a) {
 }
 
 // In-place LU with partial pivoting (first maximal |a_ik|), blocked
-// right-looking (the order of LAPACK's getrf), one launch pair per 32-column
-// panel for every leaf at once.  k_red_lu_panel (one workgroup per leaf)
-// factors the panel column by column (row interchanges applied to whole
-// rows) and solves the panel's rows of U right of it with its unit lower
-// triangle; k_red_lu_update gives every 64 x 64 tile of every leaf's
-// trailing matrix a workgroup of its own for the rank-32 update (staged
-// through LDS), so that large leaves use the whole GPU instead of one CU.
-constexpr int kLuThreads = 512, kLuNB = 32, kLuT = 64;
-__global__ __launch_bounds__(kLuThreads) void k_red_lu_panel(RedArgs a, int k0) {
+// right-looking (the order of LAPACK's getrf), three launches per 32-column
+// panel for every leaf at once: k_red_lu_panel (one workgroup per leaf)
+// factors the panel; k_red_lu_rows (a thread per column) applies its row
+// interchanges to the other columns and solves the panel's rows of U right of
+// it with its unit lower triangle; k_red_lu_update subtracts the rank-32
+// product from every 64 x 64 tile of the trailing matrix.
+// While more than kLuRows rows are left, k_red_lu_panel_mem does the work of
+// the first two in memory.
+// Measured for ten squirmers in a box (blocks up to 832 rows, 26 panels), all
+// panels: panel and rows 6.5 -> 2.0 ms (43 to 80 and 15 us each), updates
+// 1.0 -> 0.43 ms.
+constexpr int kLuThreads = 512, kLuNB = 32, kLuT = 64, kLuRows = 1024;
+__global__ __launch_bounds__(kLuThreads) void k_red_lu_panel_mem(RedArgs a, int k0) {
   const int li = blockIdx.x;
   const int n = a.leaves[li];
   const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
@@ -118,7 +123,7 @@ __global__ __launch_bounds__(kLuThreads) void k_red_lu_panel(RedArgs a, int k0) 
       }
       __syncthreads();
     }
-    const int p = si[0];
+    const int p = si[0] < n3 ? si[0] : k;   // a column of NaN has no maximum
     if (tid == 0) piv[k] = p;
     if (p != k)
       for (int jj = tid; jj < n3; jj += kLuThreads) {
@@ -154,9 +159,156 @@ __global__ __launch_bounds__(kLuThreads) void k_red_lu_panel(RedArgs a, int k0) 
   }
 }
 
+// the largest value of a wavefront, in every lane
+__device__ __forceinline__ double wave_max(double v) {
+  auto step = [&](auto ctrl) {
+    constexpr int c = decltype(ctrl)::value;   // row_shr 1, 2, 4, 8, row_bcast 15, 31: lane 63 ends with all
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int l2 = __builtin_amdgcn_update_dpp(lo, lo, c, 0xf, 0xf, false);
+    const int h2 = __builtin_amdgcn_update_dpp(hi, hi, c, 0xf, 0xf, false);
+    v = fmax(v, __hiloint2double(h2, l2));
+  };
+  step(std::integral_constant<int, 0x111>{});
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});
+  step(std::integral_constant<int, 0x143>{});
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// The panel in registers, a thread per row (at most T rows are left): per
+// column one reduction for the pivot and one exchange of two rows through LDS,
+// the eliminations from registers.
+template <int T>
+__global__ __launch_bounds__(T) void k_red_lu_panel(RedArgs a, int k0) {
+  constexpr int NW = T / 64, NB = kLuNB;
+  const int li = blockIdx.x;
+  const int n = a.leaves[li];
+  const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
+  if (k0 >= n3) return;  // the whole workgroup
+  int32_t *piv = a.piv + a.poff[li];
+  __shared__ double bv[2][NW], rowp[NB], rowk[NB];
+  __shared__ int bi[2][NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = n3 - k0, w = min(NB, m);
+  const bool own = tid < m;
+  double *row = a.blk + a.off[li] + (size_t)(k0 + min(tid, m - 1)) * n3 + k0;
+  double x[NB];
+#pragma unroll
+  for (int c = 0; c < NB; c++) x[c] = c < w ? row[c] : 0.0;
+#pragma unroll
+  for (int k = 0; k < NB; k++) {
+    if (k < w) {   // uniform
+      double v = own && tid >= k ? fabs(x[k]) : -1.0;
+      if (!(v >= 0.0)) v = -1.0;   // NaN is no pivot
+      const double wm = wave_max(v);
+      const int first = __ffsll(__ballot(v == wm)) - 1;
+      if (lane == 0) {
+        bv[k & 1][wave] = wm;
+        bi[k & 1][wave] = wave * 64 + first;
+      }
+      __syncthreads();
+      const double g = bv[k & 1][min(lane, NW - 1)];   // the same row order in every wavefront: the first maximum
+      const double gm = wave_max(g);
+      const int p = gm < 0.0 ? k : bi[k & 1][__ffsll(__ballot(g == gm)) - 1];
+      if (tid == p)
+#pragma unroll
+        for (int c = 0; c < NB; c++) rowp[c] = x[c];
+      if (tid == k)
+#pragma unroll
+        for (int c = 0; c < NB; c++) rowk[c] = x[c];
+      if (tid == 0) piv[k0 + k] = k0 + p;
+      __syncthreads();
+      if (tid == p || tid == k) {
+#pragma unroll
+        for (int c = 0; c < NB; c++) x[c] = tid == k ? rowp[c] : rowk[c];
+      }
+      if (tid > k) {
+        const double d = rowp[k];
+        if (d != 0.0) x[k] /= d;
+#pragma unroll
+        for (int c = k + 1; c < NB; c++) x[c] -= x[k] * rowp[c];
+      }
+    }
+  }
+  if (own)
+#pragma unroll
+    for (int c = 0; c < NB; c++)
+      if (c < w) row[c] = x[c];
+}
+
+// The panel's row interchanges in the columns outside it, as one permutation
+// of its rows and the (at most 32) rows they were exchanged with, and U12 =
+// L11^-1 A12 right of it: a thread per column, its rows in registers.
+__global__ __launch_bounds__(256) void k_red_lu_rows(RedArgs a, int k0) {
+  constexpr int NB = kLuNB;
+  const int li = blockIdx.x;
+  const int n = a.leaves[li];
+  const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
+  if (k0 >= n3 || (int)blockIdx.y * 256 >= n3) return;  // the whole workgroup
+  const int w = min(NB, n3 - k0), tid = threadIdx.x;
+  double *A = a.blk + a.off[li] + (size_t)k0 * n3;      // row 0: the panel's first
+  __shared__ double L[NB][NB + 1];
+  __shared__ int pv[NB], slot[NB], cur[2 * NB];
+  if (tid < NB) pv[tid] = tid < w ? a.piv[a.poff[li] + k0 + tid] - k0 : tid;
+  for (int idx = tid; idx < NB * NB; idx += 256) {
+    const int r = idx / NB, c = idx % NB;
+    L[r][c] = r < w && c < w ? A[(size_t)r * n3 + k0 + c] : 0.0;
+  }
+  __syncthreads();
+  // slots: the panel's rows, then, for exchange i with a row below, NB + (the
+  // first exchange with that row); cur[slot] is the row whose entries the
+  // slot's row ends with
+  if (tid < NB) {
+    const int p = pv[tid];
+    int sl = p;
+    if (p >= NB) {
+      int f = 0;
+      while (pv[f] != p) f++;
+      sl = NB + f;
+    }
+    slot[tid] = sl;
+    cur[tid] = tid;
+    cur[NB + tid] = p;
+  }
+  __syncthreads();
+  if (tid == 0)
+    for (int i = 0; i < w; i++) {
+      const int t = cur[i], s = slot[i];
+      cur[i] = cur[s];
+      cur[s] = t;
+    }
+  __syncthreads();
+  const int j = blockIdx.y * 256 + tid;
+  if (j >= n3 || (j >= k0 && j < k0 + w)) return;
+  double x[NB], y[NB];
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    x[i] = i < w ? A[(size_t)cur[i] * n3 + j] : 0.0;
+    y[i] = slot[i] == NB + i ? A[(size_t)cur[NB + i] * n3 + j] : 0.0;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; i++)
+    if (slot[i] == NB + i) A[(size_t)pv[i] * n3 + j] = y[i];
+  if (j >= k0 + w) {
+#pragma unroll
+    for (int k = 0; k < NB; k++)
+#pragma unroll
+      for (int i = k + 1; i < NB; i++) x[i] -= L[i][k] * x[k];
+  }
+#pragma unroll
+  for (int i = 0; i < NB; i++)
+    if (i < w) A[(size_t)i * n3 + j] = x[i];
+}
+
+typedef double rd4 __attribute__((ext_vector_type(4)));
+
 // A22 -= L21 U12 after the panel at k0: workgroup (leaf, t) updates tile t
-// of the leaf's trailing matrix (row-major over its ceil(m / 64)^2 tiles)
-__global__ __launch_bounds__(kLuThreads) void k_red_lu_update(RedArgs a, int k0) {
+// of the leaf's trailing matrix (row-major over its ceil(m / 64)^2 tiles), a
+// wavefront 32 x 32 of it on the FP64 matrix cores, operands from memory.
+__global__ __launch_bounds__(256, 2) void k_red_lu_update(RedArgs a, int k0) {
   const int li = blockIdx.x;
   const int n = a.leaves[li];
   const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
@@ -166,48 +318,45 @@ __global__ __launch_bounds__(kLuThreads) void k_red_lu_update(RedArgs a, int k0)
   const int t = blockIdx.y;
   if (t >= nt * nt) return;
   double *A = a.blk + a.off[li];
-  __shared__ double Ls[kLuT][kLuNB + 1];
-  __shared__ double Us[kLuNB][kLuT + 1];
-  const int tid = threadIdx.x;
-  const int r0 = k1 + (t / nt) * kLuT, c0 = k1 + (t % nt) * kLuT;
-  for (int idx = tid; idx < kLuT * kLuNB; idx += kLuThreads) {
-    const int r = idx / kLuNB, kk = idx % kLuNB;
-    Ls[r][kk] = r0 + r < n3 ? A[(size_t)(r0 + r) * n3 + k0 + kk] : 0.0;
-    const int kk2 = idx / kLuT, c = idx % kLuT;
-    Us[kk2][c] = c0 + c < n3 ? A[(size_t)(k0 + kk2) * n3 + c0 + c] : 0.0;
-  }
-  __syncthreads();
-  const int r = tid >> 3, cb = (tid & 7) * 8;
-  if (r0 + r < n3) {
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 4
-    for (int kk = 0; kk < kLuNB; kk++) {
-      const double l = Ls[r][kk];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int r0 = k1 + (t / nt) * kLuT + (wave >> 1) * 32, c0 = k1 + (t % nt) * kLuT + (wave & 1) * 32;
+  if (r0 >= n3 || c0 >= n3) return;   // (no barrier below)
+  rd4 acc[2][2];
 #pragma unroll
-      for (int c = 0; c < 8; c++) acc[c] += l * Us[kk][cb + c];
-    }
+  for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int c = 0; c < 8; c++)
-      if (c0 + cb + c < n3) A[(size_t)(r0 + r) * n3 + c0 + cb + c] -= acc[c];
+    for (int c = 0; c < 2; c++) acc[i][c] = rd4{0, 0, 0, 0};
+  // rows and columns past n3 repeat the last one and are not stored
+  const double *Lp[2] = {A + (size_t)min(r0 + lr, n3 - 1) * n3 + k0, A + (size_t)min(r0 + 16 + lr, n3 - 1) * n3 + k0};
+  const double *Up[2] = {A + (size_t)k0 * n3 + min(c0 + lr, n3 - 1), A + (size_t)k0 * n3 + min(c0 + 16 + lr, n3 - 1)};
+#pragma unroll
+  for (int h = 0; h < kLuNB; h += 16) {
+    double f[2][4], u[2][4];
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        f[i][s] = Lp[i][h + 4 * lk + s];
+        u[i][s] = Up[i][(size_t)(h + 4 * lk + s) * n3];
+      }
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+          acc[i][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[i][s], u[c][s], acc[i][c], 0, 0, 0);
   }
-}
-
-// the factors of each leaf to column-major order (in place), so that the
-// substitutions read whole columns contiguously
-__global__ __launch_bounds__(256) void k_red_transpose(RedArgs a) {
-  const int li = blockIdx.x;
-  const int n = a.leaves[li];
-  const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
-  double *A = a.blk + a.off[li];
-  const int64_t tot = (int64_t)n3 * n3;
-  for (int64_t idx = threadIdx.x; idx < tot; idx += 256) {
-    const int i = (int)(idx / n3), j = (int)(idx % n3);
-    if (i < j) {
-      const double t = A[(size_t)i * n3 + j];
-      A[(size_t)i * n3 + j] = A[(size_t)j * n3 + i];
-      A[(size_t)j * n3 + i] = t;
-    }
-  }
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int r = r0 + 16 * i + lk + 4 * s, q = c0 + 16 * c + lr;
+        if (r < n3 && q < n3) A[(size_t)r * n3 + q] -= acc[i][c][s];
+      }
 }
 
 // the row interchanges of each leaf's LU, applied in order to the identity:
@@ -228,124 +377,213 @@ __global__ void k_red_perm(RedArgs a, int nleaves) {
   }
 }
 
-// The inverse of each leaf block from its LU factors (set-up only), in the
-// row-major working block W (W[i n3 + j]).  A workgroup owns 64 consecutive
-// columns j of A^-1 = U^-1 L^-1 P (lane = column) and walks the rows in
-// blocks of kRedInvB; each of its kRedInvWaves wavefronts keeps the
-// column's entries of a quarter of the current row block in registers and
-// subtracts the rows solved before (each kRedInvB x kRedInvB factor tile
-// staged in LDS and read as broadcasts; the solved entries read from W,
-// coalesced across the lanes).  The first wavefront then solves the
-// diagonal tile in LDS, and every wavefront stores its rows.  Forward with
-// the unit lower triangle (row blocks ascending), then back with the upper
-// one (descending).  Each solved entry is read once per row block and
-// wavefront instead of once per row.
-constexpr int kRedInvCols = 64, kRedInvB = 32, kRedInvWaves = 4;
-__global__ __launch_bounds__(kRedInvCols * kRedInvWaves) void k_red_inv(RedArgs a, double *__restrict__ W) {
-  constexpr int B = kRedInvB, NT = kRedInvCols * kRedInvWaves, RW = B / kRedInvWaves;
-  __shared__ double F[B][B + 1];           // F[kk][r]: factor entry (row i0 + r, column k0 + kk)
-  __shared__ double Xs[B][kRedInvCols];    // the row block of the 64 columns (diagonal solve)
+// The inverses of the 32 x 32 diagonal tiles of each leaf's factors (unit
+// lower and upper triangle, row-major, padded with the identity), D[2 I] and
+// D[2 I + 1] of block row I: one wavefront per tile pair, a lane per column.
+constexpr int kInvB = 32;
+__global__ __launch_bounds__(64) void k_red_diag(RedArgs a, const int64_t *__restrict__ doff, double *__restrict__ D) {
+  constexpr int B = kInvB;
+  __shared__ double T[B][B + 1];
   const int li = blockIdx.x;
   const int n = a.leaves[li];
   const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
-  if ((int)blockIdx.y * kRedInvCols >= n3) return;  // the whole workgroup
-  const int tid = threadIdx.x, lane = tid % kRedInvCols, r0 = (tid / kRedInvCols) * RW;
-  const int j = blockIdx.y * kRedInvCols + lane;
-  const bool col = j < n3;
-  const double *A = a.blk + a.off[li];  // column-major factors: A[k n3 + i] = LU[i][k]
+  const int i0 = blockIdx.y * B;
+  if (i0 >= n3) return;
+  const double *A = a.blk + a.off[li];
+  const int lane = threadIdx.x, c = lane & 31;
+  for (int r = lane >> 5; r < B; r += 2)
+    T[r][c] = i0 + r < n3 && i0 + c < n3 ? A[(size_t)(i0 + r) * n3 + i0 + c] : (r == c ? 1.0 : 0.0);
+  __syncthreads();
+  double x[B];
+  double *O = D + doff[li] + (size_t)(2 * blockIdx.y + (lane >> 5)) * B * B + c;
+  if (lane < 32) {
+#pragma unroll
+    for (int r = 0; r < B; r++) {
+      double t = r == c ? 1.0 : 0.0;
+#pragma unroll
+      for (int q = 0; q < r; q++) t -= T[r][q] * x[q];
+      x[r] = t;
+    }
+  } else {
+#pragma unroll
+    for (int r = B - 1; r >= 0; r--) {
+      double t = r == c ? 1.0 : 0.0;
+#pragma unroll
+      for (int q = r + 1; q < B; q++) t -= T[r][q] * x[q];
+      x[r] = t / T[r][r];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < B; r++) O[(size_t)r * B] = x[r];
+}
+
+// The inverse of each leaf block from its LU factors (set-up only), column-
+// major in W (W[j n3 + i] = (A^-1)_ij = U^-1 L^-1 P).  A wavefront owns 16
+// columns and walks the rows in blocks of 32, forward with the unit lower
+// triangle, then back with the upper one: the solved blocks times the factor
+// tiles on the FP64 matrix cores (operands straight from memory, one tile
+// ahead), then the diagonal tile's inverse times the block, whose accumulator
+// registers are the B operand as they are (register r holds row lk + 4 r).
+// No barrier: the wavefronts are independent, four neighbours share a
+// workgroup for the factors' sake.  What bounds it is the chain of (n3 / 32)^2
+// tiles of 16 MFMAs per wavefront.
+// Measured for ten squirmers in a box (blocks up to 832 rows): 5.5 ms with
+// scalar sums and two transposes of 0.86 ms, now 2.2 ms.
+__global__ __launch_bounds__(256, 2) void k_red_inv(RedArgs a, const int64_t *__restrict__ doff,
+                                                    const double *__restrict__ D, double *W) {
+  constexpr int B = kInvB;
+  const int li = blockIdx.x;
+  const int n = a.leaves[li];
+  const int n3 = 3 * (a.tgt_ptr[n + 1] - a.tgt_ptr[n]);
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int j0 = (blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * 16;
+  if (j0 >= n3) return;   // (no barrier below)
+  const int j = j0 + lr, jc = min(j, n3 - 1);
+  const double *A = a.blk + a.off[li];   // row-major factors
+  const double *Dl = D + doff[li];
   const int32_t *perm = a.perm + a.poff[li];
-  double *X = W + a.off[li];
+  double *X = W + a.off[li] + (size_t)jc * n3;   // a lane past the last column computes a copy and stores nothing
   const int nb = (n3 + B - 1) / B;
-  // (the barriers also order the global stores of W before later reads by
-  // the other wavefronts)
-  auto stage = [&](int i0, int k0) {
-    __syncthreads();  // the previous tile has been read
-    for (int idx = tid; idx < B * B; idx += NT) {
-      const int kk = idx / B, r = idx % B, k = k0 + kk, i = i0 + r;
-      F[kk][r] = (k < n3 && i < n3) ? A[(size_t)k * n3 + i] : 0.0;
-    }
-    __syncthreads();
-  };
-  // this wavefront's rows r0 .. r0+RW-1 of the block, minus the already
-  // solved rows k0 .. k0+B-1 of the column times the tile
-  double acc[RW];
-  auto update = [&](int k0) {
-    for (int kk = 0; kk < B; kk++) {
-      const double xk = (col && k0 + kk < n3) ? X[(size_t)(k0 + kk) * n3 + j] : 0.0;
+  struct Tile { double f[2][2][4], x[2][4]; };
+  // factor tile (rows i0 .., columns of block K) and the solved block K;
+  // entries past n3 only in the last block
+  auto fetch = [&](int i0, int K, Tile &t) {
+    const int k0 = K * B;
+    if (k0 + B <= n3) {
 #pragma unroll
-      for (int r = 0; r < RW; r++) acc[r] -= F[kk][r0 + r] * xk;
+      for (int h = 0; h < 2; h++) {
+        const int k = k0 + 16 * h + 4 * lk;
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+          for (int s = 0; s < 4; s++) t.f[r][h][s] = A[(size_t)min(i0 + 16 * r + lr, n3 - 1) * n3 + k + s];
+#pragma unroll
+        for (int s = 0; s < 4; s++) t.x[h][s] = X[k + s];
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          const int k = k0 + 16 * h + 4 * lk + s, kc = min(k, n3 - 1);
+#pragma unroll
+          for (int r = 0; r < 2; r++) t.f[r][h][s] = A[(size_t)min(i0 + 16 * r + lr, n3 - 1) * n3 + kc];
+          const double v = X[kc];
+          t.x[h][s] = k < n3 ? v : 0.0;
+        }
     }
   };
-  // hand the rows to the diagonal solve of the first wavefront (solve),
-  // then store every wavefront's rows
-  auto diag = [&](int i0, auto solve) {
+  rd4 acc[2];
+  auto sub = [&](const Tile &t) {
 #pragma unroll
-    for (int r = 0; r < RW; r++) Xs[r0 + r][lane] = acc[r];
-    __syncthreads();
-    if (tid < kRedInvCols) solve();
-    __syncthreads();
-    if (col)
-      for (int r = r0; r < r0 + RW && i0 + r < n3; r++) X[(size_t)(i0 + r) * n3 + j] = Xs[r][lane];
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+          acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(t.f[r][h][s], -t.x[h][s], acc[r], 0, 0, 0);
+  };
+  // acc -= sum over blocks K in [ka, kb) of tile (i0, K) times block K
+  auto sweep = [&](int i0, int ka, int kb) {
+    if (ka >= kb) return;
+    Tile t0, t1;
+    fetch(i0, ka, t0);
+#pragma unroll 1
+    for (int K = ka; K < kb; K += 2) {
+      fetch(i0, min(K + 1, kb - 1), t1);
+      sub(t0);
+      if (K + 1 == kb) break;
+      fetch(i0, min(K + 2, kb - 1), t0);
+      sub(t1);
+    }
+  };
+  // block row I = D^-1 acc, stored to X
+  auto solve = [&](int I, int upper) {
+    const int i0 = I * B;
+    const double *T = Dl + (size_t)(2 * I + upper) * B * B;
+    rd4 o[2] = {rd4{0, 0, 0, 0}, rd4{0, 0, 0, 0}};
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int k = 16 * h + 4 * s + lk;
+        const double v = i0 + k < n3 ? acc[h][s] : 0.0;
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+          o[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(T[(16 * r + lr) * B + k], v, o[r], 0, 0, 0);
+      }
+    if (j < n3)
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+          if (i0 + 16 * r + lk + 4 * s < n3) X[i0 + 16 * r + lk + 4 * s] = o[r][s];
+    // the next blocks read these rows through other lanes of this wavefront
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   };
   for (int I = 0; I < nb; I++) {  // L y = P e_j
-    const int i0 = I * B;
 #pragma unroll
-    for (int r = 0; r < RW; r++) acc[r] = (col && i0 + r0 + r < n3 && perm[i0 + r0 + r] == j) ? 1.0 : 0.0;
-    for (int K = 0; K < I; K++) {
-      stage(i0, K * B);
-      update(K * B);
-    }
-    stage(i0, i0);
-    diag(i0, [&]() {
-      for (int r = 1; r < B; r++) {  // unit lower diagonal tile
-        double t = Xs[r][lane];
-        for (int q = 0; q < r; q++) t -= F[q][r] * Xs[q][lane];
-        Xs[r][lane] = t;
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int i = I * B + 16 * r + lk + 4 * s;
+        acc[r][s] = i < n3 && perm[min(i, n3 - 1)] == j ? 1.0 : 0.0;
       }
-    });
+    sweep(I * B, 0, I);
+    solve(I, 0);
   }
   for (int I = nb - 1; I >= 0; I--) {  // U x = y
-    const int i0 = I * B;
 #pragma unroll
-    for (int r = 0; r < RW; r++) acc[r] = (col && i0 + r0 + r < n3) ? X[(size_t)(i0 + r0 + r) * n3 + j] : 0.0;
-    for (int K = I + 1; K < nb; K++) {
-      stage(i0, K * B);
-      update(K * B);
-    }
-    stage(i0, i0);
-    diag(i0, [&]() {
-      for (int r = B - 1; r >= 0; r--) {  // upper diagonal tile
-        double t = Xs[r][lane];
-        for (int q = r + 1; q < B; q++) t -= F[q][r] * Xs[q][lane];
-        Xs[r][lane] = i0 + r < n3 ? t / F[r][r] : 0.0;
-      }
-    });
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) acc[r][s] = X[min(I * B + 16 * r + lk + 4 * s, n3 - 1)];
+    sweep(I * B, I + 1, nb);
+    solve(I, 1);
   }
 }
 
 // x = A^-1 v for each leaf with the column-major inverse
-// (Inv[j n3 + i] = (A^-1)_ij): workgroup (leaf, row group) holds the leaf's
-// right-hand side in LDS and gives each of its rows one thread; the columns
-// are read in order (coalesced across the rows), the sum in column order.
-// Large blocks spread over several workgroups instead of one CU.
-constexpr int kRedApplyThreads = 256;
-__global__ __launch_bounds__(kRedApplyThreads) void k_red_apply(RedArgs a, const double *__restrict__ v,
-                                                                double *__restrict__ x) {
+// (Inv[j n3 + i] = (A^-1)_ij): a workgroup takes 64 rows of a leaf (lane =
+// row, so a column's rows are read coalesced), its wavefronts an eighth of the
+// columns each, the sums added in wavefront order.  One pass over the
+// inverses, bound by their bytes; a thread walking a whole row alone had one
+// load in flight per 500 ns.
+// Measured for ten squirmers in a box (blocks up to 832 rows): 71 -> 20 us.
+constexpr int kRedApplyWaves = 8;
+__global__ __launch_bounds__(64 * kRedApplyWaves) void k_red_apply(RedArgs a, const double *__restrict__ v,
+                                                                   double *__restrict__ x) {
   extern __shared__ double b[];
+  __shared__ double part[kRedApplyWaves][64];
   const int li = blockIdx.x;
   const int n = a.leaves[li];
   const int tb = a.tgt_ptr[n], nt = a.tgt_ptr[n + 1] - tb;
   const int n3 = 3 * nt;
-  const int i0 = blockIdx.y * kRedApplyThreads;
+  const int i0 = blockIdx.y * 64;
   if (i0 >= n3) return;  // the whole workgroup
   const double *Inv = a.blk + a.off[li];
-  for (int i = threadIdx.x; i < n3; i += kRedApplyThreads) b[i] = v[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3];
+  for (int i = threadIdx.x; i < n3; i += 64 * kRedApplyWaves)
+    b[i] = v[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3];
   __syncthreads();
-  const int i = i0 + threadIdx.x;
-  if (i < n3) {
-    double acc = 0.0;
-    for (int jj = 0; jj < n3; jj++) acc += Inv[(size_t)jj * n3 + i] * b[jj];
-    x[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3] = acc;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = i0 + lane;
+  const int j1 = n3 * (w + 1) / kRedApplyWaves;
+  const double *col = Inv + min(i, n3 - 1);
+  double acc[4] = {0, 0, 0, 0};
+  int j = n3 * w / kRedApplyWaves;
+  for (; j + 8 <= j1; j += 8) {
+    double t[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) t[k] = col[(size_t)(j + k) * n3];
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc[k & 3] += t[k] * b[j + k];
+  }
+  for (; j < j1; j++) acc[0] += col[(size_t)j * n3] * b[j];
+  part[w][lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  __syncthreads();
+  if (w == 0 && i < n3) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < kRedApplyWaves; k++) t += part[k][lane];
+    x[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3] = t;
   }
 }
 
@@ -386,27 +624,37 @@ void Fmm::reduced_factor() {
     hipLaunchKernelGGL(k_red_form, dim3(n_tleaves_), dim3(256), 0, 0, a);
     NNK_HIP(hipGetLastError());
     for (int k0 = 0; k0 < red_maxn_; k0 += kLuNB) {
-      hipLaunchKernelGGL(k_red_lu_panel, dim3(n_tleaves_), dim3(kLuThreads), 0, 0, a, k0);
+      const int left = red_maxn_ - k0;
+      if (left > kLuRows) {
+        hipLaunchKernelGGL(k_red_lu_panel_mem, dim3(n_tleaves_), dim3(kLuThreads), 0, 0, a, k0);
+      } else {
+        if (left > 512) hipLaunchKernelGGL(k_red_lu_panel<1024>, dim3(n_tleaves_), dim3(1024), 0, 0, a, k0);
+        else if (left > 256) hipLaunchKernelGGL(k_red_lu_panel<512>, dim3(n_tleaves_), dim3(512), 0, 0, a, k0);
+        else hipLaunchKernelGGL(k_red_lu_panel<256>, dim3(n_tleaves_), dim3(256), 0, 0, a, k0);
+        hipLaunchKernelGGL(k_red_lu_rows, dim3(n_tleaves_, (red_maxn_ + 255) / 256), dim3(256), 0, 0, a, k0);
+      }
       const int m = red_maxn_ - k0 - kLuNB;
       if (m > 0) {
         const int nt = (m + kLuT - 1) / kLuT;
-        hipLaunchKernelGGL(k_red_lu_update, dim3(n_tleaves_, nt * nt), dim3(kLuThreads), 0, 0, a, k0);
+        hipLaunchKernelGGL(k_red_lu_update, dim3(n_tleaves_, nt * nt), dim3(256), 0, 0, a, k0);
       }
     }
     NNK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_red_transpose, dim3(n_tleaves_), dim3(256), 0, 0, a);
     hipLaunchKernelGGL(k_red_perm, dim3((n_tleaves_ + 63) / 64), dim3(64), 0, 0, a, n_tleaves_);
     NNK_HIP(hipGetLastError());
     // the blocks' inverses replace their factors: each solve is then one
     // pass over them at HBM bandwidth instead of a chain of substitutions
-    DBuf W;
+    std::vector<int64_t> doff(n_tleaves_ + 1, 0);
+    for (int i = 0; i < n_tleaves_; i++)
+      doff[i + 1] = doff[i] + (poff[i + 1] - poff[i] + kInvB - 1) / kInvB * 2 * kInvB * kInvB;
+    DBuf W, D, ddoff;
+    ddoff.upload(doff);
+    D.alloc(sizeof(double) * std::max<int64_t>(doff.back(), 1));
     W.alloc(sizeof(double) * std::max<int64_t>(off.back(), 1));
-    hipLaunchKernelGGL(k_red_inv, dim3(n_tleaves_, (red_maxn_ + kRedInvCols - 1) / kRedInvCols),
-                       dim3(kRedInvCols * kRedInvWaves), 0, 0, a, W.as<double>());
-    NNK_HIP(hipGetLastError());
-    RedArgs w = a;
-    w.blk = W.as<double>();
-    hipLaunchKernelGGL(k_red_transpose, dim3(n_tleaves_), dim3(256), 0, 0, w);
+    hipLaunchKernelGGL(k_red_diag, dim3(n_tleaves_, (red_maxn_ + kInvB - 1) / kInvB), dim3(64), 0, 0, a,
+                       ddoff.as<int64_t>(), D.as<double>());
+    hipLaunchKernelGGL(k_red_inv, dim3(n_tleaves_, (red_maxn_ + 63) / 64), dim3(256), 0, 0, a, ddoff.as<int64_t>(),
+                       D.as<double>(), W.as<double>());
     NNK_HIP(hipGetLastError());
     NNK_HIP(hipDeviceSynchronize());
     red_blk_ = std::move(W);
@@ -444,8 +692,8 @@ void Fmm::reduced_solve(const double *d_v, double *d_f, hipStream_t s) {
   if (!red_ready_) reduced_factor();
   if (!n_tleaves_) return;
   RedArgs a = red_args();
-  hipLaunchKernelGGL(k_red_apply, dim3(n_tleaves_, (red_maxn_ + kRedApplyThreads - 1) / kRedApplyThreads),
-                     dim3(kRedApplyThreads), sizeof(double) * red_maxn_, s, a, d_v, d_f);
+  hipLaunchKernelGGL(k_red_apply, dim3(n_tleaves_, (red_maxn_ + 63) / 64), dim3(64 * kRedApplyWaves),
+                     sizeof(double) * red_maxn_, s, a, d_v, d_f);
   NNK_HIP(hipGetLastError());
 }
 
