@@ -408,7 +408,27 @@ struct LeafArgs {
   int far;          // 0: sources of the leaf itself only (reducedPass.m)
   int tc;           // targets per workgroup and pass (<= T); blockIdx.y picks the chunk
   double *out;      // ntgt x 3
+  // leaves with long source lists are shared by several workgroups (null:
+  // none): items[blockIdx.x] is (leaf, part, parts, first row of its sums)
+  const int4 *items;
+  double *part;     // sums of part p: rows first + p * targets ..
 };
+__device__ __forceinline__ int4 leaf_item(const LeafArgs &a) {
+  if (a.items) return a.items[blockIdx.x];
+  return int4{a.leaves[blockIdx.x], 0, 1, 0};
+}
+
+// velocities of the shared leaves (list[blockIdx.x]: part 0's item): the sums
+// of their parts, in order
+__global__ __launch_bounds__(256) void k_leaf_parts(LeafArgs a, const int4 *__restrict__ list) {
+  const int4 it = list[blockIdx.x];
+  const int tb = a.tgt_ptr[it.x], n3 = 3 * (a.tgt_ptr[it.x + 1] - tb);
+  for (int i = threadIdx.x; i < n3; i += 256) {
+    double v = 0.0;
+    for (int p = 0; p < it.z; p++) v += a.part[3 * (size_t)it.w + (size_t)p * n3 + i];
+    a.out[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3] = a.c * v;
+  }
+}
 
 // FP32-math forms: velocity at the targets of one leaf: L2T from its down density, P2P from
 // its U-list sources, M2T from its W-list up densities (Downleaf.m:37-40).
@@ -421,7 +441,8 @@ struct LeafArgs {
 // are staged leaf by leaf.
 template <int T>
 __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
-  const int n = a.leaves[blockIdx.x];
+  const int4 it = leaf_item(a);
+  const int n = it.x;
   // the surface sources (L2T, M2T) go through the offset stage
   // with the origin at the centre of the surface's node (this leaf for
   // L2T, the smaller W node for M2T); the U-list sources keep the FP64
@@ -498,9 +519,9 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
     };
     // the U-list sources as one list: entry g lies in leaf e with
     // upre[e] <= g < upre[e + 1] (binary search; empty leaves are skipped)
-    auto usources = [&]() {
+    auto usources = [&](int ga, int gb) {
       const int tot = upre[nu];
-      for (int g0 = 0; g0 < tot; g0 += T) {
+      for (int g0 = ga; g0 < gb; g0 += T) {
         const int cnt = min(T, tot - g0);
         if (tid < cnt) {
           const int g = g0 + tid;
@@ -520,11 +541,17 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
       }
     };
     if (a.far) {
-      surface(n, 1, a.downpot);
-      for (int64_t e = a.wptr[n]; e < a.wptr[n + 1]; e++) surface(a.widx[e], 0, a.uppot);
-      if (ucat) usources();
+      // the list in steps (a surface; T sources, or a leaf's, of the U list):
+      // a part takes whole steps, so each step's sums are those of an unshared leaf
+      const int nw = 1 + (int)(a.wptr[n + 1] - a.wptr[n]);
+      const int64_t steps = nw + (ucat ? (upre[nu] + T - 1) / T : nu);
+      const int lo = (int)(steps * it.y / it.z), hi = (int)(steps * (it.y + 1) / it.z);
+      if (lo == 0) surface(n, 1, a.downpot);
+      for (int e = max(lo, 1); e < min(hi, nw); e++) surface(a.widx[a.wptr[n] + e - 1], 0, a.uppot);
+      const int ua = max(lo - nw, 0), ub = hi - nw;
+      if (ucat) usources(ua * T, min(ub * T, upre[nu]));
       else
-        for (int64_t e = u0; e < u1; e++) sources(a.uidx[e]);
+        for (int e = ua; e < ub; e++) sources(a.uidx[u0 + e]);
     } else {
       sources(n);
     }
@@ -538,9 +565,11 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
         sz += red[3 * (s * ntc + tid) + 2];
       }
       const int o = a.tgt_out[tb + t0 + tid];
-      a.out[3 * (size_t)o] = a.c * sx;
-      a.out[3 * (size_t)o + 1] = a.c * sy;
-      a.out[3 * (size_t)o + 2] = a.c * sz;
+      double *u = it.z > 1 ? a.part + 3 * ((size_t)it.w + (size_t)it.y * nt + t0 + tid) : a.out + 3 * (size_t)o;
+      const double c = it.z > 1 ? 1.0 : a.c;
+      u[0] = c * sx;
+      u[1] = c * sy;
+      u[2] = c * sz;
     }
     __syncthreads();
   }
@@ -554,8 +583,8 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
 template <int NT>
 __device__ __forceinline__ void leaf_block64(const LeafArgs &a, const double *__restrict__ src_pos,
                                              const double *__restrict__ src_q, const double *__restrict__ tgt_pos,
-                                             int n, int t0, int ntc, int blk, int sp, int nsplit, int *pre,
-                                             SrcBatch buf, double *red) {
+                                             int n, int part, int parts, int t0, int ntc, int blk, int sp, int nsplit,
+                                             int *pre, SrcBatch buf, double *red) {
   double tx[NT], ty[NT], tz[NT], u[3 * NT];
 #pragma unroll
   for (int k = 0; k < NT; k++) {
@@ -578,7 +607,10 @@ __device__ __forceinline__ void leaf_block64(const LeafArgs &a, const double *__
       const int32_t *list = a.uidx + b0;
       if (b0 > u0) __syncthreads();
       source_prefix(list, nu, a.src_ptr, pre);
-      sum_sources<NT>(tx, ty, tz, a.e2, sp, nsplit, s0 + pre[nu], buf, [&](int g) {
+      const int64_t tot = s0 + pre[nu];
+      const int ga = (int)(tot * part / parts), gb = (int)(tot * (part + 1) / parts);
+      sum_sources<NT>(tx, ty, tz, a.e2, sp, nsplit, gb - ga, buf, [&](int i) {
+        const int g = ga + i;
         if (g >= s0) return point(source_index(list, nu, a.src_ptr, pre, g - s0));
         const int k = g / a.nq, p = g - k * a.nq;
         const int node = k ? a.widx[w0 + k - 1] : n;
@@ -606,7 +638,8 @@ __global__ __launch_bounds__(256) void k_leaf64(LeafArgs a, const double *__rest
   __shared__ int pre[kLeafMaxU + 1];
   __shared__ SrcBatch buf;
   __shared__ double red[4][24];
-  const int n = a.leaves[blockIdx.x], tid = threadIdx.x;
+  const int4 it = leaf_item(a);
+  const int n = it.x, tid = threadIdx.x;
   const int tb = a.tgt_ptr[n], nt = a.tgt_ptr[n + 1] - tb, t0 = 32 * (int)blockIdx.y;
   if (t0 >= nt) return;
   const int ntc = min(32, nt - t0);
@@ -614,7 +647,7 @@ __global__ __launch_bounds__(256) void k_leaf64(LeafArgs a, const double *__rest
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), blk = w % nblk, sp = w / nblk, nsplit = 4 / nblk;
 #define NNK_LEAF_CASE(NT)                                                                                       \
   case NT:                                                                                                      \
-    leaf_block64<NT>(a, src_pos, src_q, tgt_pos, n, tb + t0, ntc, blk, sp, nsplit, pre, buf, red[w]);           \
+    leaf_block64<NT>(a, src_pos, src_q, tgt_pos, n, it.y, it.z, tb + t0, ntc, blk, sp, nsplit, pre, buf, red[w]); \
     break
   switch (per) {
     NNK_LEAF_CASE(1);
@@ -632,7 +665,8 @@ __global__ __launch_bounds__(256) void k_leaf64(LeafArgs a, const double *__rest
     const int t = tid / 3, d = tid - 3 * t, b = t / per;
     double v = 0.0;
     for (int s = 0; s < nsplit; s++) v += red[s * nblk + b][3 * (t - b * per) + d];
-    a.out[3 * (size_t)a.tgt_out[tb + t0 + t] + d] = a.c * v;
+    if (it.z > 1) a.part[3 * ((size_t)it.w + (size_t)it.y * nt + t0 + t) + d] = v;
+    else a.out[3 * (size_t)a.tgt_out[tb + t0 + t] + d] = a.c * v;
   }
 }
 
@@ -1205,14 +1239,17 @@ Fmm::Fmm(std::shared_ptr<const Tree> t, double eps, double mu, int res, int shel
   // targets x (U-list sources + surface points of the leaf and its W list)),
   // so that the heaviest start first instead of finishing last on a few
   // CUs.  The results do not depend on the order.
+  std::vector<int64_t> leaf_src;
   {
     auto nsrc = [&](int n) -> int64_t { return src_ptr[n + 1] - src_ptr[n]; };
     std::vector<int64_t> wp(nc + 1, 0), wt(nc + 1, 0);
+    leaf_src.assign(nc + 1, 0);
     for (int n : pl) wp[n] = nsrc(n);
     for (int n : tl) {
       int64_t u = 0;
       for (int64_t e = T.lptr[0][n]; e < T.lptr[0][n + 1]; e++) u += nsrc(T.lidx[0][e]);
-      wt[n] = (int64_t)(tgt_ptr[n + 1] - tgt_ptr[n]) * (u + (int64_t)nq_ * (1 + T.lptr[2][n + 1] - T.lptr[2][n]));
+      leaf_src[n] = u + (int64_t)nq_ * (1 + T.lptr[2][n + 1] - T.lptr[2][n]);
+      wt[n] = (int64_t)(tgt_ptr[n + 1] - tgt_ptr[n]) * leaf_src[n];
     }
     order_by_work(pl, wp);
     order_by_work(tl, wt);
@@ -1228,6 +1265,7 @@ Fmm::Fmm(std::shared_ptr<const Tree> t, double eps, double mu, int res, int shel
   }
   pleaves_.upload(pl);
   tleaves_.upload(tl);
+  plan_leaf_parts(tl, leaf_src, tgt_ptr);
   chk_.alloc(sizeof(double) * (size_t)nc * K_);
   uppot_.alloc(sizeof(double) * (size_t)nc * K_);
   downpot_.alloc(sizeof(double) * (size_t)nc * K_);
@@ -1871,6 +1909,44 @@ void Fmm::launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const in
   NNK_HIP(hipGetLastError());
 }
 
+// Shares the leaves with long source lists among several workgroups.  A
+// large leaf next to a fine region has a U list of up to 10^5 sources and more,
+// which one workgroup walks long after the others are done.  Work is counted
+// in source visits of a workgroup (the FP64 kernel's takes 32 targets, the
+// FP32-math kernel's all); a part is an eighth of a CU's share of the whole, but
+// at least 2,048 visits (8 batches), and lists of up to two parts stay whole.
+// Leaf kernel before and now: 8 bodies over a wall 355 -> 89 us and 6 us for
+// the sums; 64 bodies 1.8-2.3 -> 1.2-1.3 ms; 20 bodies in mixed form 0.5-5.7
+// (one leaf of more than 512 U leaves) -> 0.33 ms; a clustered set of 10^5
+// points in mixed form 0.86 -> 0.39 ms.  Ordinary trees have no such leaf.
+void Fmm::plan_leaf_parts(const std::vector<int32_t> &leaves, const std::vector<int64_t> &nsrc,
+                          const std::vector<int32_t> &tgt_ptr) {
+  auto blocks = [&](int n) -> int64_t { return (tgt_ptr[n + 1] - tgt_ptr[n] + 31) / 32; };
+  int64_t total = 0;
+  for (int n : leaves) total += nsrc[n] * blocks(n);
+  const int64_t per = std::max<int64_t>(2048, total / (8 * (int64_t)ncu_));
+  std::vector<int4> items, rest, list;
+  int64_t rows = 0;
+  for (int n : leaves) {
+    const int64_t w = nsrc[n] * (fp32_math() ? blocks(n) : 1);
+    if (w <= 2 * per) {
+      rest.push_back(int4{n, 0, 1, 0});
+      continue;
+    }
+    const int parts = (int)std::min<int64_t>((w + per - 1) / per, 1024), nt = tgt_ptr[n + 1] - tgt_ptr[n];
+    list.push_back(int4{n, 0, parts, (int)rows});
+    for (int p = 0; p < parts; p++) items.push_back(int4{n, p, parts, (int)rows});
+    rows += (int64_t)parts * nt;
+  }
+  if (list.empty() || rows > (1 << 28)) return;
+  items.insert(items.end(), rest.begin(), rest.end());
+  n_leaf_items_ = (int)items.size();
+  n_leaf_shared_ = (int)list.size();
+  leaf_items_.upload(items);
+  leaf_shared_.upload(list);
+  leaf_part_.alloc(sizeof(double) * 3 * rows);
+}
+
 void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   if (!n_tleaves_) return;
   LeafArgs a{};
@@ -1892,6 +1968,12 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   a.c = 1.0 / (8.0 * kPi * mu_);
   a.far = far;
   a.out = d_u;
+  const bool shared = far && n_leaf_shared_;
+  const int nwg = shared ? n_leaf_items_ : n_tleaves_;
+  if (shared) {
+    a.items = leaf_items_.as<int4>();
+    a.part = leaf_part_.as<double>();
+  }
   const int T = far ? leaf_threads_ : 256;
   // Few target leaves (small trees, large leaves) would leave most CUs idle
   // with one workgroup per leaf: their targets are then split into chunks
@@ -1899,16 +1981,18 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   // sources T / tc ways), until there are about two workgroups per CU
   a.tc = T;
   while (a.tc > 32 && (int64_t)n_tleaves_ * ((max_leaf_tgt_ + a.tc - 1) / a.tc) < 2 * (int64_t)ncu_) a.tc /= 2;
-  const dim3 grid((unsigned)n_tleaves_, (unsigned)std::max(1, (max_leaf_tgt_ + a.tc - 1) / a.tc));
+  const dim3 grid((unsigned)nwg, (unsigned)std::max(1, (max_leaf_tgt_ + a.tc - 1) / a.tc));
   auto go = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, grid, dim3(threads), 0, s, a); };
   if (fp32_math()) {
     if (T == 128) go(k_leaf<128>, 128);
     else if (T == 512) go(k_leaf<512>, 512);
     else go(k_leaf<256>, 256);
   } else {
-    hipLaunchKernelGGL(k_leaf64, dim3((unsigned)n_tleaves_, (unsigned)std::max(1, (max_leaf_tgt_ + 31) / 32)), dim3(256),
-                       0, s, a, a.src_pos, a.src_q, a.tgt_pos);
+    hipLaunchKernelGGL(k_leaf64, dim3((unsigned)nwg, (unsigned)std::max(1, (max_leaf_tgt_ + 31) / 32)), dim3(256), 0, s,
+                       a, a.src_pos, a.src_q, a.tgt_pos);
   }
+  if (shared)
+    hipLaunchKernelGGL(k_leaf_parts, dim3((unsigned)n_leaf_shared_), dim3(256), 0, s, a, leaf_shared_.as<int4>());
   NNK_HIP(hipGetLastError());
 }
 

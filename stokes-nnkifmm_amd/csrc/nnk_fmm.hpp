@@ -368,6 +368,8 @@ class Fmm {
   // the fastest, re-timing the near-ties
   void autotune(hipStream_t s);
   void autotune_leaf(hipStream_t s);
+  void plan_leaf_parts(const std::vector<int32_t> &leaves, const std::vector<int64_t> &nsrc,
+                       const std::vector<int32_t> &tgt_ptr);
   int leaf_threads_ = 256;          // threads per target leaf in the leaf kernel
   void launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const int32_t *lidx, int down,
                    int accumulate, double *chk, hipStream_t s);
@@ -390,6 +392,8 @@ class Fmm {
   DBuf pleaves_, tleaves_;
   std::vector<int32_t> src_ptr_h_;  // host copy of src_ptr_ (launch order by work)
   int n_pleaves_ = 0, n_tleaves_ = 0;
+  DBuf leaf_items_, leaf_shared_, leaf_part_;   // leaves shared by several workgroups (none: empty)
+  int n_leaf_items_ = 0, n_leaf_shared_ = 0;
   int max_leaf_tgt_ = 0, ncu_ = 256;  // most targets in a leaf; compute units of the device
   // work buffers
   DBuf chk_, uppot_, downpot_, tmp_;

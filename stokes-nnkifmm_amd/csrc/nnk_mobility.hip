@@ -94,8 +94,8 @@ __global__ __launch_bounds__(256) void k_multidot(int64_t n, int k, const double
 // norm) over the slice it has just changed.  Bound by reading V four times;
 // with few vectors by the launches.  All sums in fixed orders.
 // Measured per GMRES iteration (nine launches, partial sums by one thread per
-// vector, before): 50 iterations, n about 10^4, 125 -> 30 us; 100 iterations of
-// 8 bodies, n about 3 x 10^4, 185 -> 47 us.
+// vector, before): ten squirmers in a box, 50 iterations, 125 -> 30 us; 8
+// bodies, 104 iterations, 185 -> 47 us.
 constexpr int kCgsThreads = 512, kCgsWaves = kCgsThreads / 64, kCgsSlices = 128, kCgsChunk = 1024;
 
 __device__ __forceinline__ double wave_sum(double v) {
