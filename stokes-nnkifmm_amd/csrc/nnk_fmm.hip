@@ -95,7 +95,23 @@ struct SurfArgs {
   const double *src_pos, *src_q;
   double e2, c;
   double *chk;
+  // FP64 P2L with nodes shared by several workgroups (null: none): items[
+  // blockIdx.x] is (node, part, parts, first row of its sums)
+  const int4 *items;
+  double *part;               // rows of K, part p of a node at first + p
 };
+
+// check potentials of the shared nodes (list: part 0's items): the sums of
+// their parts, in order
+__global__ __launch_bounds__(256) void k_surf_parts(SurfArgs a, const int4 *__restrict__ list) {
+  const int4 it = list[blockIdx.x];
+  for (int i = threadIdx.x; i < a.K; i += 256) {
+    double v = 0.0;
+    for (int p = 0; p < it.z; p++) v += a.part[(size_t)(it.w + p) * a.K + i];
+    double *o = a.chk + (size_t)(it.x - 1) * a.K + i;
+    *o = a.accumulate ? *o + v : v;
+  }
+}
 
 // FP32-math forms: check potential on a node surface from the sources of a
 // set of leaves (S2M: the leaf itself onto its down surface; P2L: the X list onto the up
@@ -349,7 +365,8 @@ __global__ __launch_bounds__(256) void k_surf64(SurfArgs a, const double *__rest
                                                const double *__restrict__ src_q) {
   __shared__ int pre[kLeafMaxU + 1];
   __shared__ SrcBatch buf;
-  const int n = a.nodes[blockIdx.x];
+  const int4 it = a.items ? a.items[blockIdx.x] : int4{a.nodes[blockIdx.x], 0, 1, 0};
+  const int n = it.x;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const double *box = a.corners + 6 * (size_t)(n - 1);
   const int p0 = (blockIdx.y * 4 + w) * NT;
@@ -375,8 +392,10 @@ __global__ __launch_bounds__(256) void k_surf64(SurfArgs a, const double *__rest
       const int32_t *list = a.lidx + b0;
       if (b0 > lb) __syncthreads();
       source_prefix(list, nu, a.src_ptr, pre);
-      sum_sources<NT>(tx, ty, tz, a.e2, sp, 1, pre[nu], buf,
-                      [&](int g) { return source(source_index(list, nu, a.src_ptr, pre, g)); }, u);
+      const int64_t tot = pre[nu];
+      const int ga = (int)(tot * it.y / it.z), gb = (int)(tot * (it.y + 1) / it.z);
+      sum_sources<NT>(tx, ty, tz, a.e2, sp, 1, gb - ga, buf,
+                      [&](int g) { return source(source_index(list, nu, a.src_ptr, pre, ga + g)); }, u);
     }
   } else {
     const int sb = a.src_ptr[n];
@@ -386,8 +405,9 @@ __global__ __launch_bounds__(256) void k_surf64(SurfArgs a, const double *__rest
   int idx = 0, cnt = 3 * min(NT, a.nq - p0);
   wave_scatter_sum<3 * NT, 32>(u, lane, idx, cnt);
   if (cnt > 0) {
-    double *o = a.chk + (size_t)(n - 1) * a.K + 3 * p0 + idx;
-    *o = a.c * u[0];
+    const double v = a.c * u[0];
+    double *o = (it.z > 1 ? a.part + (size_t)(it.w + it.y) * a.K : a.chk + (size_t)(n - 1) * a.K) + 3 * p0 + idx;
+    *o = a.accumulate && it.z == 1 ? *o + v : v;
   }
 }
 
@@ -1744,6 +1764,16 @@ void Fmm::plan() {
     order_by_work(xall, wx);
     n_x_all_ = (int)xall.size();
     x_all_.upload(xall);
+    if (!fp32_math()) {
+      // as the leaf kernel's lists (a node's workgroups take 32 surface points
+      // each).  P2L of 8 bodies over a wall, 250 ->
+      // 225 us a product; where the lists are even, nothing changes.
+      int64_t total = 0;
+      for (int n : xall) total += wx[n] * ((nq_ + 31) / 32);
+      x_parts_.plan(
+          xall, [&](int n) { return wx[n]; }, std::max<int64_t>(2048, total / (8 * (int64_t)ncu_)),
+          [](int) { return 1; }, (int64_t)sizeof(double) * K_);
+    }
     if (n_x_all_ && prec_ == 0) xchk_.alloc(sizeof(double) * (size_t)nc * K_);
     else xchk_ = DBuf();
   }
@@ -1902,11 +1932,49 @@ void Fmm::launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const in
   // in each of 512 leaves 30 -> 22.6 us; 32 in each of 32,768 0.19 against
   // 0.50 ms.
   if (fp32_math()) hipLaunchKernelGGL(k_surf_eval, dim3(n), dim3(kSurfThreads), 0, s, a);
-  else if (lptr || nsrc_ >= 64 * (int64_t)n)
-    hipLaunchKernelGGL(k_surf64<8>, dim3(n, (nq_ + 31) / 32), dim3(256), 0, s, a, a.src_pos, a.src_q);
+  else if (lptr || nsrc_ >= 64 * (int64_t)n) {
+    const bool shared = lptr && x_parts_.nshared;   // (the lists are the plan's: P2L has one launch)
+    if (shared) {
+      a.items = x_parts_.items.as<int4>();
+      a.part = x_parts_.part.as<double>();
+    }
+    hipLaunchKernelGGL(k_surf64<8>, dim3(shared ? x_parts_.nitems : n, (nq_ + 31) / 32), dim3(256), 0, s, a, a.src_pos,
+                       a.src_q);
+    if (shared)
+      hipLaunchKernelGGL(k_surf_parts, dim3(x_parts_.nshared), dim3(256), 0, s, a, x_parts_.shared.as<int4>());
+  }
   else
     hipLaunchKernelGGL(k_s2m64, dim3(n), dim3(64 * std::min((nq_ + 63) / 64, 8)), 0, s, a, a.src_pos, a.src_q);
   NNK_HIP(hipGetLastError());
+}
+
+// the work items of a launch whose workgroups walk lists of very different
+// lengths: item (n, part, parts, first) takes one of the parts of n; lists of
+// up to two parts stay whole.  rows(n): rows of sums per part.  False: nothing
+// is shared.
+bool WorkParts::plan(const std::vector<int32_t> &nodes, const std::function<int64_t(int)> &work, int64_t per,
+                     const std::function<int(int)> &rows, int64_t row_bytes) {
+  std::vector<int4> shares, rest, list;
+  int64_t first = 0;
+  for (int n : nodes) {
+    const int64_t w = work(n);
+    if (w <= 2 * per) {
+      rest.push_back(int4{n, 0, 1, 0});
+      continue;
+    }
+    const int parts = (int)std::min<int64_t>((w + per - 1) / per, 1024);
+    list.push_back(int4{n, 0, parts, (int)first});
+    for (int p = 0; p < parts; p++) shares.push_back(int4{n, p, parts, (int)first});
+    first += (int64_t)parts * rows(n);
+  }
+  if (list.empty() || first > (1 << 28) || first * row_bytes > ((int64_t)1 << 30)) return false;
+  shares.insert(shares.end(), rest.begin(), rest.end());
+  nitems = (int)shares.size();
+  nshared = (int)list.size();
+  items.upload(shares);
+  shared.upload(list);
+  part.alloc((size_t)(first * row_bytes));
+  return true;
 }
 
 // Shares the leaves with long source lists among several workgroups.  A
@@ -1925,26 +1993,9 @@ void Fmm::plan_leaf_parts(const std::vector<int32_t> &leaves, const std::vector<
   int64_t total = 0;
   for (int n : leaves) total += nsrc[n] * blocks(n);
   const int64_t per = std::max<int64_t>(2048, total / (8 * (int64_t)ncu_));
-  std::vector<int4> items, rest, list;
-  int64_t rows = 0;
-  for (int n : leaves) {
-    const int64_t w = nsrc[n] * (fp32_math() ? blocks(n) : 1);
-    if (w <= 2 * per) {
-      rest.push_back(int4{n, 0, 1, 0});
-      continue;
-    }
-    const int parts = (int)std::min<int64_t>((w + per - 1) / per, 1024), nt = tgt_ptr[n + 1] - tgt_ptr[n];
-    list.push_back(int4{n, 0, parts, (int)rows});
-    for (int p = 0; p < parts; p++) items.push_back(int4{n, p, parts, (int)rows});
-    rows += (int64_t)parts * nt;
-  }
-  if (list.empty() || rows > (1 << 28)) return;
-  items.insert(items.end(), rest.begin(), rest.end());
-  n_leaf_items_ = (int)items.size();
-  n_leaf_shared_ = (int)list.size();
-  leaf_items_.upload(items);
-  leaf_shared_.upload(list);
-  leaf_part_.alloc(sizeof(double) * 3 * rows);
+  leaf_parts_.plan(
+      leaves, [&](int n) { return nsrc[n] * (fp32_math() ? blocks(n) : 1); }, per,
+      [&](int n) { return tgt_ptr[n + 1] - tgt_ptr[n]; }, 3 * sizeof(double));
 }
 
 void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
@@ -1968,11 +2019,11 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   a.c = 1.0 / (8.0 * kPi * mu_);
   a.far = far;
   a.out = d_u;
-  const bool shared = far && n_leaf_shared_;
-  const int nwg = shared ? n_leaf_items_ : n_tleaves_;
+  const bool shared = far && leaf_parts_.nshared;
+  const int nwg = shared ? leaf_parts_.nitems : n_tleaves_;
   if (shared) {
-    a.items = leaf_items_.as<int4>();
-    a.part = leaf_part_.as<double>();
+    a.items = leaf_parts_.items.as<int4>();
+    a.part = leaf_parts_.part.as<double>();
   }
   const int T = far ? leaf_threads_ : 256;
   // Few target leaves (small trees, large leaves) would leave most CUs idle
@@ -1992,7 +2043,7 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
                        a, a.src_pos, a.src_q, a.tgt_pos);
   }
   if (shared)
-    hipLaunchKernelGGL(k_leaf_parts, dim3((unsigned)n_leaf_shared_), dim3(256), 0, s, a, leaf_shared_.as<int4>());
+    hipLaunchKernelGGL(k_leaf_parts, dim3((unsigned)leaf_parts_.nshared), dim3(256), 0, s, a, leaf_parts_.shared.as<int4>());
   NNK_HIP(hipGetLastError());
 }
 
@@ -2218,17 +2269,23 @@ void Fmm::apply_impl(const double *d_f, double *d_u, hipStream_t s) {
     gemm(P.up_solve2, tmp, K_, up, K_, 0, s);
   }
   mark(2, false, s);
-  if (n_x_all_) {  // P2L of every level into its own buffer
+  // P2L of every level: onto the check potentials where the frequency-space
+  // M2L has formed them all, else into its own buffer, from which each level adds
+  // its rows when its M2L is done (4.6 us per level)
+  bool x_now = spec_ != nullptr;
+  for (int l = 2; l <= maxlev_; l++) x_now = x_now && (!plans_[l].n_x || plans_[l].m2l_spec_on);
+  auto p2l = [&](int accumulate, double *out) {
     mark(5, true, s);
-    launch_surf(x_all_.as<int32_t>(), n_x_all_, xptr_.as<int64_t>(), xidx_.as<int32_t>(), 0, 0,
-                xchk_.as<double>(), s);
+    launch_surf(x_all_.as<int32_t>(), n_x_all_, xptr_.as<int64_t>(), xidx_.as<int32_t>(), 0, accumulate, out, s);
     mark(5, false, s);
-  }
+  };
+  if (n_x_all_ && !x_now) p2l(0, xchk_.as<double>());
   if (spec_) {  // the M2L of every frequency-space level (chk of levels switched to dense is rewritten below)
     mark(3, true, s);
     spec_->run(up, chk, s);
     mark(3, false, s);
   }
+  if (n_x_all_ && x_now) p2l(1, chk);
   for (int l = 2; l <= maxlev_; l++) {
     LevelPlan &P = plans_[l];
     if (!P.n_down) continue;
@@ -2241,7 +2298,7 @@ void Fmm::apply_impl(const double *d_f, double *d_u, hipStream_t s) {
     mark(4, true, s);
     gemm(P.l2l, dn, K_, chk, K_, 1, s);
     mark(4, false, s);
-    if (P.n_x) {  // chk += the P2L check potentials (as one addition each)
+    if (P.n_x && !x_now) {  // chk += the P2L check potentials (as one addition each)
       mark(5, true, s);
       hipLaunchKernelGGL(k_add_rows, dim3(P.n_x), dim3(256), 0, s, P.x_nodes.as<int32_t>(), xchk_.as<double>(), chk,
                          K_);

@@ -5,6 +5,7 @@
 
 #include <array>
 #include <map>
+#include <functional>
 #include <memory>
 #include <vector>
 
@@ -104,6 +105,15 @@ constexpr int64_t kPairBufMaxElems = (int64_t)1 << 28;
 // for 2 M^2 FP64 flops, or ~700 TF/s for the 6 M^2 flops of two-part
 // 16-bit products
 constexpr int64_t kPairRtFP64 = 90, kPairRt16 = 470;
+
+// Launches with one workgroup (row) per node whose longest lists are shared by
+// several: the items of all workgroups, the shared nodes, the parts' sums.
+struct WorkParts {
+  DBuf items, shared, part;
+  int nitems = 0, nshared = 0;
+  bool plan(const std::vector<int32_t> &nodes, const std::function<int64_t(int)> &work, int64_t per,
+            const std::function<int(int)> &rows, int64_t row_bytes);
+};
 
 struct GemmBatch {
   DBuf jobs;                 // GemmJob[n]
@@ -392,8 +402,7 @@ class Fmm {
   DBuf pleaves_, tleaves_;
   std::vector<int32_t> src_ptr_h_;  // host copy of src_ptr_ (launch order by work)
   int n_pleaves_ = 0, n_tleaves_ = 0;
-  DBuf leaf_items_, leaf_shared_, leaf_part_;   // leaves shared by several workgroups (none: empty)
-  int n_leaf_items_ = 0, n_leaf_shared_ = 0;
+  WorkParts leaf_parts_, x_parts_;   // the leaf kernel's leaves, the FP64 P2L's nodes
   int max_leaf_tgt_ = 0, ncu_ = 256;  // most targets in a leaf; compute units of the device
   // work buffers
   DBuf chk_, uppot_, downpot_, tmp_;
