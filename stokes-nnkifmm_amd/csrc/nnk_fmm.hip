@@ -459,9 +459,9 @@ __global__ __launch_bounds__(256) void k_leaf_parts(LeafArgs a, const int4 *__re
 // at a time (a leaf holds ~32: staging leaf by leaf would pay a load
 // latency and two barriers per leaf); lists longer than kLeafMaxU leaves
 // are staged leaf by leaf.
-template <int T>
+template <int T, bool SHARED>
 __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
-  const int4 it = leaf_item(a);
+  const int4 it = SHARED ? a.items[blockIdx.x] : int4{a.leaves[blockIdx.x], 0, 1, 0};
   const int n = it.x;
   // the surface sources (L2T, M2T) go through the offset stage
   // with the origin at the centre of the surface's node (this leaf for
@@ -560,7 +560,13 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
         __syncthreads();
       }
     };
-    if (a.far) {
+    if (a.far && !SHARED) {
+      surface(n, 1, a.downpot);
+      for (int64_t e = a.wptr[n]; e < a.wptr[n + 1]; e++) surface(a.widx[e], 0, a.uppot);
+      if (ucat) usources(0, upre[nu]);
+      else
+        for (int64_t e = u0; e < u1; e++) sources(a.uidx[e]);
+    } else if (a.far) {
       // the list in steps (a surface; T sources, or a leaf's, of the U list):
       // a part takes whole steps, so each step's sums are those of an unshared leaf
       const int nw = 1 + (int)(a.wptr[n + 1] - a.wptr[n]);
@@ -2035,9 +2041,10 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   const dim3 grid((unsigned)nwg, (unsigned)std::max(1, (max_leaf_tgt_ + a.tc - 1) / a.tc));
   auto go = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, grid, dim3(threads), 0, s, a); };
   if (fp32_math()) {
-    if (T == 128) go(k_leaf<128>, 128);
-    else if (T == 512) go(k_leaf<512>, 512);
-    else go(k_leaf<256>, 256);
+    // (the sharing costs an unshared launch 8 %)
+    if (T == 128) shared ? go(k_leaf<128, true>, 128) : go(k_leaf<128, false>, 128);
+    else if (T == 512) shared ? go(k_leaf<512, true>, 512) : go(k_leaf<512, false>, 512);
+    else shared ? go(k_leaf<256, true>, 256) : go(k_leaf<256, false>, 256);
   } else {
     hipLaunchKernelGGL(k_leaf64, dim3((unsigned)nwg, (unsigned)std::max(1, (max_leaf_tgt_ + 31) / 32)), dim3(256), 0, s,
                        a, a.src_pos, a.src_q, a.tgt_pos);
