@@ -1122,6 +1122,9 @@ void Fmm::gemm_dims(const GemmBatch &b, const double *X, int ldx, double *C, int
                     hipStream_t s, int M, int K, int Mpad, int Kpad, int nsplit, const DBuf *slot, int tag) {
   if (b.njobs == 0 || b.maxN == 0) return;
   if (Mpad % GBM || Kpad % GBK) throw Error(NNK_ESTATE, "gemm_dims: bad padding");
+  if (tag == 0 && nsplit == 1 &&
+      launch_gemm_ordered(M, K, Mpad, Kpad, X, ldx, C, ldc, beta, b.jobs.as<GemmJob>(), b.njobs, b.maxN, s))
+    return;
   // tag 1: the M2L's own kernel symbol (profiles tell it from the other GEMMs)
   auto go = [&](int bt, double *P, int ns) {
     if (tag == 1) launch_gemm<GBN1, 1>(Mpad / GBM, M, K, Mpad, Kpad, X, ldx, C, ldc, bt, b, s, ns, P);

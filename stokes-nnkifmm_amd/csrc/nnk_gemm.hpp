@@ -231,10 +231,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_gather(int M, int K, int Mpad, 
 // few tiles, which are bound by the latency of the chunks in a row.
 // The row blocks of a column tile are 8 workgroups apart, on one XCD, so its
 // columns come from one L2.
-template <int TM, int TN, int KS>
+// ORD (KS = 1): the summation order of k_gemm_gather, to the bit: product s of a
+// chunk takes k = 4 s + lk.
+template <int TM, int TN, int KS, bool ORD = false>
 __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
     int M, int K, int Mpad, int Kpad, const double *__restrict__ X, int ldx, double *__restrict__ C, int ldc, int beta,
     const GemmJob *__restrict__ jobs, int njobs, int nrb, int nct) {
+  static_assert(!ORD || KS == 1, "one chain per sum");
   constexpr int WAVES = KS > 4 ? KS : 4, CW = WAVES / KS;   // wavefronts, column tiles of a workgroup
   __shared__ double red[KS > 1 ? (WAVES - CW) * TM * TN * 256 : 1];
   __shared__ int act[16], nact_s;
@@ -293,6 +296,20 @@ __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
         xc[j] = (gcd)X + (size_t)(g < 0 ? 0 : g) * ldx;
       }
     }
+    if constexpr (ORD) {
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int k = min(k0 - 3 * lk + 4 * s, K - 1);   // (chunk start) + lk + 4 s
+#pragma unroll
+        for (int i = 0; i < TM; i++) a[s][i] = Ab[(size_t)k * Mpad + min((rt0 + i) * 16, Mpad - 16) + lr];
+#pragma unroll
+        for (int j = 0; j < TN; j++) x[j][s] = xc[j][k];
+      }
+      // hi: products with k < K count
+#pragma unroll
+      for (int j = 0; j < TN; j++) lo[j] = on[j] ? (K - (k0 - 3 * lk) + 3) / 4 : 0;
+      return;
+    }
     const int kb = max(min(k0, K - 4), 0);
 #pragma unroll
     for (int s = 0; s < 4; s++)
@@ -310,7 +327,7 @@ __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
     for (int s = 0; s < 4; s++) {
       double v[TN];
 #pragma unroll
-      for (int j = 0; j < TN; j++) v[j] = s >= lo[j] && s < K ? x[j][s] : 0.0;
+      for (int j = 0; j < TN; j++) v[j] = (ORD ? s < lo[j] : s >= lo[j] && s < K) ? x[j][s] : 0.0;
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -329,7 +346,7 @@ __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
       fetch(min(c + 1, c1 - 1), a1, x1, l1);
       if (c + 1 == c1)
 #pragma unroll
-        for (int j = 0; j < TN; j++) l1[j] = 4;
+        for (int j = 0; j < TN; j++) l1[j] = ORD ? 0 : 4;
       __builtin_amdgcn_sched_barrier(0);   // the loads go out before the products, not among them
       product(a0, x0, l0);
       fetch(min(c + 2, c1 - 1), a0, x0, l0);
@@ -396,6 +413,21 @@ inline void launch_gemm_direct(int M, int K, int Mpad, int Kpad, const double *X
   if (wgs(48, 128) >= 512) go(k_gemm_direct<3, 2, 1>, 256, 48, 128);
   else if (wgs(48, 32) >= 256) go(k_gemm_direct<3, 2, 4>, 256, 48, 32);
   else go(k_gemm_direct<2, 1, 8>, 512, 32, 16);
+}
+
+// The product in k_gemm_gather's order, for the truncated forms' launches of few
+// of its tiles.  False: not launched, k_gemm_gather is the faster.  L2L of a
+// 20-body suspension (up to 144 tiles per level) 0.215 -> 0.137 ms; of 10^5
+// clustered points, levels of 192 to 512 tiles included, 0.45 against 0.52 ms.
+inline bool launch_gemm_ordered(int M, int K, int Mpad, int Kpad, const double *X, int ldx, double *C, int ldc,
+                                int beta, const GemmJob *jobs, int njobs, int maxN, hipStream_t s) {
+  if ((int64_t)njobs * (Mpad / GBM) * ((maxN + GBN0 - 1) / GBN0) >= 192) return false;
+  const int nrb = (M + 31) / 32, nct = (maxN + 63) / 64;
+  const int64_t units = ((int64_t)njobs * nct + 7) / 8 * 8;
+  hipLaunchKernelGGL((k_gemm_direct<2, 1, 1, true>), dim3((unsigned)(units * nrb)), dim3(256), 0, s, M, K, Mpad, Kpad, X,
+                     ldx, C, ldc, beta, jobs, njobs, nrb, nct);
+  NNK_HIP(hipGetLastError());
+  return true;
 }
 
 // C[slot[c]][row] = sum over splits of P[split][c][row], splits in order

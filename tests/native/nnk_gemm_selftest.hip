@@ -14,7 +14,7 @@ using namespace nnk;
 // none)
 extern "C" int nnk_selftest_gemm_direct(int M, int K, int Mpad, int Kpad, const double *at, int nb, const double *x,
                                         int nx, int ldx, const int *gidx, const int *cidx, const int *N, int njobs,
-                                        double *c, int nc, int ldc, int beta) {
+                                        double *c, int nc, int ldc, int beta, int ordered) {
   try {
     const size_t mat = (size_t)Kpad * Mpad;
     DBuf dA, dX, dC, dP, dJ;
@@ -46,8 +46,17 @@ extern "C" int nnk_selftest_gemm_direct(int M, int K, int Mpad, int Kpad, const 
       maxN = std::max(maxN, N[j]);
     }
     dJ.upload(jobs);
-    launch_gemm_direct(M, K, Mpad, Kpad, dX.as<double>(), ldx, dC.as<double>(), ldc, beta, dJ.as<GemmJob>(), njobs,
-                       maxN, 0);
+    if (!ordered)
+      launch_gemm_direct(M, K, Mpad, Kpad, dX.as<double>(), ldx, dC.as<double>(), ldc, beta, dJ.as<GemmJob>(), njobs,
+                         maxN, 0);
+    else if (ordered == 1) {
+      if (!launch_gemm_ordered(M, K, Mpad, Kpad, dX.as<double>(), ldx, dC.as<double>(), ldc, beta, dJ.as<GemmJob>(),
+                               njobs, maxN, 0))
+        return 2;
+    } else   // the kernel whose order it has
+      hipLaunchKernelGGL((k_gemm_gather<GBM, GBN0, GBK, 0>), dim3(njobs * (Mpad / GBM) * ((maxN + GBN0 - 1) / GBN0)),
+                         dim3(256), 0, 0, M, K, Mpad, Kpad, dX.as<double>(), ldx, dC.as<double>(), ldc, beta,
+                         dJ.as<GemmJob>(), njobs, Mpad / GBM, 1, nullptr, maxN);
     NNK_HIP(hipDeviceSynchronize());
     NNK_HIP(hipMemcpy(c, dC.p, sizeof(double) * (size_t)nc * ldc, hipMemcpyDeviceToHost));
     return 0;

@@ -27,6 +27,21 @@ def selftest(nnk):
     (24, 24, 8, (65500,), 0), (456, 168, 2, (6530,), 1), (100, 2, 1, (22000,), 0),            # 48 x 128, one
 ])
 def test_direct_gemm(selftest, M, K, nb, widths, beta):
+    c, ref, mod = _run(selftest, M, K, nb, widths, beta, 0)
+    assert (np.abs(c - ref) <= (nb * K + 8) * EPS * mod).all()
+
+
+@pytest.mark.parametrize("M,K,nb,widths,beta", [
+    (24, 24, 8, (1,), 0), (2, 3, 1, (5,), 0), (3, 2, 8, (17, 3), 1), (33, 4, 2, (16,), 0), (168, 168, 8, (65,), 0),
+    (457, 457, 1, (64, 9, 0, 200), 1), (456, 30, 3, (101,), 1), (17, 1158, 1, (130,), 0)])
+def test_ordered_gemm(selftest, M, K, nb, widths, beta):
+    """The ordered launch has the bits of the kernel whose order it keeps."""
+    c, ref, mod = _run(selftest, M, K, nb, widths, beta, 1)
+    assert (np.abs(c - ref) <= (nb * K + 8) * EPS * mod).all()
+    assert np.array_equal(c, _run(selftest, M, K, nb, widths, beta, 2)[0])
+
+
+def _run(selftest, M, K, nb, widths, beta, ordered):
     rng = np.random.default_rng(M * K + nb)
     Mpad, Kpad, ldx, ldc = -(-M // 160) * 160, -(-K // 16) * 16, max(K, 32) + 2, M + 3
     nx, nc = 60, sum(widths) + 4
@@ -51,5 +66,5 @@ def test_direct_gemm(selftest, M, K, nb, widths, beta):
     w = np.array(widths, np.int32)
     assert selftest.nnk_selftest_gemm_direct(
         M, K, Mpad, Kpad, at.ctypes.data_as(d), nb, x.ctypes.data_as(d), nx, ldx, gf.ctypes.data_as(ip),
-        slots.ctypes.data_as(ip), w.ctypes.data_as(ip), len(widths), c.ctypes.data_as(d), nc, ldc, beta) == 0
-    assert (np.abs(c - ref) <= (nb * K + 8) * EPS * mod).all()
+        slots.ctypes.data_as(ip), w.ctypes.data_as(ip), len(widths), c.ctypes.data_as(d), nc, ldc, beta, ordered) == 0
+    return c, ref, mod
