@@ -31,7 +31,9 @@ Forms timed (all reported under "forms"):
 
 Prints one JSON line.  Besides the throughput it reports:
   roofline      the headline form's M2L translation GEMM (the dominant
-                kernel): its MFMA flops (FP64: 2 (3Nq)^2 per V-list pair;
+                kernel): its MFMA flops (FP64 in frequency space: 72
+                per V-list pair and frequency, the transforms not
+                counted; FP64 truncated: 2 R^2 per pair;
                 mixed: 3 BF16 products of 2 R^2 per pair, R the
                 pseudo-inverse rank) over its HIP-event time in the timed
                 region, against the MI355X dense MFMA peak of that type;
@@ -258,7 +260,10 @@ def run_form(nnk, lib, tree, fd, args, eps, mu, precision, res, svd_tol):
     K, R = int(st[12]), int(st[13])
     ms_step = dt / args.steps * 1e3
     phases = ["strengths", "S2M", "up", "M2L", "L2L", "P2L", "down", "leaf"]
-    if precision in ("fp64", "fp64t"):
+    if precision == "fp64" and all(int(dep[l]) == 1 for l in range(16) if spl[l] > 0):
+        flops = m2l_frequency_flops(res) * st[0]
+        peak, kern = FP64_MFMA_PEAK_TFLOPS, "k_spec_gemm (M2L in frequency space, FP64 MFMA; k_spec_fwd, k_spec_inv)"
+    elif precision in ("fp64", "fp64t"):
         r = K if precision == "fp64" else R
         flops = 2.0 * r * r * st[0]
         pairs = any(int(dep[l]) == 1 for l in range(16) if spl[l] > 0)
@@ -282,7 +287,7 @@ def run_form(nnk, lib, tree, fd, args, eps, mu, precision, res, svd_tol):
     achieved = flops / (m2l_ms * 1e-3) / 1e12 if m2l_ms > 0 else 0.0
     rec = {"precision": precision, "coronaRes": res, "svd_tol": svd_tol if precision != "fp64" else None,
            "rank": R if precision != "fp64" else K,
-           "matvec_roofline": matvec_roofline(precision, st, K, R, ms_step), "Mpts_s": round(tree.points.shape[0] / (ms_step * 1e-3) / 1e6, 4),
+           "matvec_roofline": matvec_roofline(precision, st, K, R, ms_step, res), "Mpts_s": round(tree.points.shape[0] / (ms_step * 1e-3) / 1e6, 4),
            "ms_per_step": round(ms_step, 3), "setup_s": round(t_setup, 3),
            "phase_ms_per_step": {p: round(float(ms[i] / args.steps), 3) for i, p in enumerate(phases)},
            "m2l_launch_per_level": {str(l): {"split": int(spl[l]), "depth": int(dep[l])}
@@ -294,13 +299,21 @@ def run_form(nnk, lib, tree, fd, args, eps, mu, precision, res, svd_tol):
     return u, rec
 
 
-def matvec_roofline(precision, st, K, R, ms_step):
+def m2l_frequency_flops(res):
+    """Flops of one V-list pair in frequency space: a complex 3 x 3 product
+    (9 multiply-adds of 8 flops) at each of the ((2 res - 1)^3 + 1) / 2
+    frequencies of a real transform."""
+    return 72.0 * ((2 * res - 1) ** 3 + 1) / 2
+
+
+def matvec_roofline(precision, st, K, R, ms_step, res):
     """Sum over the matvec's kernel classes of (algorithmic flops / that
     class's peak), over the measured time per matvec.  Work counts from
     nnk_fmm_stats: 0 M2L pairs, 1 P2P pairs, 2 S2M pairs, 3 L2T pairs,
     4 M2T pairs, 5 P2L pairs, 6 up-solve nodes, 7 down-solve nodes, 8 M2M
-    parents, 9 L2L nodes.  FP64 form: every translation and solve is a
-    (3Nq)^2 FP64 GEMM per node (two factors per solve).  Truncated forms:
+    parents, 9 L2L nodes.  FP64 form: the M2L in frequency space (coronaRes
+    3 to 10; its transforms are not counted), every other translation and
+    solve a (3Nq)^2 FP64 GEMM per node (two factors per solve).  Truncated forms:
     R x R translations and the leaves' R x 3Nq up expansions (the down and
     W expansions are not counted); M2L on 16-bit parts counts every split
     product (3 or 6); direct sums at 33 flop per pair on the VALU (FP32
@@ -312,7 +325,7 @@ def matvec_roofline(precision, st, K, R, ms_step):
     cls = {"direct_sums (P2P, S2M, L2T, M2T, P2L)": (PAIR_FLOPS * pairs, direct_peak)}
     if precision == "fp64":
         k2 = 2.0 * K * K
-        cls["M2L"] = (k2 * st[0], f64m)
+        cls["M2L"] = ((m2l_frequency_flops(res) if 3 <= res <= 10 else k2) * st[0], f64m)
         cls["M2M + L2L"] = (k2 * (8 * st[8] + st[9]), f64m)
         cls["equivalent-density solves"] = (2 * k2 * (st[6] + st[7]), f64m)
     else:
@@ -329,13 +342,13 @@ def matvec_roofline(precision, st, K, R, ms_step):
                         for k, (f, pk) in cls.items()}}
 
 
-def handle_ideal_ms(lib, h, precision):
+def handle_ideal_ms(lib, h, precision, res):
     """Ideal time (ms) of one matvec of a KIFMM handle: the roofline sum of
     matvec_roofline over its work counts."""
     P = ctypes.POINTER
     st = np.zeros(14, np.int64)
     lib.nnk_fmm_stats(h.h, st.ctypes.data_as(P(ctypes.c_int64)), 14)
-    return matvec_roofline(precision, st, int(st[12]), int(st[13]), 1.0)["ideal_ms"]
+    return matvec_roofline(precision, st, int(st[12]), int(st[13]), 1.0, res)["ideal_ms"]
 
 
 def direct_sample(lib, pts, fd, idx, eps, mu):
@@ -423,8 +436,8 @@ def spheroid_solve(nnk):
     # coronaRes-4 matvec at their ideal (roofline-sum) times; the leaf-block
     # solves, SpMVs and Arnoldi vectors are not counted (a lower bound)
     lib = nnk.lib()
-    i6 = handle_ideal_ms(lib, sw.FMM._handle(), "fp64")
-    i4 = handle_ideal_ms(lib, sw.FMM._handle(res=4), "fp64")
+    i6 = handle_ideal_ms(lib, sw.FMM._handle(), "fp64", 6)
+    i4 = handle_ideal_ms(lib, sw.FMM._handle(res=4), "fp64", 4)
     ideal_s = (info["iter"] + 2) * (i6 + i4) * 1e-3
     out["fp64_precon"] = {"wall_s": round(dt, 3), "iterations": info["iter"], "relres": info["relres"],
                           "roofline": {"frac": round(ideal_s / dt, 4), "ideal_s": round(ideal_s, 4),
@@ -457,7 +470,7 @@ def spheroid_solve(nnk):
     # one mixed coronaRes-4 matvec, each outer iteration the FP64 pair, at
     # their ideal (roofline-sum) times (a lower bound, as for the FP64 solve)
     inner6, inner4 = sw._mobility.inner[("mixed", 1e-8, True, 6)]
-    m6, m4 = handle_ideal_ms(lib, inner6, "mixed"), handle_ideal_ms(lib, inner4, "mixed")
+    m6, m4 = handle_ideal_ms(lib, inner6, "mixed", 6), handle_ideal_ms(lib, inner4, "mixed", 4)
     ideal_f = (info["iter"] * (m6 + m4) + (info["outer"] + 2) * (i6 + i4)) * 1e-3
     out["mixed_fgmres_precon"] = {
         "wall_s": round(dt, 3), "inner_iterations": info["iter"], "outer": info["outer"], "inner_tol": 1e-2,
@@ -474,8 +487,8 @@ def spheroid_solve(nnk):
 def batched_solves(nnk):
     """256 independent single-body problems (spheres and spheroids, 200-5000
     force points log-uniform, 4x refined quadrature, eps in [0.002, 0.02]):
-    one batched GMRES to 1e-6, HIP-graph replay of the persistent batched
-    operator with its P2P workgroup size autotuned, FP64 and FP32-math."""
+    one batched GMRES to 1e-6, HIP-graph replay of the batched
+    operator, FP64 and FP32-math."""
     import importlib as il
     geo = il.import_module("stokes-nnkifmm_amd.geometries")
     t0 = time.perf_counter()

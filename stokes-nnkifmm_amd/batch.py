@@ -90,8 +90,8 @@ class BatchedMobility:
         self.last_solve = {}
 
     def p2pWaves(self):
-        """Wavefronts per workgroup of the batched P2P (autotuned on the
-        first operator application when autotune=True; 4 otherwise)."""
+        """4 (the batched pair sums have one launch shape; kept for callers
+        that report it)."""
         v = ctypes.c_int32()
         check(lib().nnk_batch_p2p_waves(self.h, ctypes.byref(v)))
         return int(v.value)

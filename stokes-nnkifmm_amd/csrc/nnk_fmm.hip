@@ -1,16 +1,18 @@
 // KIFMM matvec on gfx950, FP64 form.
 //
 // Pass structure follows Tools/Passes/upwardPass.m and downwardPass.m:
+// (kernels of the FP64 form; the FP32-math forms evaluate surfaces with
+// k_surf_eval and leaves with k_leaf)
 //   S2M   (Up.m:31-33)          check potential of a leaf's sources on its
-//                               down surface                  k_surf_eval
+//                               down surface                  k_s2m64, k_surf64
 //   M2M   (upwardPass.m:81-93)  children's up densities onto the parent's
 //                               down surface                  gemm (8 ops)
 //   up solve  K(up->down) \ chk per level                     gemm x2 (SVD)
-//   M2L   (DownNonleaf.m:42)    V list onto the up surface    gemm (189 ops)
+//   M2L   (DownNonleaf.m:42)    V list onto the up surface    SpectralM2L, else gemm (189 ops)
 //   L2L   (DownNonleaf.m:44)    parent down density           gemm (1 op, +=)
-//   P2L   (DownNonleaf.m:43)    X-list sources                k_surf_eval
+//   P2L   (DownNonleaf.m:43)    X-list sources                k_surf64
 //   down solve  K(down->up) \ chk per level                   gemm x2 (SVD)
-//   L2T+P2P+M2T (Downleaf.m:37-40) per target leaf            k_leaf
+//   L2T+P2P+M2T (Downleaf.m:37-40) per target leaf            k_leaf64
 // Per-level operators use the level's canonical box geometry (all boxes of a
 // level share their width; their absolute corners differ from the canonical
 // ones only by rounding).  The check-to-equivalent solves apply one-sided
