@@ -2065,6 +2065,7 @@ void Fmm::apply(const double *d_f, double *d_u, hipStream_t s) {
     autotune(s);
     autotune_leaf(s);
     tuned_ = true;
+    launches_changed();
   }
   apply_impl(d_f, d_u, s);
 }
@@ -2086,22 +2087,34 @@ void Fmm::launch_config(int level, int *split, int *depth) const {
   }
 }
 
+// before buffers that captured launches may hold are freed, or once the
+// launches are others: replays in flight end, captured graphs are not used
+// again
+void Fmm::launches_changed() {
+  NNK_HIP(hipDeviceSynchronize());
+  gen_++;
+  gop_.reset();
+}
+
 void Fmm::set_launch_config(int level, int split, int depth) {
   if (level < 2 || level > maxlev_) throw Error(NNK_EARG, "launch config: level without M2L");
   LevelPlan &P = plans_[level];
   const bool mixed = m16();
   if (mixed ? !P.mx_m2l_jobs : !P.n_down) throw Error(NNK_EARG, "launch config: level without M2L");
+  if (split < 1 || split > 64) throw Error(NNK_EARG, "launch config: split-K factor out of range");
   if (P.m2l_spec && depth == 1) {
     if (split != 1) throw Error(NNK_EARG, "launch config: the frequency-space M2L takes split 1");
     P.m2l_spec_on = true;
-    gop_.reset();
+    launches_changed();
     return;
   }
-  if (P.m2l_spec && depth == 0) plan_m2l_dense(level);
+  if (P.m2l_spec && depth == 0 && !P.m2l_dense) {
+    launches_changed();   // the part and pair buffers may move, also where the split is refused below
+    plan_m2l_dense(level);
+  }
   const size_t per_split = mixed ? (size_t)P.mx_m2l_jobs * P.mx_m2l_maxN * RP_
                                  : (size_t)P.m2l.njobs * P.m2l.maxN * m2l_ld();
-  if (split < 1 || split > 64 || (split > 1 && ((size_t)split * per_split > part_elems_ ||
-                                                !(mixed ? P.mx_slot.p : P.m2l_slot.p))))
+  if (split > 1 && ((size_t)split * per_split > part_elems_ || !(mixed ? P.mx_slot.p : P.m2l_slot.p)))
     throw Error(NNK_EARG, "launch config: split-K factor out of range");
   if (!mixed) {
     if (depth == 1) {
@@ -2129,7 +2142,7 @@ void Fmm::set_launch_config(int level, int split, int depth) {
     P.mx_depth = depth;
     P.m2l_pair_on = false;
   }
-  gop_.reset();
+  launches_changed();
 }
 
 void Fmm::autotune(hipStream_t s) {

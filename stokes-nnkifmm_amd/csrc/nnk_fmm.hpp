@@ -285,6 +285,10 @@ class Fmm {
   // or 4 for the DMA-staged FP16 kernel); throws if the level has no M2L
   // or the form cannot run it.  A captured graph is dropped.
   void set_launch_config(int level, int split, int depth);
+  // counts the changes to what a graph captured from this operator holds
+  // (launches, buffer addresses): such a graph replays only while the count
+  // it was captured at stands
+  uint64_t generation() const { return gen_; }
   // threads per target leaf of the leaf kernel (L2T + P2P + M2T)
   int leaf_threads() const { return leaf_threads_; }
   // leaf-local product (reducedPass.m) on device pointers
@@ -452,6 +456,8 @@ class Fmm {
   bool prof_ = false;
   bool tune_ = false, tuned_ = false;
   GraphOp gop_;
+  uint64_t gen_ = 0;
+  void launches_changed();
   struct Mark { int phase; hipEvent_t a, b; };
   std::vector<Mark> marks_;
   hipEvent_t open_ = nullptr;

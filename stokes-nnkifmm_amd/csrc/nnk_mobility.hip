@@ -445,10 +445,16 @@ void Mobility::op(const double *x, double *y, bool use_precon, hipStream_t s) {
 
 void Mobility::op_any(const double *x, double *y, bool use_precon, hipStream_t s) {
   if (!graph_) { op(x, y, use_precon, s); return; }
-  GraphOp &G = gops_[(use_precon ? 1 : 0) + (Fcur_ ? 2 : 0)];
-  if (!G.ready()) {
+  const int k = (use_precon ? 1 : 0) + (Fcur_ ? 2 : 0);
+  GraphOp &G = gops_[k];
+  auto gen = [](const Fmm *f) { return f ? f->generation() : 0; };
+  auto gens = [&]() { return std::array<uint64_t, 4>{gen(F_), gen(F4_), gen(Fi_), gen(F4i_)}; };
+  // an operator whose launches have changed since the capture (a caller's
+  // launch configuration) may also have moved the buffers the graph names
+  if (!G.ready() || gens_[k] != gens()) {
     op(x, y, use_precon, s);  // eager first call: settles lazy set-up (leaf LU, buffers)
     NNK_HIP(hipStreamSynchronize(s));
+    gens_[k] = gens();
     G.capture(n_, n_, [&](const double *in, double *out, hipStream_t cs) { op(in, out, use_precon, cs); });
     return;
   }

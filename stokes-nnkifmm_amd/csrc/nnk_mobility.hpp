@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <vector>
 
 #include "nnk_common.hpp"
@@ -82,6 +83,8 @@ class Mobility {
   DBuf aos_a_, aos_b_, t3a_, t3b_, s6a_, s6b_, px_, part_;
   bool graph_ = false;
   GraphOp gops_[4];
+  // generations of F_, F4_, Fi_, F4i_ when each graph was captured
+  std::array<uint64_t, 4> gens_[4] = {};
 };
 
 }  // namespace nnk
