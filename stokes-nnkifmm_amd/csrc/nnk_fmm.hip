@@ -1636,7 +1636,7 @@ void Fmm::plan() {
     if (gidx) { B.owned.emplace_back(make_dbuf(*gidx)); j.gidx = B.owned.back().as<int32_t>(); }
     if (cidx) { B.owned.emplace_back(make_dbuf(*cidx)); j.cidx = B.owned.back().as<int32_t>(); }
     j.nb = (int)A.size();
-    if (j.nb > 512) throw Error(NNK_ESTATE, "too many operator blocks in one GEMM job");
+    if (j.nb > kMaxBlocks) throw Error(NNK_ESTATE, "too many operator blocks in one GEMM job");
     j.N = N;
     jobs.push_back(j);
     B.maxN = std::max(B.maxN, N);
@@ -1833,7 +1833,7 @@ void Fmm::plan_m2l_dense(int l) {
     if (H.cls[a].empty()) continue;
     for (int sl : class_offset_slots(a)) cops[a].push_back(trans_[l] ? trans_[l]->tslot[sl] : nullptr);
     const int nb = (int)cops[a].size(), N = (int)H.cls[a].size();
-    if (nb > 512) throw Error(NNK_ESTATE, "too many operator blocks in one GEMM job");
+    if (nb > kMaxBlocks) throw Error(NNK_ESTATE, "too many operator blocks in one GEMM job");
     // active blocks per 64-column tile of the M2L launch
     std::vector<int32_t> tp, tl;
     tile_lists(H.gv[a], nb, N, GBN1, tp, tl);

@@ -22,6 +22,8 @@ struct RedArgs;
 // operators' padding); columns per tile of its M2L launches (GBN1) and of the
 // truncated forms' expansions, M2M and L2L (GBN0)
 constexpr int GBM = 160, GBK = 16, GBN1 = 64, GBN0 = 32;
+// most operator blocks of a job (the kernels list the active ones in LDS)
+constexpr int kMaxBlocks = 512;
 
 struct GemmJob {
   const double *const *A;  // nb operator pointers, each At[Kpad][Mpad] (k-major)

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_gather(int M, int K, int Mpad, 
   constexpr int BKP = BK + 2;           // padded B row (keeps 16-byte alignment)
   __shared__ __attribute__((aligned(16))) double As[2][BK][BM];
   __shared__ __attribute__((aligned(16))) double Bs[2][BN][BKP];
-  __shared__ int act[512];
+  __shared__ int act[kMaxBlocks];
   __shared__ int nact_s;
 
   const int bid = blockIdx.x;
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_gather(int M, int K, int Mpad, 
 }
 
 // The same product for the FP64 form's M2M, L2L and check-to-equivalent
-// solves (jobs of at most 16 operator blocks), without LDS staging.  An FP64
+// solves (jobs of one or eight operator blocks), without LDS staging.  An FP64
 // MFMA holds the matrix core for 64 cycles, so a wavefront of TM x TN tiles of
 // 16 x 16 needs one fragment load per TM TN / (TM + TN) products: little
 // enough to load the fragments straight from memory, one 16-deep K chunk
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
   static_assert(!ORD || KS == 1, "one chain per sum");
   constexpr int WAVES = KS > 4 ? KS : 4, CW = WAVES / KS;   // wavefronts, column tiles of a workgroup
   __shared__ double red[KS > 1 ? (WAVES - CW) * TM * TN * 256 : 1];
-  __shared__ int act[16], nact_s;
+  __shared__ int act[kMaxBlocks], nact_s;
   const int q = blockIdx.x >> 3, u = (q / nrb) * 8 + (blockIdx.x & 7), rb = q % nrb;
   if (u >= njobs * nct) return;
   const GemmJob J = jobs[u % njobs];
