@@ -96,6 +96,7 @@ struct SurfArgs {
   const int32_t *src_ptr;     // per node id, [src_ptr[n], src_ptr[n+1])
   const double *src_pos, *src_q;
   double e2, c;
+  double pad;                 // an x coordinate beyond every surface point
   double *chk;
   // FP64 P2L with nodes shared by several workgroups (null: none): items[
   // blockIdx.x] is (node, part, parts, first row of its sums)
@@ -326,11 +327,12 @@ typedef double SrcBatch[2][6][256];
 // chunks sp, sp + nsplit, ... of a batch.  Called by the whole workgroup.
 template <int NT, class Get>
 __device__ __forceinline__ void sum_sources(const double (&tx)[NT], const double (&ty)[NT], const double (&tz)[NT],
-                                            double e2, int sp, int nsplit, int tot, SrcBatch buf, Get &&get,
+                                            double e2, double pad, int sp, int nsplit, int tot, SrcBatch buf, Get &&get,
                                             double (&u)[3 * NT]) {
   const int tid = threadIdx.x, lane = tid & 63;
-  // past the end: strength zero, one unit off a target
-  const Src6 none{tx[0] + 1.0, ty[0], tz[0], 0.0, 0.0, 0.0};
+  // past the end: strength zero, away from every target (where 0 x the kernel
+  // would be NaN if eps^-3 overflows)
+  const Src6 none{pad, ty[0], tz[0], 0.0, 0.0, 0.0};
   auto stage = [&](int b, const Src6 &s) {
     buf[b][0][tid] = s.x;
     buf[b][1][tid] = s.y;
@@ -396,12 +398,12 @@ __global__ __launch_bounds__(256) void k_surf64(SurfArgs a, const double *__rest
       source_prefix(list, nu, a.src_ptr, pre);
       const int64_t tot = pre[nu];
       const int ga = (int)(tot * it.y / it.z), gb = (int)(tot * (it.y + 1) / it.z);
-      sum_sources<NT>(tx, ty, tz, a.e2, sp, 1, gb - ga, buf,
+      sum_sources<NT>(tx, ty, tz, a.e2, a.pad, sp, 1, gb - ga, buf,
                       [&](int g) { return source(source_index(list, nu, a.src_ptr, pre, ga + g)); }, u);
     }
   } else {
     const int sb = a.src_ptr[n];
-    sum_sources<NT>(tx, ty, tz, a.e2, sp, 1, a.src_ptr[n + 1] - sb, buf, [&](int g) { return source(sb + g); }, u);
+    sum_sources<NT>(tx, ty, tz, a.e2, a.pad, sp, 1, a.src_ptr[n + 1] - sb, buf, [&](int g) { return source(sb + g); }, u);
   }
   if (p0 >= a.nq) return;
   int idx = 0, cnt = 3 * min(NT, a.nq - p0);
@@ -427,6 +429,7 @@ struct LeafArgs {
   const int64_t *wptr; const int32_t *widx;
   const double *uppot, *downpot;
   double e2, c;
+  double pad;       // an x coordinate beyond every target
   int far;          // 0: sources of the leaf itself only (reducedPass.m)
   int tc;           // targets per workgroup and pass (<= T); blockIdx.y picks the chunk
   double *out;      // ntgt x 3
@@ -637,7 +640,7 @@ __device__ __forceinline__ void leaf_block64(const LeafArgs &a, const double *__
       source_prefix(list, nu, a.src_ptr, pre);
       const int64_t tot = s0 + pre[nu];
       const int ga = (int)(tot * part / parts), gb = (int)(tot * (part + 1) / parts);
-      sum_sources<NT>(tx, ty, tz, a.e2, sp, nsplit, gb - ga, buf, [&](int i) {
+      sum_sources<NT>(tx, ty, tz, a.e2, a.pad, sp, nsplit, gb - ga, buf, [&](int i) {
         const int g = ga + i;
         if (g >= s0) return point(source_index(list, nu, a.src_ptr, pre, g - s0));
         const int k = g / a.nq, p = g - k * a.nq;
@@ -654,7 +657,7 @@ __device__ __forceinline__ void leaf_block64(const LeafArgs &a, const double *__
     } while (b0 < u1);
   } else {  // reducedPass.m: the leaf's own sources
     const int sb = a.src_ptr[n];
-    sum_sources<NT>(tx, ty, tz, a.e2, sp, nsplit, a.src_ptr[n + 1] - sb, buf, [&](int g) { return point(sb + g); }, u);
+    sum_sources<NT>(tx, ty, tz, a.e2, a.pad, sp, nsplit, a.src_ptr[n + 1] - sb, buf, [&](int g) { return point(sb + g); }, u);
   }
   int idx = 0, cnt = 3 * NT;
   wave_scatter_sum<3 * NT, 32>(u, threadIdx.x & 63, idx, cnt);
@@ -1934,6 +1937,7 @@ void Fmm::launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const in
   a.src_pos = src_pos_.as<double>();
   a.src_q = src_q_.as<double>();
   a.e2 = eps_ * eps_;
+  a.pad = tree_.corners[3] + 4.0 * w0_;
   a.c = 1.0 / (8.0 * kPi * mu_);
   a.chk = chk;
   // FP64 S2M: k_s2m64 walks a leaf's sources one after the other on three
@@ -2027,6 +2031,7 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
   a.uppot = uppot_.as<double>();
   a.downpot = downpot_.as<double>();
   a.e2 = eps_ * eps_;
+  a.pad = tree_.corners[3] + 4.0 * w0_;
   a.c = 1.0 / (8.0 * kPi * mu_);
   a.far = far;
   a.out = d_u;
