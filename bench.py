@@ -260,13 +260,13 @@ def run_form(nnk, lib, tree, fd, args, eps, mu, precision, res, svd_tol):
     K, R = int(st[12]), int(st[13])
     ms_step = dt / args.steps * 1e3
     phases = ["strengths", "S2M", "up", "M2L", "L2L", "P2L", "down", "leaf"]
-    if precision == "fp64" and all(int(dep[l]) == 1 for l in range(16) if spl[l] > 0):
+    if precision == "fp64" and 3 <= res <= 10 and all(int(dep[l]) == 1 for l in range(16) if spl[l] > 0):
         flops = m2l_frequency_flops(res) * st[0]
         peak, kern = FP64_MFMA_PEAK_TFLOPS, "k_spec_gemm (M2L in frequency space, FP64 MFMA; k_spec_fwd, k_spec_inv)"
     elif precision in ("fp64", "fp64t"):
         r = K if precision == "fp64" else R
         flops = 2.0 * r * r * st[0]
-        pairs = any(int(dep[l]) == 1 for l in range(16) if spl[l] > 0)
+        pairs = any(int(dep[l]) in (1, 2) for l in range(16) if spl[l] > 0)
         peak, kern = FP64_MFMA_PEAK_TFLOPS, "k_gemm_gather<160,64,16,1> (M2L, FP64 MFMA" + \
             ("; per-offset pair jobs + k_pair_sum at some levels)" if pairs else ")")
     else:

@@ -220,8 +220,9 @@ int32_t nnk_fmm_launch_config(const nnk_fmm *h, int32_t *split, int32_t *depth, 
  *           class tiles, or 1 (split 1) for what the planner chose over
  *           them: the frequency-space M2L ("fp64", coronaRes 3-10 with one
  *           shell), or per-offset pair jobs (sparse adaptive levels, whose
- *           class tiles would mostly multiply empty columns); 2 or 3
- *           (register-ring depth) for
+ *           class tiles would mostly multiply empty columns), or 2 (split 1)
+ *           for such pair jobs on a level whose depth 1 is the
+ *           frequency-space M2L; 2 or 3 (register-ring depth) for
  *           the mixed forms, 2 only for "mixed3"; 4 selects the DMA-staged
  *           kernel (any mixed form; for "mixedh" at most 320 operator blocks
  *           per split-K part; 5 and 6 its 64 x 48 wave-tile and four-stage

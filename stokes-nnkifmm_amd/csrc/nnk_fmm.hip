@@ -2086,9 +2086,9 @@ void Fmm::launch_config(int level, int *split, int *depth) const {
       *depth = P.m2l_pair_on ? 10 + P.mx_pair_depth : P.mx_depth;
     }
   } else if (P.n_down) {
-    const bool one = P.m2l_spec_on || P.m2l_pair_on;
-    *split = one ? 1 : P.m2l_split;
-    *depth = one ? 1 : 0;
+    *split = P.m2l_spec_on || P.m2l_pair_on ? 1 : P.m2l_split;
+    // 1: what the planner chose over class tiles; 2: pair jobs of a level where that is the frequency-space M2L
+    *depth = P.m2l_spec_on ? 1 : P.m2l_pair_on ? (P.m2l_spec ? 2 : 1) : 0;
   }
 }
 
@@ -2113,7 +2113,11 @@ void Fmm::set_launch_config(int level, int split, int depth) {
     launches_changed();
     return;
   }
-  if (P.m2l_spec && depth == 0 && !P.m2l_dense) {
+  if (depth == 2 && !mixed) {
+    if (!P.m2l_spec) throw Error(NNK_EARG, "launch config: depth 2 is for levels in frequency space");
+    if (split != 1) throw Error(NNK_EARG, "launch config: the per-offset M2L takes split 1");
+  }
+  if (P.m2l_spec && (depth == 0 || depth == 2) && !P.m2l_dense) {
     launches_changed();   // the part and pair buffers may move, also where the split is refused below
     plan_m2l_dense(level);
   }
@@ -2122,15 +2126,16 @@ void Fmm::set_launch_config(int level, int split, int depth) {
   if (split > 1 && ((size_t)split * per_split > part_elems_ || !(mixed ? P.mx_slot.p : P.m2l_slot.p)))
     throw Error(NNK_EARG, "launch config: split-K factor out of range");
   if (!mixed) {
-    if (depth == 1) {
+    if (depth == 1 || depth == 2) {
       if (!P.m2l_npairs) throw Error(NNK_EARG, "launch config: no per-offset M2L plan at this level");
       if (split != 1) throw Error(NNK_EARG, "launch config: the per-offset M2L takes split 1");
       P.m2l_pair_on = true;
+      P.m2l_spec_on = false;
     } else if (depth == 0) {
       P.m2l_split = split;
       P.m2l_pair_on = P.m2l_spec_on = false;
     } else {
-      throw Error(NNK_EARG, "launch config: the FP64 forms take depth 0 or 1");
+      throw Error(NNK_EARG, "launch config: the FP64 forms take depths 0 to 2");
     }
   } else if ((depth >= 12 && depth <= 14) || depth == 17) {  // per-offset pair jobs, kernel depth 2-4, 7
     if (!P.m2l_npairs) throw Error(NNK_EARG, "launch config: no per-offset M2L plan at this level");

@@ -93,3 +93,51 @@ def test_mobility_graph_follows_the_configuration(oracle, nnk):
                     assert _set(nnk, h, levels, 1, 0) == 0
         same()
         same()
+
+
+def test_depths_name_one_launch(oracle, nnk):
+    """On a level in frequency space depth 1 is that, 2 its pair jobs, 0 class
+    tiles; what is reported brings the same bits back.  Where there is no
+    frequency-space M2L, 1 is the pair jobs and 2 is refused."""
+    rng = np.random.default_rng(5)
+    p = blobs(rng)
+    t = nnk.OcTree(p, p, "nodeCapacity", 24)
+    q = rng.standard_normal(p.shape)
+    f = nnk.KIFMM(t, [2e-3, 1.0], "coronaRes", 6)
+    h = f._handle().h
+    s0, d0 = _config(nnk, h)
+    levels = np.flatnonzero(s0)
+    assert (s0[levels] == 1).all() and (d0[levels] == 1).all()
+    u = f.computeVel(q)
+    assert _set(nnk, h, levels, 1, 0) == 0
+    tiles = f.computeVel(q)
+    sparse = [lv for lv in levels if _set(nnk, h, [lv], 1, 2) == 0]
+    print(f"[config] pair jobs on levels {sparse} of {levels.tolist()}", flush=True)
+    assert sparse and all(_set(nnk, h, [lv], 2, 2) != 0 for lv in levels)
+    s, d = _config(nnk, h)
+    assert (s[sparse] == 1).all() and (d[sparse] == 2).all()
+    pairs = f.computeVel(q)
+    assert _set(nnk, h, levels, 1, 1) == 0
+    np.testing.assert_array_equal(f.computeVel(q), u)
+    assert _set(nnk, h, levels, s[levels], d[levels]) == 0     # as reported
+    np.testing.assert_array_equal(f.computeVel(q), pairs)
+    uo = oracle.Tree(p, p, nodeCapacity=24).matvec(q, 2e-3, 1.0, 6, 1)
+    for v in (u, tiles, pairs):
+        assert np.linalg.norm(v - uo) <= 1e-10 * np.linalg.norm(uo)
+
+    # an autotuned mix of tiles and pair jobs replays from its report
+    f = nnk.KIFMM(t, [2e-3, 1.0], "coronaRes", 6, "autotune", 1)
+    h = f._handle().h
+    assert _set(nnk, h, levels, 1, 0) == 0
+    u = f.computeVel(q)
+    s, d = _config(nnk, h)
+    assert (d != 1).all()
+    assert _set(nnk, h, levels, 1, 1) == 0
+    assert _set(nnk, h, levels, s[levels], d[levels]) == 0
+    np.testing.assert_array_equal(f.computeVel(q), u)
+
+    f = nnk.KIFMM(t, [2e-3, 1.0], "coronaRes", 6, "coronaShells", 2)
+    h = f._handle().h
+    levels = np.flatnonzero(_config(nnk, h)[0])
+    assert all(_set(nnk, h, [lv], 1, 2) != 0 for lv in levels)
+    assert any(_set(nnk, h, [lv], 1, 1) == 0 for lv in levels)
