@@ -434,14 +434,11 @@ struct LeafArgs {
   int tc;           // targets per workgroup and pass (<= T); blockIdx.y picks the chunk
   double *out;      // ntgt x 3
   // leaves with long source lists are shared by several workgroups (null:
-  // none): items[blockIdx.x] is (leaf, part, parts, first row of its sums)
+  // none): items[blockIdx.x] is (leaf, part, parts, first row of its sums);
+  // the FP64 form's is (leaf, part + parts << 16, block of 32 targets, first row)
   const int4 *items;
   double *part;     // sums of part p: rows first + p * targets ..
 };
-__device__ __forceinline__ int4 leaf_item(const LeafArgs &a) {
-  if (a.items) return a.items[blockIdx.x];
-  return int4{a.leaves[blockIdx.x], 0, 1, 0};
-}
 
 // velocities of the shared leaves (list[blockIdx.x]: part 0's item): the sums
 // of their parts, in order
@@ -607,7 +604,8 @@ __global__ __launch_bounds__(T) void k_leaf(LeafArgs a) {
 }
 
 // The FP64 form of the leaf kernel: a workgroup takes up to 32 targets of a
-// leaf as 1, 2 or 4 blocks of at most 8 (as even as possible); its four
+// leaf (its item names them: a grid of items x the largest leaf's blocks would
+// be mostly empty where one leaf is crowded) as 1, 2 or 4 blocks of at most 8 (as even as possible); its four
 // wavefronts are blocks x source shares.  The sources are one list: the
 // points of the leaf's down surface and of its W nodes' up surfaces (with
 // their densities), then the U-list sources.
@@ -669,16 +667,16 @@ __global__ __launch_bounds__(256) void k_leaf64(LeafArgs a, const double *__rest
   __shared__ int pre[kLeafMaxU + 1];
   __shared__ SrcBatch buf;
   __shared__ double red[4][24];
-  const int4 it = leaf_item(a);
-  const int n = it.x, tid = threadIdx.x;
-  const int tb = a.tgt_ptr[n], nt = a.tgt_ptr[n + 1] - tb, t0 = 32 * (int)blockIdx.y;
+  const int4 it = a.items ? a.items[blockIdx.x] : int4{a.leaves[blockIdx.x], 1 << 16, 0, 0};
+  const int n = it.x, part = it.y & 0xffff, parts = it.y >> 16, tid = threadIdx.x;
+  const int tb = a.tgt_ptr[n], nt = a.tgt_ptr[n + 1] - tb, t0 = 32 * it.z;
   if (t0 >= nt) return;
   const int ntc = min(32, nt - t0);
   const int nblk = ntc <= 6 ? 1 : ntc <= 14 ? 2 : 4, per = (ntc + nblk - 1) / nblk;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), blk = w % nblk, sp = w / nblk, nsplit = 4 / nblk;
 #define NNK_LEAF_CASE(NT)                                                                                       \
   case NT:                                                                                                      \
-    leaf_block64<NT>(a, src_pos, src_q, tgt_pos, n, it.y, it.z, tb + t0, ntc, blk, sp, nsplit, pre, buf, red[w]); \
+    leaf_block64<NT>(a, src_pos, src_q, tgt_pos, n, part, parts, tb + t0, ntc, blk, sp, nsplit, pre, buf, red[w]); \
     break
   switch (per) {
     NNK_LEAF_CASE(1);
@@ -696,7 +694,7 @@ __global__ __launch_bounds__(256) void k_leaf64(LeafArgs a, const double *__rest
     const int t = tid / 3, d = tid - 3 * t, b = t / per;
     double v = 0.0;
     for (int s = 0; s < nsplit; s++) v += red[s * nblk + b][3 * (t - b * per) + d];
-    if (it.z > 1) a.part[3 * ((size_t)it.w + (size_t)it.y * nt + t0 + t) + d] = v;
+    if (parts > 1) a.part[3 * ((size_t)it.w + (size_t)part * nt + t0 + t) + d] = v;
     else a.out[3 * (size_t)a.tgt_out[tb + t0 + t] + d] = a.c * v;
   }
 }
@@ -1966,9 +1964,9 @@ void Fmm::launch_surf(const int32_t *nodes, int n, const int64_t *lptr, const in
 // the work items of a launch whose workgroups walk lists of very different
 // lengths: item (n, part, parts, first) takes one of the parts of n; lists of
 // up to two parts stay whole.  rows(n): rows of sums per part.  False: nothing
-// is shared.
+// is shared (all_items, if asked for, then holds the nodes, each whole).
 bool WorkParts::plan(const std::vector<int32_t> &nodes, const std::function<int64_t(int)> &work, int64_t per,
-                     const std::function<int(int)> &rows, int64_t row_bytes) {
+                     const std::function<int(int)> &rows, int64_t row_bytes, std::vector<int4> *all_items) {
   std::vector<int4> shares, rest, list;
   int64_t first = 0;
   for (int n : nodes) {
@@ -1982,13 +1980,20 @@ bool WorkParts::plan(const std::vector<int32_t> &nodes, const std::function<int6
     for (int p = 0; p < parts; p++) shares.push_back(int4{n, p, parts, (int)first});
     first += (int64_t)parts * rows(n);
   }
-  if (list.empty() || first > (1 << 28) || first * row_bytes > ((int64_t)1 << 30)) return false;
+  if (list.empty() || first > (1 << 28) || first * row_bytes > ((int64_t)1 << 30)) {
+    if (all_items) {
+      all_items->clear();
+      for (int n : nodes) all_items->push_back(int4{n, 0, 1, 0});
+    }
+    return false;
+  }
   shares.insert(shares.end(), rest.begin(), rest.end());
   nitems = (int)shares.size();
   nshared = (int)list.size();
   items.upload(shares);
   shared.upload(list);
   part.alloc((size_t)(first * row_bytes));
+  if (all_items) *all_items = shares;
   return true;
 }
 
@@ -2008,9 +2013,36 @@ void Fmm::plan_leaf_parts(const std::vector<int32_t> &leaves, const std::vector<
   int64_t total = 0;
   for (int n : leaves) total += nsrc[n] * blocks(n);
   const int64_t per = std::max<int64_t>(2048, total / (8 * (int64_t)ncu_));
+  std::vector<int4> items;
   leaf_parts_.plan(
       leaves, [&](int n) { return nsrc[n] * (fp32_math() ? blocks(n) : 1); }, per,
-      [&](int n) { return tgt_ptr[n + 1] - tgt_ptr[n]; }, 3 * sizeof(double));
+      [&](int n) { return tgt_ptr[n + 1] - tgt_ptr[n]; }, 3 * sizeof(double), &items);
+  if (fp32_math()) return;
+  // k_leaf64's items, by blocks of 32 targets; not needed where every leaf is
+  // one block and whole.  First every leaf's first block, then the second ones:
+  // the short last blocks fill the end of the launch (leaf by leaf, 2^20 points,
+  // 32 a leaf, 10.03 -> 10.13 ms a matvec)
+  auto split = [&](const std::vector<int4> &in, DBuf &list, int &count) {
+    std::vector<int4> out, left = in, more;
+    for (int b = 0; !left.empty(); b++, left.swap(more)) {
+      more.clear();
+      for (const int4 &it : left) {
+        out.push_back(int4{it.x, it.y + (it.z << 16), b, it.w});
+        if (b + 1 < blocks(it.x)) more.push_back(it);
+      }
+    }
+    if (out.size() > (size_t)INT32_MAX) throw Error(NNK_EARG, "leaf kernel: too many targets");
+    count = (int)out.size();
+    list.upload(out);
+  };
+  leaf_blocks_ = DBuf();
+  own_blocks_ = DBuf();
+  if (max_leaf_tgt_ > 32) {   // the leaf's own sources only: nothing is shared
+    std::vector<int4> whole;
+    for (int n : leaves) whole.push_back(int4{n, 0, 1, 0});
+    split(whole, own_blocks_, n_own_blocks_);
+  }
+  if (max_leaf_tgt_ > 32 || leaf_parts_.nshared) split(items, leaf_blocks_, n_leaf_blocks_);
 }
 
 void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
@@ -2056,8 +2088,10 @@ void Fmm::launch_leaf(int far, double *d_u, hipStream_t s) {
     else if (T == 512) shared ? go(k_leaf<512, true>, 512) : go(k_leaf<512, false>, 512);
     else shared ? go(k_leaf<256, true>, 256) : go(k_leaf<256, false>, 256);
   } else {
-    hipLaunchKernelGGL(k_leaf64, dim3((unsigned)nwg, (unsigned)std::max(1, (max_leaf_tgt_ + 31) / 32)), dim3(256), 0, s,
-                       a, a.src_pos, a.src_q, a.tgt_pos);
+    const DBuf &list = far ? leaf_blocks_ : own_blocks_;
+    a.items = list.as<int4>();
+    const int wgs = !a.items ? n_tleaves_ : far ? n_leaf_blocks_ : n_own_blocks_;
+    hipLaunchKernelGGL(k_leaf64, dim3((unsigned)wgs), dim3(256), 0, s, a, a.src_pos, a.src_q, a.tgt_pos);
   }
   if (shared)
     hipLaunchKernelGGL(k_leaf_parts, dim3((unsigned)leaf_parts_.nshared), dim3(256), 0, s, a, leaf_parts_.shared.as<int4>());

@@ -114,7 +114,7 @@ struct WorkParts {
   DBuf items, shared, part;
   int nitems = 0, nshared = 0;
   bool plan(const std::vector<int32_t> &nodes, const std::function<int64_t(int)> &work, int64_t per,
-            const std::function<int(int)> &rows, int64_t row_bytes);
+            const std::function<int(int)> &rows, int64_t row_bytes, std::vector<int4> *all_items = nullptr);
 };
 
 struct GemmBatch {
@@ -409,6 +409,8 @@ class Fmm {
   std::vector<int32_t> src_ptr_h_;  // host copy of src_ptr_ (launch order by work)
   int n_pleaves_ = 0, n_tleaves_ = 0;
   WorkParts leaf_parts_, x_parts_;   // the leaf kernel's leaves, the FP64 P2L's nodes
+  DBuf leaf_blocks_, own_blocks_;    // k_leaf64's items (none: a workgroup per leaf): all sources, the leaf's own
+  int n_leaf_blocks_ = 0, n_own_blocks_ = 0;
   int max_leaf_tgt_ = 0, ncu_ = 256;  // most targets in a leaf; compute units of the device
   // work buffers
   DBuf chk_, uppot_, downpot_, tmp_;
