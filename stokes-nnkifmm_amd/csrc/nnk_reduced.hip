@@ -543,11 +543,12 @@ __global__ __launch_bounds__(256, 2) void k_red_inv(RedArgs a, const int64_t *__
 }
 
 // x = A^-1 v for each leaf with the column-major inverse
-// (Inv[j n3 + i] = (A^-1)_ij): a workgroup takes 64 rows of a leaf (lane =
-// row, so a column's rows are read coalesced), its wavefronts an eighth of the
-// columns each, the sums added in wavefront order.  One pass over the
-// inverses, bound by their bytes; a thread walking a whole row alone had one
-// load in flight per 500 ns.
+// (Inv[j n3 + i] = (A^-1)_ij), one pass over the inverses, in three shapes
+// (reduced_solve has the lines between them).
+// Few large blocks: a workgroup takes 64 rows of a leaf (lane = row, so a
+// column's rows are read coalesced), its wavefronts an eighth of the columns
+// each, the sums added in wavefront order.  A thread walking a whole row alone
+// has one load in flight per 500 ns.
 // Measured for ten squirmers in a box (blocks up to 832 rows): 71 -> 20 us.
 constexpr int kRedApplyWaves = 8;
 __global__ __launch_bounds__(64 * kRedApplyWaves) void k_red_apply(RedArgs a, const double *__restrict__ v,
@@ -584,6 +585,63 @@ __global__ __launch_bounds__(64 * kRedApplyWaves) void k_red_apply(RedArgs a, co
 #pragma unroll
     for (int k = 0; k < kRedApplyWaves; k++) t += part[k][lane];
     x[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3] = t;
+  }
+}
+
+// Many blocks, bound by their bytes: a thread per row, its columns in order;
+// long runs of rows, 2 KB of a column at a time, read memory best.
+constexpr int kRedRowThreads = 256;
+__global__ __launch_bounds__(kRedRowThreads) void k_red_apply_row(RedArgs a, const double *__restrict__ v,
+                                                                  double *__restrict__ x) {
+  extern __shared__ double b[];
+  const int li = blockIdx.x;
+  const int n = a.leaves[li];
+  const int tb = a.tgt_ptr[n], n3 = 3 * (a.tgt_ptr[n + 1] - tb);
+  const int i0 = blockIdx.y * kRedRowThreads;
+  if (i0 >= n3) return;  // the whole workgroup
+  const double *Inv = a.blk + a.off[li];
+  for (int i = threadIdx.x; i < n3; i += kRedRowThreads) b[i] = v[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3];
+  __syncthreads();
+  const int i = i0 + threadIdx.x;
+  if (i < n3) {
+    double acc = 0.0;
+    for (int j = 0; j < n3; j++) acc += Inv[(size_t)j * n3 + i] * b[j];
+    x[3 * (size_t)a.tgt_out[tb + i / 3] + i % 3] = acc;
+  }
+}
+
+// Small blocks: a leaf of at most T rows per workgroup; T / n3 threads share a
+// row's columns (rows fastest), their sums added in order.
+template <int T>
+__global__ __launch_bounds__(T) void k_red_apply_leaf(RedArgs a, const double *__restrict__ v, double *__restrict__ x) {
+  __shared__ double b[T], part[T];
+  const int li = blockIdx.x, tid = threadIdx.x;
+  const int n = a.leaves[li];
+  const int tb = a.tgt_ptr[n], n3 = 3 * (a.tgt_ptr[n + 1] - tb);
+  const double *Inv = a.blk + a.off[li];
+  if (tid < n3) b[tid] = v[3 * (size_t)a.tgt_out[tb + tid / 3] + tid % 3];
+  __syncthreads();
+  const int ns = min(T / n3, 8), sh = tid / n3, i = tid - sh * n3;
+  double acc[2] = {0, 0};
+  if (sh < ns) {
+    const int j1 = n3 * (sh + 1) / ns;
+    const double *col = Inv + i;
+    int j = n3 * sh / ns;
+    for (; j + 8 <= j1; j += 8) {
+      double t[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) t[k] = col[(size_t)(j + k) * n3];
+#pragma unroll
+      for (int k = 0; k < 8; k++) acc[k & 1] += t[k] * b[j + k];
+    }
+    for (; j < j1; j++) acc[0] += col[(size_t)j * n3] * b[j];
+  }
+  part[tid] = acc[0] + acc[1];
+  __syncthreads();
+  if (tid < n3) {
+    double t = part[tid];
+    for (int k = 1; k < ns; k++) t += part[k * n3 + tid];
+    x[3 * (size_t)a.tgt_out[tb + tid / 3] + tid % 3] = t;
   }
 }
 
@@ -692,8 +750,25 @@ void Fmm::reduced_solve(const double *d_v, double *d_f, hipStream_t s) {
   if (!red_ready_) reduced_factor();
   if (!n_tleaves_) return;
   RedArgs a = red_args();
-  hipLaunchKernelGGL(k_red_apply, dim3(n_tleaves_, (red_maxn_ + 63) / 64), dim3(64 * kRedApplyWaves),
-                     sizeof(double) * red_maxn_, s, a, d_v, d_f);
+  auto go = [&](auto kern, int rows, int threads, size_t lds) {
+    hipLaunchKernelGGL(kern, dim3(n_tleaves_, (red_maxn_ + rows - 1) / rows), dim3(threads), lds, s, a, d_v, d_f);
+  };
+  // Measured by number of leaves x rows per leaf (eight wavefronts per 64
+  // rows; a thread per row; a leaf per workgroup), us: 32,768 x 30 113, 78, 74;
+  // 32,768 x 72 412, 297, 282; 4,096 x 120 96, 89, 87; 64 x 255 13.3, 18, 13.4;
+  // 512 x 234 (at most 312) 47, 39, 39; 4,096 x 220 (312) 385, 320, 319;
+  // 512 x 352 (432) 107, 100, 117; 512 x 495 186, 167, 180; 64 x 330 14, 31, 22;
+  // 1,807 x 166 (600) 186, 193; 512 x 586 (723) 283, 317; and by the inverses'
+  // bytes: 64 x 1,500 (1.2 GB) 199, 252; 256 x 1,020 (2.1 GB) 403, 367;
+  // 64 x 2,100 (2.3 GB) 400, 381; 512 x 1,500 (9.2 GB) 1,827, 1,585.
+  const size_t lds = sizeof(double) * red_maxn_;
+  const bool many = n_tleaves_ >= ncu_;
+  if (red_maxn_ <= 64) go(k_red_apply_leaf<128>, 64, 128, 0);
+  else if (red_maxn_ <= 128) go(k_red_apply_leaf<256>, 128, 256, 0);
+  else if (red_maxn_ <= 256 || (red_maxn_ <= 320 && many)) go(k_red_apply_leaf<512>, 320, 512, 0);
+  else if ((red_maxn_ <= 512 && many) || red_blk_.bytes >= ((size_t)7 << 28))
+    go(k_red_apply_row, kRedRowThreads, kRedRowThreads, lds);
+  else go(k_red_apply, 64, 64 * kRedApplyWaves, lds);
   NNK_HIP(hipGetLastError());
 }
 
