@@ -652,12 +652,14 @@ void Fmm::reduced_factor() {
   std::vector<int32_t> tl(n_tleaves_), tp(T.count + 2);
   NNK_HIP(hipMemcpy(tl.data(), tleaves_.p, sizeof(int32_t) * n_tleaves_, hipMemcpyDeviceToHost));
   NNK_HIP(hipMemcpy(tp.data(), tgt_ptr_.p, sizeof(int32_t) * (T.count + 2), hipMemcpyDeviceToHost));
-  std::vector<int64_t> off(n_tleaves_ + 1, 0), poff(n_tleaves_ + 1, 0);
+  // first entry of each leaf's block, its rows, and its diagonal tiles' inverses
+  std::vector<int64_t> off(n_tleaves_ + 1, 0), poff(n_tleaves_ + 1, 0), doff(n_tleaves_ + 1, 0);
   red_maxn_ = 0;
   for (int i = 0; i < n_tleaves_; i++) {
     int64_t n3 = 3 * (tp[tl[i] + 1] - tp[tl[i]]);
     off[i + 1] = off[i] + n3 * n3;
     poff[i + 1] = poff[i] + n3;
+    doff[i + 1] = doff[i] + (n3 + kInvB - 1) / kInvB * 2 * kInvB * kInvB;
     red_maxn_ = std::max<int>(red_maxn_, (int)n3);
   }
   if ((size_t)red_maxn_ * sizeof(double) > 64 * 1024)
@@ -670,10 +672,15 @@ void Fmm::reduced_factor() {
       for (int k = tp[tl[i]]; k < tp[tl[i] + 1]; k++) o2l[to[k]] = k - tp[tl[i]];
   }
   red_off_.upload(off);
-  DBuf dpoff;
-  dpoff.upload(poff);
+  DBuf dpoff;   // poff, then doff
+  const int64_t *const ddoff = [&] {
+    std::vector<int64_t> both = poff;
+    both.insert(both.end(), doff.begin(), doff.end());
+    dpoff.upload(both);
+    return dpoff.as<int64_t>() + poff.size();
+  }();
   red_ord2loc_.upload(o2l);
-  red_blk_.alloc(sizeof(double) * std::max<int64_t>(off.back(), 1));
+  red_blk_.alloc(sizeof(double) * (off.back() + doff.back()));   // the tiles' inverses behind the blocks
   red_piv_.alloc(sizeof(int32_t) * std::max<int64_t>(poff.back(), 1));
   red_perm_.alloc(sizeof(int32_t) * std::max<int64_t>(poff.back(), 1));
   red_poff_ = std::move(dpoff);
@@ -702,17 +709,13 @@ void Fmm::reduced_factor() {
     NNK_HIP(hipGetLastError());
     // the blocks' inverses replace their factors: each solve is then one
     // pass over them at HBM bandwidth instead of a chain of substitutions
-    std::vector<int64_t> doff(n_tleaves_ + 1, 0);
-    for (int i = 0; i < n_tleaves_; i++)
-      doff[i + 1] = doff[i] + (poff[i + 1] - poff[i] + kInvB - 1) / kInvB * 2 * kInvB * kInvB;
-    DBuf W, D, ddoff;
-    ddoff.upload(doff);
-    D.alloc(sizeof(double) * std::max<int64_t>(doff.back(), 1));
+    DBuf W;
+    double *D = red_blk_.as<double>() + off.back();
     W.alloc(sizeof(double) * std::max<int64_t>(off.back(), 1));
     hipLaunchKernelGGL(k_red_diag, dim3(n_tleaves_, (red_maxn_ + kInvB - 1) / kInvB), dim3(64), 0, 0, a,
-                       ddoff.as<int64_t>(), D.as<double>());
-    hipLaunchKernelGGL(k_red_inv, dim3(n_tleaves_, (red_maxn_ + 63) / 64), dim3(256), 0, 0, a, ddoff.as<int64_t>(),
-                       D.as<double>(), W.as<double>());
+                       ddoff, D);
+    hipLaunchKernelGGL(k_red_inv, dim3(n_tleaves_, (red_maxn_ + 63) / 64), dim3(256), 0, 0, a, ddoff, D,
+                       W.as<double>());
     NNK_HIP(hipGetLastError());
     NNK_HIP(hipDeviceSynchronize());
     red_blk_ = std::move(W);
