@@ -94,8 +94,8 @@ __device__ __forceinline__ void put_record(double *rec, bool f32, int64_t sb, in
   }
 }
 
-// g[q] = sum_e NN(q, col e) f(col e)    (the quadrature strengths, 3 each)
-// and, unless null, the sources' records
+// g[q] = sum_e NN(q, col e) f(col e)    (the quadrature strengths, 3 each), or,
+// unless null, into the sources' records
 __global__ void k_bgather(int64_t qtot, const int64_t *__restrict__ ptr, const int32_t *__restrict__ col,
                           const double *__restrict__ val, const double *__restrict__ x,
                           const int64_t *__restrict__ xbase, const int64_t *__restrict__ xstride,
@@ -113,13 +113,14 @@ __global__ void k_bgather(int64_t qtot, const int64_t *__restrict__ ptr, const i
     gy += v * x[b + st];
     gz += v * x[b + 2 * st];
   }
-  g[3 * q] = gx;
-  g[3 * q + 1] = gy;
-  g[3 * q + 2] = gz;
   if (rec) {
     const int p = fpid[q];
     const int64_t sb = foff[p];
     put_record(rec, f32, sb, p, foff[p + 1] - sb, q - sb, fine + 3 * q, gx, gy, gz);
+  } else {
+    g[3 * q] = gx;
+    g[3 * q + 1] = gy;
+    g[3 * q + 2] = gz;
   }
 }
 
@@ -269,6 +270,108 @@ __global__ __launch_bounds__(64 * kSumWaves<F32>) void k_bsum(const BatchItem *_
   P[((size_t)it.slot * 3 + v) * kTile + lane] = u;
 }
 
+// The same sums where a launch has tiles enough to fill the chip by themselves:
+// a tile's four runs on the four wavefronts of a workgroup, each adding its
+// run's terms as it evaluates them, from records staged 64 at a time in its own
+// LDS; the runs' sums are added in order there, without a pass through memory.
+// The terms and the order of the additions are k_bsum's, to the bit.  Bound by
+// the terms (FP64 transpose of 256 problems, 1.68e10 pairs, 0.93e12 pairs/s).
+template <bool F32>
+__global__ __launch_bounds__(64 * kRuns) void k_btile(const int2 *__restrict__ tiles, const int64_t *__restrict__ toff,
+                                                      const int64_t *__restrict__ soff, const double *__restrict__ tgt,
+                                                      const double *__restrict__ rec, const double *__restrict__ eps,
+                                                      const int32_t *__restrict__ active, double c,
+                                                      double *__restrict__ out) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  constexpr int C = 64, G = F32 ? 4 : 2;   // records of a chunk, of a step
+  __shared__ __attribute__((aligned(16))) double st[kRuns][6 * C];
+  __shared__ double red[kRuns][3][64];
+  const int2 it = tiles[blockIdx.x];
+  if (!active[it.x]) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int64_t i = toff[it.x] + (int64_t)kTile * it.y + lane, end = toff[it.x + 1];
+  const double *p = tgt + 3 * min(i, end - 1);
+  const double tx = p[0], ty = p[1], tz = p[2], e2 = eps[it.x] * eps[it.x];
+  const int64_t sb = soff[it.x], ns = soff[it.x + 1] - sb;
+  const int n = (int)((ns - w + kRuns - 1) / kRuns);
+  const d2 *__restrict__ r = reinterpret_cast<const d2 *>(rec + 6 * rec_run(sb, it.x, w, ns));
+  double ux = 0.0, uy = 0.0, uz = 0.0;
+  d2 v[3];
+  auto fetch = [&](int j) {   // past the end: the last one again, not used
+#pragma unroll
+    for (int k = 0; k < 3; k++) v[k] = r[3 * (size_t)min(j, n - 1) + k];
+  };
+  if (n > 0) fetch(lane);
+  for (int j0 = 0; j0 < n; j0 += C) {
+    d2 *own = reinterpret_cast<d2 *>(st[w]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the chunk before has been read
+#pragma unroll
+    for (int k = 0; k < 3; k++) own[3 * lane + k] = v[k];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (j0 + C < n) fetch(j0 + C + lane);
+    const int cnt = min(C, n - j0);
+    const double *q = st[w];
+    int k = 0;
+    for (; k + G <= cnt; k += G, q += 6 * G) {
+      double s[6 * G];
+#pragma unroll
+      for (int m = 0; m < 6 * G; m++) s[m] = q[m];
+      if constexpr (F32) {
+        float g[3];
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+          const float4 f = rec_strength(s + 6 * m + 3);
+          float a[3];
+          stokeslet_term_f32_fixed(tx, ty, tz, s[6 * m], s[6 * m + 1], s[6 * m + 2], f.x, f.y, f.z, (float)e2, a[0],
+                                   a[1], a[2]);
+          for (int d = 0; d < 3; d++) g[d] = m == 0 ? a[d] : g[d] + a[d];
+        }
+        ux += (double)g[0];
+        uy += (double)g[1];
+        uz += (double)g[2];
+      } else {
+        double ax[G], ay[G], az[G];
+        stokeslet_terms_fixed<G>(tx, ty, tz, s, e2, ax, ay, az);
+#pragma unroll
+        for (int m = 0; m < G; m++) {
+          ux += ax[m];
+          uy += ay[m];
+          uz += az[m];
+        }
+      }
+    }
+    for (; k < cnt; k++, q += 6) {   // the run's last one (FP64) or up to three
+      if constexpr (F32) {
+        const float4 f = rec_strength(q + 3);
+        float a[3];
+        stokeslet_term_f32_fixed(tx, ty, tz, q[0], q[1], q[2], f.x, f.y, f.z, (float)e2, a[0], a[1], a[2]);
+        ux += (double)a[0];
+        uy += (double)a[1];
+        uz += (double)a[2];
+      } else {
+        double s[6], ax[1], ay[1], az[1];
+#pragma unroll
+        for (int m = 0; m < 6; m++) s[m] = q[m];
+        stokeslet_terms_fixed<1>(tx, ty, tz, s, e2, ax, ay, az);
+        ux += ax[0];
+        uy += ay[0];
+        uz += az[0];
+      }
+    }
+  }
+  red[w][0][lane] = ux;
+  red[w][1][lane] = uy;
+  red[w][2][lane] = uz;
+  __syncthreads();
+  if (w < 3 && i < end) {
+    double u = red[0][w][lane];
+#pragma unroll
+    for (int k = 1; k < kRuns; k++) u += red[k][w][lane];
+    out[3 * i + w] = c * u;
+  }
+}
+
 // a point's pair sum: its tile's runs in order (slot0: the problem's first)
 __device__ __forceinline__ void run_sum(const double *__restrict__ P, int32_t slot0, int64_t loc, double u[3]) {
   const double *q = P + ((size_t)slot0 + (size_t)(loc / kTile) * kRuns) * (3 * kTile) + loc % kTile;
@@ -280,7 +383,8 @@ __device__ __forceinline__ void run_sum(const double *__restrict__ P, int32_t sl
   }
 }
 
-// forward: u_i = c sum_q S(x_i - y_q) g_q, then + BT (U; W) on body points
+// forward: u_i = c sum_q S(x_i - y_q) g_q, then + BT (U; W) on body points.
+// slot0 null: P holds k_btile's sums of the points, times c already
 __global__ void k_bfinish(int64_t ntot, const int32_t *__restrict__ ppid, const int32_t *__restrict__ slot0,
                           const double *__restrict__ P, const int64_t *__restrict__ poff,
                           const int64_t *__restrict__ voff, const int32_t *__restrict__ nsw,
@@ -293,8 +397,12 @@ __global__ void k_bfinish(int64_t ntot, const int32_t *__restrict__ ppid, const 
   if (!active[p]) return;
   const int64_t loc = i - poff[p];
   double u[3];
-  run_sum(P, slot0[p], loc, u);
-  for (int d = 0; d < 3; d++) u[d] *= c;
+  if (slot0) {
+    run_sum(P, slot0[p], loc, u);
+    for (int d = 0; d < 3; d++) u[d] *= c;
+  } else {
+    for (int d = 0; d < 3; d++) u[d] = P[3 * i + d];
+  }
   const Slots S = slots(p, poff, voff, nsw);
   const int b = pbody[i];
   if (b >= 0) {
@@ -605,6 +713,18 @@ __global__ void k_bscale(int64_t n, const int32_t *__restrict__ pid, const doubl
 
 // ---------------------------------------------------------------------------
 
+// Launches of so many tiles take k_btile, and transposes of at most kBatchRunT
+// force points a problem (short runs gain nothing from more wavefronts; two
+// launches less).  k_bsum against k_btile, us an
+// application, FP64 and FP32 math:
+// transpose: 24 tiles, at most 60 points, 56, 54 and 56, 54; 236 tiles, 600
+// points, 65, 62 and 63, 60; 542 tiles, 2,166 points, 161, 169 and 120, 132; 730
+// tiles 83, 72 and 79, 68; 3,706 365, 328 and 277, 231; 97,930 20,818, 18,111
+// and 12,621, 11,224.  Forward (long runs, of uneven lengths): 2,414 tiles
+// 8,011, 8,197 and 4,635, 5,096; 4,920 2,799, 2,426 and 1,976, 1,809; 6,236
+// 20,844, 19,330 and 11,978, 11,805.
+constexpr int kBatchTiles = 4096, kBatchTilesT = 640, kBatchRunT = 1024;
+
 Batch::Batch(int nprob, const int64_t *pt_off, const double *pts, const int64_t *fine_off, const double *fine,
              const int64_t *nn_ptr, const int32_t *nn_col, const double *nn_val, const double *w,
              const double *pm, const double *rot, const int32_t *pt_body, const int64_t *body_off,
@@ -718,17 +838,24 @@ Batch::Batch(int nprob, const int64_t *pt_off, const double *pts, const int64_t 
     return sorted;
   };
   auto it_f = make_items(false), it_t = make_items(true);
-  std::vector<BatchItem> sum_f, sum_t;
-  std::vector<int32_t> slot_f, slot_t;
+  // which sums go a tile per workgroup, and the run items of the others
+  int64_t most = 0;
+  for (int p = 0; p < nprob; p++) most = std::max(most, hpoff_[p + 1] - hpoff_[p]);
+  tiles_ = (int)it_f.size() >= kBatchTiles;
+  tilesT_ = (int)it_t.size() >= kBatchTilesT || most <= kBatchRunT;
   hfoff_ = hfoff;
-  const int64_t slots = std::max(pair_items(false, sum_f, slot_f), pair_items(true, sum_t, slot_t));
-  nsums_ = (int)sum_f.size();
-  nsumsT_ = (int)sum_t.size();
-  sums_.upload(sum_f);
-  sumsT_.upload(sum_t);
-  slot0_.upload(slot_f);
-  slot0T_.upload(slot_t);
-  sumbuf_.alloc(sizeof(double) * 3 * kTile * (size_t)std::max<int64_t>(slots, 1));
+  int64_t sums = tiles_ ? 3 * ntot_ : 0;
+  auto runs = [&](bool transpose, DBuf &list, int &count, DBuf &first) {
+    std::vector<BatchItem> items;
+    std::vector<int32_t> slot0;
+    sums = std::max(sums, 3 * kTile * pair_items(transpose, items, slot0));
+    count = (int)items.size();
+    list.upload(items);
+    first.upload(slot0);
+  };
+  if (!tiles_) runs(false, sums_, nsums_, slot0_);
+  if (!tilesT_) runs(true, sumsT_, nsumsT_, slot0T_);
+  sumbuf_.alloc(sizeof(double) * (size_t)std::max<int64_t>(sums, 1));
   std::vector<int32_t> fpid(qtot_);
   for (int p = 0; p < nprob; p++)
     for (int64_t q = hfoff[p]; q < hfoff[p + 1]; q++) fpid[q] = p;
@@ -800,16 +927,33 @@ void Batch::pair_sums(const DBuf &items, int n, bool transpose, hipStream_t s) {
   else launch(k_bsum<false>);
 }
 
+// c times the tiles' sums, three values a target
+void Batch::tile_sums(bool transpose, double c, double *out, hipStream_t s) {
+  const DBuf &items = transpose ? itemsT_ : items_;
+  const int n = transpose ? nitemsT_ : nitems_;
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * kRuns), 0, s, items.as<int2>(),
+                       (transpose ? foff_ : poff_).as<int64_t>(), (transpose ? poff_ : foff_).as<int64_t>(),
+                       (transpose ? fine_ : pts_).as<double>(), rec_.as<double>(), eps_.as<double>(),
+                       active_.as<int32_t>(), c, out);
+  };
+  if (f32_) launch(k_btile<true>);
+  else launch(k_btile<false>);
+}
+
 void Batch::op(const double *x, double *y, hipStream_t s) {
+  const double c = 1.0 / (8.0 * kPi * mu_);
   if (qtot_)
     hipLaunchKernelGGL(k_bgather, dim3(nblk(qtot_)), dim3(256), 0, s, qtot_, nnptr_.as<int64_t>(),
                        nncol_.as<int32_t>(), nnval_.as<double>(), x, xbase_.as<int64_t>(),
                        xstride_.as<int64_t>(), g_.as<double>(), rec_.as<double>(), f32_ != 0, fpid_.as<int32_t>(),
                        foff_.as<int64_t>(), fine_.as<double>());
-  pair_sums(sums_, nsums_, false, s);
-  hipLaunchKernelGGL(k_bfinish, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, pidf_.as<int32_t>(), slot0_.as<int32_t>(),
-                     sumbuf_.as<double>(), poff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(),
-                     rot_.as<double>(), pbody_.as<int32_t>(), active_.as<int32_t>(), 1.0 / (8.0 * kPi * mu_), x, y);
+  if (tiles_) tile_sums(false, c, sumbuf_.as<double>(), s);
+  else pair_sums(sums_, nsums_, false, s);
+  hipLaunchKernelGGL(k_bfinish, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, pidf_.as<int32_t>(),
+                     tiles_ ? nullptr : slot0_.as<int32_t>(), sumbuf_.as<double>(), poff_.as<int64_t>(),
+                     voff_.as<int64_t>(), nsw_.as<int32_t>(), rot_.as<double>(), pbody_.as<int32_t>(),
+                     active_.as<int32_t>(), c, x, y);
   if (nbody_)
     hipLaunchKernelGGL(k_bB, dim3(nbody_), dim3(256), 0, s, bprob_.as<int32_t>(), blocal_.as<int32_t>(),
                        bpt_.as<int64_t>(), poff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(),
@@ -818,14 +962,18 @@ void Batch::op(const double *x, double *y, hipStream_t s) {
 }
 
 void Batch::opT(const double *x, double *y, hipStream_t s) {
+  const double c = 1.0 / (8.0 * kPi * mu_);
   hipLaunchKernelGGL(k_brecordT, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, x, xbase_.as<int64_t>(),
                      xstride_.as<int64_t>(), rec_.as<double>(), f32_ != 0, pidf_.as<int32_t>(), poff_.as<int64_t>(),
                      pts_.as<double>());
-  pair_sums(sumsT_, nsumsT_, true, s);
-  if (qtot_)
+  if (tilesT_) {
+    if (nitemsT_) tile_sums(true, c, v_.as<double>(), s);
+  } else if (qtot_) {
+    pair_sums(sumsT_, nsumsT_, true, s);
     hipLaunchKernelGGL(k_bfinishT, dim3(nblk(qtot_)), dim3(256), 0, s, qtot_, fpid_.as<int32_t>(),
-                       slot0T_.as<int32_t>(), sumbuf_.as<double>(), foff_.as<int64_t>(), active_.as<int32_t>(),
-                       1.0 / (8.0 * kPi * mu_), v_.as<double>());
+                       slot0T_.as<int32_t>(), sumbuf_.as<double>(), foff_.as<int64_t>(), active_.as<int32_t>(), c,
+                       v_.as<double>());
+  }
   hipLaunchKernelGGL(k_bgatherT, dim3(nblk(ntot_)), dim3(256), 0, s, ntot_, pidf_.as<int32_t>(),
                      nntptr_.as<int64_t>(), nntrow_.as<int32_t>(), nntval_.as<double>(), v_.as<double>(),
                      poff_.as<int64_t>(), voff_.as<int64_t>(), nsw_.as<int32_t>(), w_.as<double>(), pm_.as<double>(),

@@ -77,6 +77,8 @@ class Batch {
   // points onto quadrature points)
   int64_t pair_items(bool transpose, std::vector<BatchItem> &items, std::vector<int32_t> &slot0) const;
   void pair_sums(const DBuf &items, int n, bool transpose, hipStream_t s);
+  void tile_sums(bool transpose, double c, double *out, hipStream_t s);
+  bool tiles_ = false, tilesT_ = false;   // the sums a tile per workgroup (k_btile)
   void segdots(int k, const double *V, const double *w, double *host_out, hipStream_t s);
 
   int np_ = 0, nbody_ = 0;
