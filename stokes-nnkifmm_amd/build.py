@@ -64,7 +64,7 @@ def build(verbose=False):
     # test-only companion library (GEMM / internal-array probes, host-only
     # planner checks; its source lives with the tests)
     stos = []
-    for name in ("nnk_selftest", "nnk_spectral_selftest", "nnk_gemm_selftest"):
+    for name in ("nnk_selftest", "nnk_spectral_selftest", "nnk_gemm_selftest", "nnk_shape_selftest"):
         st = os.path.join(os.path.dirname(HERE), "tests", "native", name + ".hip")
         stos.append(os.path.join(objdir, name + ".o"))
         _run([HIPCC, "-x", "hip"] + COMMON + DEVICE_FLAGS + ["-I" + CSRC, "-c", st, "-o", stos[-1]])

@@ -291,6 +291,9 @@ class Fmm {
   // (launches, buffer addresses): such a graph replays only while the count
   // it was captured at stands
   uint64_t generation() const { return gen_; }
+  // lists shared by several workgroups: the leaf kernel's, the FP64 P2L's
+  int shared_leaves() const { return leaf_parts_.nshared; }
+  int shared_x_lists() const { return x_parts_.nshared; }
   // threads per target leaf of the leaf kernel (L2T + P2P + M2T)
   int leaf_threads() const { return leaf_threads_; }
   // leaf-local product (reducedPass.m) on device pointers

@@ -474,13 +474,14 @@ double Mobility::dot(const double *a, const double *b, hipStream_t s) {
   return t;
 }
 
+size_t Mobility::cgs2_part(int m1) { return 2 * (size_t)m1 * kCgsSlices; }
+
 // w -= V[0..kk) c with c = V^T w, twice (classical Gram-Schmidt with one
 // reorthogonalisation), then y = w / ||w||; nothing waits on the host.  The
 // coefficients of the two passes land in hc[0..kk) and hc[m1..m1+kk), the
 // norm in hc[2 m1].  part holds two sets of m1 x kCgsSlices partials.
-void Mobility::cgs2(const double *V, int kk, double *w, double *y, double *hc, int m1, double *part,
+void Mobility::cgs2(int64_t n, const double *V, int kk, double *w, double *y, double *hc, int m1, double *part,
                     hipStream_t s) {
-  const int64_t n = n_;
   // slices of 128 entries or more, then as many as kCgsSlices: a workgroup of
   // a shorter slice waits longer for its sums than it works
   const int64_t S = std::max<int64_t>(128, ((n + kCgsSlices - 1) / kCgsSlices + 63) / 64 * 64);
@@ -512,7 +513,7 @@ GmresResult Mobility::gmres(const double *b, double *x, double tol, int maxit, b
   V.alloc(sizeof(double) * (size_t)(m + 1) * n);
   w.alloc(sizeof(double) * n);
   hdev.alloc(sizeof(double) * (m + 1));
-  part.alloc(sizeof(double) * 2 * (size_t)(m + 1) * kCgsSlices);
+  part.alloc(sizeof(double) * cgs2_part(m + 1));
   hc.alloc(sizeof(double) * (2 * (size_t)(m + 1) + 1));
   NNK_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, s));
   const double bnorm = std::sqrt(dot(b, b, s));
@@ -531,7 +532,7 @@ GmresResult Mobility::gmres(const double *b, double *x, double tol, int maxit, b
   bool done = false;
   for (k = 0; k < m && !done; k++) {
     op_any(Vp + (size_t)k * n, w.as<double>(), use_precon, s);
-    cgs2(Vp, k + 1, w.as<double>(), Vp + (size_t)(k + 1) * n, hc.as<double>(), m + 1, part.as<double>(), s);
+    cgs2(n, Vp, k + 1, w.as<double>(), Vp + (size_t)(k + 1) * n, hc.as<double>(), m + 1, part.as<double>(), s);
     read_column(hc.as<double>(), m + 1, k + 1, h, hh, s);
     const double hn = h[k + 1];
     for (int j = 0; j < k; j++) {  // previous rotations
@@ -622,7 +623,7 @@ GmresResult Mobility::fgmres(const double *b, double *x, double tol, int maxit, 
   Z.alloc(sizeof(double) * (size_t)m * n);
   w.alloc(sizeof(double) * n);
   hdev.alloc(sizeof(double) * (m + 1));
-  part.alloc(sizeof(double) * 2 * (size_t)(m + 1) * kCgsSlices);
+  part.alloc(sizeof(double) * cgs2_part(m + 1));
   hc.alloc(sizeof(double) * (2 * (size_t)(m + 1) + 1));
   GmresResult R{};
   NNK_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, s));
@@ -655,7 +656,7 @@ GmresResult Mobility::fgmres(const double *b, double *x, double tol, int maxit, 
     Fcur_ = nullptr;
     used += std::max(gi.iter, 1);
     apply(Zp + (size_t)k * n, w.as<double>(), s);  // FP64 operator
-    cgs2(Vp, k + 1, w.as<double>(), Vp + (size_t)(k + 1) * n, hc.as<double>(), m + 1, part.as<double>(), s);
+    cgs2(n, Vp, k + 1, w.as<double>(), Vp + (size_t)(k + 1) * n, hc.as<double>(), m + 1, part.as<double>(), s);
     read_column(hc.as<double>(), m + 1, k + 1, h, hh, s);
     const double hn = h[k + 1];
     for (int j = 0; j < k; j++) {

@@ -64,6 +64,12 @@ class Mobility {
   // replay the GMRES operator (A or A P) from HIP graphs, one per
   // (preconditioned, inner operator) combination, captured on first use
   void set_graph(bool on) { graph_ = on; }
+  // one step of the orthogonalisation: w against the kk vectors of V (n
+  // entries each), y = w / ||w||; hc holds 2 m1 + 1 values, part
+  // cgs2_part(m1), kk <= m1
+  static void cgs2(int64_t n, const double *V, int kk, double *w, double *y, double *hc, int m1, double *part,
+                   hipStream_t s);
+  static size_t cgs2_part(int m1);
 
  private:
   void op(const double *x, double *y, bool use_precon, hipStream_t s);
@@ -71,7 +77,6 @@ class Mobility {
   void kifmm(Fmm *Fm, const double *f, double *u, bool accumulate, hipStream_t s);
   void reduced(const double *v, double *f, hipStream_t s);
   double dot(const double *a, const double *b, hipStream_t s);
-  void cgs2(const double *V, int kk, double *w, double *y, double *hc, int m1, double *part, hipStream_t s);
   void read_column(const double *hc, int m1, int kk, std::vector<double> &h, std::vector<double> &hh,
                    hipStream_t s);
 
