@@ -370,8 +370,9 @@ int32_t nnk_batch_apply_device(nnk_batch *h, const double *d_x, double *d_y, voi
 /* on = 1: replay the batched operators from HIP graphs captured on first use. */
 int32_t nnk_batch_set_graph(nnk_batch *h, int32_t on);
 /* Accepted for callers that tuned the batched P2P at 1, 2 and 4 wavefronts:
- * its pair sums now have one launch shape (four runs of a tile's sources,
- * which is what nnk_batch_p2p_waves reports), so there is nothing to time. */
+ * its pair sums are always added in four runs of a tile's sources (which is
+ * what nnk_batch_p2p_waves reports), in launches chosen by the number of
+ * tiles with the same bits, so there is nothing to time. */
 int32_t nnk_batch_set_autotune(nnk_batch *h, int32_t on);
 int32_t nnk_batch_p2p_waves(const nnk_batch *h, int32_t *waves);
 /* Unrestarted GMRES from x = 0 on every problem at once, on A (transpose =

@@ -3,8 +3,8 @@ which runs one mobilityProblem per body: Mobility/mobilityProblem.m:24-72).
 
 BatchedMobility takes a list of Swimmers systems (any bodies, optional
 fixed boundary, nearest quadrature or none) with their eps, and solves all
-their mobility problems at once on the GPU (libnnkifmm nnk_batch_*): one
-persistent P2P launch per matvec over (problem, target tile) work items,
+their mobility problems at once on the GPU (libnnkifmm nnk_batch_*): a matvec
+is a few launches over the (problem, target tile) work items of all problems,
 lockstep GMRES, optional HIP-graph replay, the transpose operator and
 adjoint gradients with respect to node positions and eps.  Per problem the
 system is the reference's [S BT; B 0] with S the direct Stokeslet sum (what
@@ -90,7 +90,7 @@ class BatchedMobility:
         self.last_solve = {}
 
     def p2pWaves(self):
-        """4 (the batched pair sums have one launch shape; kept for callers
+        """4, the runs that a tile's sources are summed in (kept for callers
         that report it)."""
         v = ctypes.c_int32()
         check(lib().nnk_batch_p2p_waves(self.h, ctypes.byref(v)))

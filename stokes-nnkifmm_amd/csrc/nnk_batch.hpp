@@ -15,8 +15,9 @@
 // [f (3 N_p, all x, all y, all z); U (3 nsw_p: all x, all y, all z);
 // Omega (3 nsw_p)].  The operator is four launches: the quadrature
 // strengths g = (NN (x) I3) f, the pair sums of (problem, 64-target tile,
-// source part) work items largest first, the sums of their parts plus
-// BT (U; W), and one workgroup per body for B f.  The transpose (adjoint) operator
+// source run) work items largest first (or, where there are tiles enough,
+// of whole tiles), the sums of their runs plus BT (U; W), and one workgroup
+// per body for B f.  The transpose (adjoint) operator
 // runs the P2P from force points onto quadrature points and gathers with
 // NN^T.  GMRES runs all problems in lockstep (segmented dot products,
 // per-problem Givens on the host) and retires each problem as it converges.
@@ -56,7 +57,7 @@ class Batch {
   // y = A x (transpose: y = A^T x) for every problem (device vectors)
   void apply(const double *x, double *y, bool transpose, hipStream_t s);
   void set_graph(bool on) { graph_ = on; }
-  // runs a tile's sources are summed in (wavefronts that used to share them)
+  // runs a tile's sources are summed in
   int p2p_waves() const { return 4; }
   // unrestarted GMRES from x = 0 per problem on A (or A^T); per-problem
   // flag (0 when the recomputed relative residual is <= tol), that residual

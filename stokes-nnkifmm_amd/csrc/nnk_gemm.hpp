@@ -393,7 +393,13 @@ __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256, 2) void k_gemm_direct(
 // wavefronts from one per CU, else 32 x 16 shared by eight.  Both sides of the
 // lines at K = 456: 4,096 columns (320 workgroups of 48 x 128) take 0.16 ms
 // less over a matvec's up pass with the shared tiles; 512 columns 36 against
-// 23 us for an L2L.
+// 23 us for an L2L.  Other ranks, a matvec's up pass in us by the rule and with
+// each shape throughout (48 x 128; 48 x 32; 32 x 16): K = 168, 512 leaves 43
+// (165; 70; 42), 4,096 leaves 88 (299; 129; 106), 32,768 leaves 257 (522; 365;
+// 550); K = 888, 512 leaves 166 (696; 234; 184), 8,192 leaves 1,120 (2,221;
+// 1,272; 1,850); K = 1,464, 512 leaves 388 (1,131; 371; 464), 2,048 leaves 1,089
+// (2,224; 922; 1,358): at the largest rank the shared tiles would be the better a
+// little earlier.
 // FP64 matvecs before (160 x 32 tiles staged through LDS, M2M split over the
 // children where columns are few) and now, res 6: up pass 198 -> 76 us, solves
 // 155 -> 46 us, L2L 49 -> 23 us with 64 and 512 leaves; 2^20 points 1.42 ->

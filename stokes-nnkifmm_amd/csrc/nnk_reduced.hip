@@ -2,8 +2,8 @@
 // for every target leaf, solve K(leaf sources -> leaf targets) x = v, or in
 // NEAREST mode (K(fine -> targets) kron(NN_leaf, I3)) x = v (ReducedSolve.m
 // :170-187).  The 3n x 3n blocks are formed and LU-factored with partial
-// pivoting once per tree on the GPU (one workgroup per leaf), and each
-// block's inverse is formed from its factors; each solve is then one
+// pivoting once per tree on the GPU (panel by panel, all leaves in a launch),
+// and each block's inverse is formed from its factors; each solve is then one
 // block-diagonal matrix-vector product.  MATLAB's mldivide would use
 // Cholesky on the symmetric non-NEAREST blocks; both give the solution up
 // to rounding (relative error of order cond(A) times the FP64 epsilon).

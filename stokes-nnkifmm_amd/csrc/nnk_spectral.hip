@@ -341,8 +341,10 @@ struct SpecTile {
 // parents and split the directions, partial sums added in wavefront order
 // (few parents: four times the workgroups, and no idle wavefronts in the
 // tiles of the levels near the root, at a table load per 16 parents).
-// Measured WD = 1 / 4: 72 parents 0.204 / 0.147 ms, ~460 parents 0.525 /
-// 0.552 ms, 4,681 parents 5.9 / 7.3 ms.  32 parents per wavefront (236
+// Measured WD = 1 / 4 at res 6: 72 parents 0.204 / 0.147 ms, ~460 parents
+// 0.525 / 0.552 ms, 4,681 parents 5.9 / 7.3 ms; the whole M2L at 148 and 292
+// parents, res 4 102 / 87 and 175 / 153 us, res 8 779 / 651 and 1,245 / 1,329,
+// res 10 1,616 / 1,384 and 2,640 / 2,825.  32 parents per wavefront (236
 // registers, two wavefronts per SIMD instead of three) was slower
 // everywhere: 6.0 ms at 4,681 parents, 0.34 ms at 72.
 template <int WD>
@@ -706,8 +708,12 @@ void SpectralM2L::run(const double *up, double *chk, hipStream_t s) const {
       const int f0 = plane_base(P, kx0), f1 = kx0 + nkx == P ? (n * n * n + 1) / 2 : plane_base(P, kx0 + nkx);
       const int nf = f1 - f0;
       if (ns_) {
-        // one plane per workgroup takes 0.81 ms at 4,681 parents, all of them 0.31 ms; with
-        // fewer parents than fill the chip a few times the planes run side by side (15 us at 72)
+        // few parents: the planes side by side, a workgroup each; many: all planes by
+        // one workgroup, which reads the densities once.  The whole M2L in us, side by
+        // side / all by one: 72 parents res 6 172 / 182, res 10 832 / 828; 292 res 6 508 /
+        // 511, res 10 2,635 / 2,496; 916 1,280 / 1,247 and 7,122 / 6,586; 1,172 1,625 /
+        // 1,596 and 9,055 / 7,991; 4,681 res 6 6,747 / 6,310.  (The sides meet near 300
+        // parents at res 6; up to the line at 1,024 that is 2 to 8 % of the M2L.)
         const int kxn = ns_ < 1024 ? 1 : nkx;
         hipLaunchKernelGGL((k_spec_fwd<P, T>), dim3(ns_, (nkx + kxn - 1) / kxn), dim3(T), 0, s, up, K_,
                            src0_.as<int32_t>(), smask_.as<int32_t>(), qmap_.as<int32_t>(), tw_.as<double>(), kx0, nkx,
@@ -728,6 +734,9 @@ void SpectralM2L::run(const double *up, double *chk, hipStream_t s) const {
                            (size_t)48 * nt_, K_, tgt0_.as<int32_t>(), tmask_.as<int32_t>(), qmap_.as<int32_t>(),
                            tw_.as<double>(), kx0, nkx, kx0 > 0 ? 1 : 0, chk);
       };
+      // 2 children a workgroup / 8, the whole M2L in us: 72 parents res 6 171 / 181, res
+      // 10 832 / 808; 292 509 / 506 and 2,644 / 2,554; 916 1,283 / 1,261 and 7,128 /
+      // 6,728; 1,172 1,608 / 1,595 and 8,483 / 7,985; 4,681 res 6 6,455 / 6,310
       if (nt_ < 1024) inv(std::integral_constant<int, 2>());
       else inv(std::integral_constant<int, 8>());
       NNK_HIP(hipGetLastError());
