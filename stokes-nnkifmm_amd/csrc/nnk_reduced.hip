@@ -766,7 +766,9 @@ void Fmm::reduced_solve(const double *d_v, double *d_f, hipStream_t s) {
   // 64 x 2,100 (2.3 GB) 400, 381; 512 x 1,500 (9.2 GB) 1,827, 1,585.
   const size_t lds = sizeof(double) * red_maxn_;
   const bool many = n_tleaves_ >= ncu_;
-  if (red_maxn_ <= 64) go(k_red_apply_leaf<128>, 64, 128, 0);
+  // (346 x 63 (192), 11 MB, alone on the device 9.1, 27, 12.1)
+  if (n_tleaves_ < 4 * ncu_ && red_blk_.bytes < ((size_t)64 << 20)) go(k_red_apply, 64, 64 * kRedApplyWaves, lds);
+  else if (red_maxn_ <= 64) go(k_red_apply_leaf<128>, 64, 128, 0);
   else if (red_maxn_ <= 128) go(k_red_apply_leaf<256>, 128, 256, 0);
   else if (red_maxn_ <= 256 || (red_maxn_ <= 320 && many)) go(k_red_apply_leaf<512>, 320, 512, 0);
   else if ((red_maxn_ <= 512 && many) || red_blk_.bytes >= ((size_t)7 << 28))

@@ -12,18 +12,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("cells,sizes,eps", [
-    (8, [21, 5, 6, 10], 0.02),                    # 512 leaves of at most 63 rows
-    (8, [42, 8, 22, 11], 0.02), (8, [85, 13, 43, 64], 0.015),
-    (8, [106, 30, 86, 40], 0.01), (4, [85, 30], 0.03),   # 512 threads: one to five share a row
+    (16, [21, 5, 6, 10], 0.01),                   # 4,096 leaves of at most 63 rows
+    (16, [42, 8, 22, 11], 0.01), (8, [85, 43, 64, 70], 0.015),
+    (8, [106, 30, 86, 40], 0.01),                 # 512 threads: one to five share a row
     (8, [170, 60, 107, 90], 0.008),               # a thread per row: 510 rows
-    (4, [86, 30], 0.03), (4, [341, 100], 0.02),   # 64 leaves: eight wavefronts
+    (8, [21, 5, 6, 10], 0.02), (4, [86, 30], 0.03), (4, [341, 100], 0.02),   # few: eight wavefronts
     (4, [700], 0.02)])                            # 2.3 GB
 def test_shapes(nnk, cells, sizes, eps):
     rng = np.random.default_rng(cells + sizes[0])
     grid = np.stack(np.meshgrid(*[np.arange(cells)] * 3, indexing="ij"), -1).reshape(-1, 3)
     count = rng.choice(sizes[1:] or sizes, len(grid))
     count[::17] = sizes[0]
-    count[3] = 1 if cells == 8 else sizes[0]      # a parent's points are still more than the largest leaf's
+    count[3] = 1 if cells >= 8 else sizes[0]      # a parent's points are still more than the largest leaf's
     p = (np.repeat(grid, count, axis=0) + rng.random((count.sum(), 3))) / cells
     tree = nnk.OcTree(p, p, "nodeCapacity", max(sizes), "rootCube", [0.0, 1.0])
     assert tree.nodeCount == (8 * cells ** 3 - 1) // 7
