@@ -722,8 +722,11 @@ __global__ void k_bscale(int64_t n, const int32_t *__restrict__ pid, const doubl
 // tiles 83, 72 and 79, 68; 3,706 365, 328 and 277, 231; 97,930 20,818, 18,111
 // and 12,621, 11,224.  Forward (long runs, of uneven lengths): 2,414 tiles
 // 8,011, 8,197 and 4,635, 5,096; 4,920 2,799, 2,426 and 1,976, 1,809; 6,236
-// 20,844, 19,330 and 11,978, 11,805.
-constexpr int kBatchTiles = 4096, kBatchTilesT = 640, kBatchRunT = 1024;
+// 20,844, 19,330 and 11,978, 11,805.  The last are 256 problems of up to 78,000
+// quadrature points; a solve of them ends with a few long ones, which k_bsum
+// shortens: ms 1,172, 1,170 and 798, 853.  With FP32 math only runs of up to
+// kBatchRun32 points a problem go forward in tiles.
+constexpr int kBatchTiles = 4096, kBatchTilesT = 640, kBatchRunT = 1024, kBatchRun32 = 16384;
 
 Batch::Batch(int nprob, const int64_t *pt_off, const double *pts, const int64_t *fine_off, const double *fine,
              const int64_t *nn_ptr, const int32_t *nn_col, const double *nn_val, const double *w,
@@ -839,9 +842,12 @@ Batch::Batch(int nprob, const int64_t *pt_off, const double *pts, const int64_t 
   };
   auto it_f = make_items(false), it_t = make_items(true);
   // which sums go a tile per workgroup, and the run items of the others
-  int64_t most = 0;
-  for (int p = 0; p < nprob; p++) most = std::max(most, hpoff_[p + 1] - hpoff_[p]);
-  tiles_ = (int)it_f.size() >= kBatchTiles;
+  int64_t most = 0, most_q = 0;
+  for (int p = 0; p < nprob; p++) {
+    most = std::max(most, hpoff_[p + 1] - hpoff_[p]);
+    most_q = std::max(most_q, hfoff[p + 1] - hfoff[p]);
+  }
+  tiles_ = (int)it_f.size() >= kBatchTiles && (!f32_ || most_q <= kBatchRun32);
   tilesT_ = (int)it_t.size() >= kBatchTilesT || most <= kBatchRunT;
   hfoff_ = hfoff;
   int64_t sums = tiles_ ? 3 * ntot_ : 0;
